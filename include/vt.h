@@ -446,7 +446,7 @@ int vt_batch_autotune(vt_ctx* ctx, const vt_world* world, const vt_view* views,
  * hipMalloc).  Renders the views like vt_batch_create + vt_batch_launch (same
  * kernels, same outputs bit for bit) but allocates nothing: the view table
  * and the work-queue counters live in a fixed device array of the library
- * (about 45 KiB per GPU, held until the process ends), whose address each
+ * (about 46 KiB per GPU, held until the process ends), whose address each
  * vt_create takes once per device.  The view records are handed over as
  * kernel arguments, so `views` may be freed when the call returns.  At most
  * VT_NOALLOC_MAX_VIEWS views (else VT_ERR_INVALID_ARGUMENT).  All calls on

@@ -26,9 +26,15 @@ struct BatchView {
 };
 
 constexpr uint32_t kQueues = 8;
+// Words from one queue counter to the next: each has a 128-byte line of its
+// own.  Atomics on one line serialise in the memory system at about 15 ns
+// each, and with the eight counters on one line they were the batch's time:
+// 64 views over the 1024^3 world (281,000 grabs of one tile) took 4.24 ms,
+// 24 views over the 512^3 world 1.45 ms.
+constexpr uint32_t kQueueLine = 32;
 
 __global__ void k_batch_reset(uint32_t* __restrict__ queues) {
-  if (threadIdx.x < kQueues) queues[threadIdx.x] = 0u;
+  if (threadIdx.x < kQueues) queues[threadIdx.x * kQueueLine] = 0u;
 }
 
 // 7 waves per SIMD (72 VGPRs): the view record and queue state push the
@@ -58,7 +64,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VT_BATCH_WA
     const uint32_t hi = (uint32_t)(((uint64_t)total_tiles * (q + 1)) / kQueues);
     for (;;) {
       uint32_t got = 0;
-      if (lane == 0) got = atomicAdd(queues + q, chunk);
+      if (lane == 0) got = atomicAdd(queues + q * kQueueLine, chunk);
       got = __builtin_amdgcn_readfirstlane(__shfl(got, 0, 64));
       if (got >= hi - lo) break;
       const uint32_t t1 = lo + min(got + chunk, hi - lo);
@@ -99,7 +105,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VT_BATCH_WA
 // device at vt_create (noalloc_init) with that device current.
 struct NoallocScratch {
   BatchView views[VT_NOALLOC_MAX_VIEWS];
-  uint32_t queues[kQueues];
+  uint32_t queues[kQueues * kQueueLine];
 };
 
 static __device__ __align__(256) NoallocScratch scratch;
@@ -306,7 +312,8 @@ int vt_batch_create(vt_ctx* ctx, const vt_world* world, const vt_view* views, ui
   for (uint32_t i = 0; i < n_views; i++) b->steps_out |= views[i].frame.steps != nullptr;
   b->nblocks = (uint32_t)ctx->compute_units * t.blocks_per_cu;
   hipError_t e = hipMalloc((void**)&b->d_views, sizeof(vt::BatchView) * n_views);
-  if (e == hipSuccess) e = hipMalloc((void**)&b->d_queues, sizeof(uint32_t) * vt::kQueues);
+  if (e == hipSuccess)
+    e = hipMalloc((void**)&b->d_queues, sizeof(uint32_t) * vt::kQueues * vt::kQueueLine);
   if (e == hipSuccess)
     e = hipMemcpy(b->d_views, table.data(), sizeof(vt::BatchView) * n_views,
                   hipMemcpyHostToDevice);
