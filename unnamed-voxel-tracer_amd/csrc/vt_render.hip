@@ -274,6 +274,9 @@ hipError_t launch_render_brickmap(const BrickmapWorld& w_in, const ViewConsts& v
                                   TileShape tile, uint32_t compute_units, hipStream_t stream) {
   (void)compute_units;
   BrickmapWorld w = w_in;
+  // a map of fewer blocks a side than two empty-space iterations take steps
+  // (8^3: one chunk) stays on the literal loop (dense_left_grid)
+  if (w.dim < 2u * (uint32_t)kSkipLong) w.occ = nullptr;
   // step counts stored, or statistics (of traceMap's steps on this layout):
   // no early end of rays
   if (out.steps || out.stats) {
