@@ -58,7 +58,6 @@ void free_world(vt_world* w) {
   dev_free(w->occ);
   dev_free(w->brick_bits);
   dev_free(w->freemap);
-  dev_free(w->free_tmp);
   delete[] w->chunk_mirror;
   delete w;
 }
@@ -85,14 +84,10 @@ int dev_alloc(vt_world* w, void** p, size_t bytes, const char* what) {
   return VT_OK;
 }
 
-// The free-region map and its build scratch (built by vt::rebuild_freemap).
+// The free-region map (built by vt::rebuild_freemap).
 int alloc_freemap(vt_world* w) {
-  const uint32_t R = vt::free_regions(w->dim);
-  int st;
-  if ((st = dev_alloc(w, (void**)&w->freemap, 8u * vt::free_words_per_octant(w->dim) * 4u,
-                      "free-region map")) != VT_OK)
-    return st;
-  return dev_alloc(w, (void**)&w->free_tmp, (size_t)8u * R * R * R, "free-region scratch");
+  return dev_alloc(w, (void**)&w->freemap, (8u * vt::free_words_per_octant(w->dim) + 1u) * 4u,
+                   "free-region map");
 }
 
 }  // namespace
@@ -164,37 +159,6 @@ void scan_brickmap_box(const uint32_t* chunks, const uint32_t* pool, uint32_t di
             grow_box(w, (int32_t)(8u * cx + (i & 7u)), (int32_t)(8u * cy + ((i >> 3) & 7u)),
                      (int32_t)(8u * cz + (i >> 6)));
       }
-}
-
-// The box of the nonempty voxels of a linear grid (x + dim (y + dim z)).
-void scan_dense_box(const uint8_t* grid, uint32_t dim, vt_world* w) {
-  w->box_any = false;
-  for (int i = 0; i < 3; i++) {
-    w->box_lo[i] = (int32_t)dim;
-    w->box_hi[i] = -1;
-  }
-  for (uint32_t z = 0; z < dim; z++)
-    for (uint32_t y = 0; y < dim; y++) {
-      const uint8_t* row = grid + (size_t)dim * (y + (size_t)dim * z);
-      uint64_t any = 0;
-      for (uint32_t x = 0; x + 8 <= dim; x += 8) {
-        uint64_t q;
-        std::memcpy(&q, row + x, 8);
-        any |= q;
-      }
-      for (uint32_t x = dim & ~7u; x < dim; x++) any |= row[x];
-      if (!any) continue;
-      uint32_t x0 = 0, x1 = dim - 1;
-      while (!row[x0]) x0++;
-      while (!row[x1]) x1--;
-      w->box_any = true;
-      w->box_lo[0] = std::min(w->box_lo[0], (int32_t)x0);
-      w->box_hi[0] = std::max(w->box_hi[0], (int32_t)x1);
-      w->box_lo[1] = std::min(w->box_lo[1], (int32_t)y);
-      w->box_hi[1] = std::max(w->box_hi[1], (int32_t)y);
-      w->box_lo[2] = std::min(w->box_lo[2], (int32_t)z);
-      w->box_hi[2] = std::max(w->box_hi[2], (int32_t)z);
-    }
 }
 
 BrickmapWorld brickmap_view(const vt_world* w) {
@@ -389,16 +353,18 @@ int vt_create(vt_ctx** out, int device) {
   c->compute_units = prop.multiProcessorCount;
   std::snprintf(c->name, sizeof c->name, "%s", prop.gcnArchName);
   c->stage = nullptr;
-  e = hipMalloc(&c->stage, kCtxStageBytes);
+  e = hipHostMalloc(&c->stage, kCtxStageBytes + kCtxReportBytes, hipHostMallocDefault);
+  if (e == hipSuccess) e = hipHostGetDevicePointer(&c->stage_dev, c->stage, 0);
   if (e != hipSuccess) {
     (void)hipGetLastError();
+    if (c->stage) (void)hipHostFree(c->stage);
     delete c;
-    return fail(VT_ERR_OUT_OF_MEMORY, "vt_create: %zu bytes of staging: %s", kCtxStageBytes,
-                hipGetErrorString(e));
+    return fail(VT_ERR_OUT_OF_MEMORY, "vt_create: %zu bytes of staging: %s",
+                kCtxStageBytes + kCtxReportBytes, hipGetErrorString(e));
   }
   int st = vt::noalloc_init(device);
   if (st != VT_OK) {
-    dev_free(c->stage);
+    (void)hipHostFree(c->stage);
     delete c;
     return st;
   }
@@ -409,7 +375,7 @@ int vt_create(vt_ctx** out, int device) {
 int vt_destroy(vt_ctx* ctx) {
   if (!ctx) return fail(VT_ERR_NULL_POINTER, "vt_destroy: ctx is NULL");
   (void)hipSetDevice(ctx->device);
-  dev_free(ctx->stage);
+  if (ctx->stage) (void)hipHostFree(ctx->stage);
   delete ctx;
   return VT_OK;
 }
@@ -464,18 +430,23 @@ int vt_world_create_dense_u8(vt_ctx* ctx, const uint8_t* grid, uint32_t dim,
     free_world(w);
     return fail(VT_ERR_OUT_OF_MEMORY, "vt_world_create_dense_u8: staging %zu bytes", n);
   }
-  vt::scan_dense_box(grid, dim, w);
   e = hipMemcpy(lin, grid, n, hipMemcpyHostToDevice);
   if (e == hipSuccess) e = hipMemcpy(w->palette, palette_rgba8, 256 * 4, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = vt::launch_build_dense(lin, dim, w->vox, w->l0, w->l1, w->l1b, nullptr);
+  // (the box is summed up in the free-region map's memory, which is built after)
+  if (e == hipSuccess)
+    e = vt::launch_build_dense(lin, dim, w->vox, w->l0, w->l1, w->l1b, (int32_t*)w->freemap,
+                               ctx->report_dev(), nullptr);
   if (e == hipSuccess) e = vt::rebuild_freemap(w, nullptr);
   if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
-  if (e == hipSuccess) e = vt::finish_freemap(w);
   dev_free(lin);
   if (e != hipSuccess) {
     free_world(w);
     return hip_fail(e, "vt_world_create_dense_u8: upload/build");
   }
+  vt::finish_freemap(w);
+  std::memcpy(w->box_lo, ctx->report()->box_lo, sizeof w->box_lo);
+  std::memcpy(w->box_hi, ctx->report()->box_hi, sizeof w->box_hi);
+  w->box_any = w->box_lo[0] <= w->box_hi[0];
   *out = w;
   return VT_OK;
 }
@@ -540,14 +511,14 @@ int vt_world_create_brickmap(vt_ctx* ctx, uint32_t dim, const uint32_t* chunks,
       free_world(w);
       return st;
     }
-    e = vt::launch_build_occupancy(vt::brickmap_view(w), w->occ, nullptr);
+    e = vt::launch_build_occupancy(vt::brickmap_view(w), w->occ, w->brick_bits, nullptr);
     if (e == hipSuccess) e = vt::rebuild_freemap(w, nullptr);
     if (e == hipSuccess) e = hipDeviceSynchronize();
-    if (e == hipSuccess) e = vt::finish_freemap(w);
     if (e != hipSuccess) {
       free_world(w);
       return hip_fail(e, "vt_world_create_brickmap: occupancy");
     }
+    vt::finish_freemap(w);
   }
   *out = w;
   return VT_OK;

@@ -29,47 +29,82 @@
 
 namespace vt {
 
-__global__ __launch_bounds__(256) void k_scatter_u32(uint32_t* __restrict__ dst,
-                                                     const uint64_t* __restrict__ addr,
-                                                     const uint32_t* __restrict__ val, uint32_t n) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[addr[i]] = val[i];
+// The edits of a brickmap world.  data: n records (pool word, value, block's
+// Morton code), then m records (chunk, its new entry).
+__global__ __launch_bounds__(256) void k_edit_brickmap(uint32_t* __restrict__ pool,
+                                                       uint8_t* __restrict__ occ,
+                                                       uint32_t* __restrict__ chunks,
+                                                       const uint32_t* __restrict__ data,
+                                                       uint32_t n, uint32_t m,
+                                                       uint32_t* __restrict__ changed) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i == 0u && changed) *changed = 0u;  // for the kernels that follow
+  if (i < n) {
+    const uint3 r = reinterpret_cast<const uint3*>(data)[i];
+    pool[r.x] = r.y;
+    if (occ) occ[r.z] = r.y != 0u ? 1 : 0;
+  }
+  if (i < m) {
+    const uint32_t* c = data + 3u * (size_t)n + 2u * (size_t)i;
+    chunks[c[0]] = c[1];
+  }
 }
 
-// dst[addr[i]] = 0 for i < n (undoing k_scatter_u32 of new chunk entries).
-__global__ __launch_bounds__(256) void k_fill_u32(uint32_t* __restrict__ dst,
-                                                  const uint64_t* __restrict__ addr, uint32_t n) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[addr[i]] = 0u;
+// The brick bits of the listed 4^3 bricks, from their 64 occupancy bytes
+// (one wave per brick; several bricks of a word: atomics on its bits).  Sets
+// *changed when a word (a 16^3 region) stops or starts being zero.
+__global__ __launch_bounds__(256) void k_edit_bricks(const uint8_t* __restrict__ occ,
+                                                     const uint32_t* __restrict__ bricks,
+                                                     uint32_t n,
+                                                     unsigned long long* __restrict__ bits,
+                                                     uint32_t* __restrict__ changed) {
+  const uint32_t wave = (blockIdx.x * 256u + threadIdx.x) >> 6, lane = threadIdx.x & 63u;
+  if (wave >= n) return;  // whole waves leave together
+  const uint32_t b = bricks[wave];
+  const bool any = __ballot(occ[(size_t)b * 64u + lane] != 0) != 0ull;
+  if (lane != 0u) return;
+  const unsigned long long bit = 1ull << (b & 63u);
+  if (any) {
+    if (atomicOr(bits + (b >> 6), bit) == 0ull) *changed = 1u;
+  } else {
+    const unsigned long long old = atomicAnd(bits + (b >> 6), ~bit);
+    if (old != 0ull && (old & ~bit) == 0ull) *changed = 1u;
+  }
 }
 
-__global__ __launch_bounds__(256) void k_scatter_u8(uint8_t* __restrict__ dst,
-                                                    const uint64_t* __restrict__ addr,
-                                                    const uint32_t* __restrict__ val, uint32_t n) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[addr[i]] = (uint8_t)val[i];
+// Undoes new chunk entries: data holds m records (chunk, entry).
+__global__ __launch_bounds__(256) void k_unset_chunks(uint32_t* __restrict__ chunks,
+                                                      const uint32_t* __restrict__ data,
+                                                      uint32_t m) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i < m) chunks[data[2u * (size_t)i]] = 0u;
 }
 
-__global__ __launch_bounds__(256) void k_scatter_nonzero_u8(uint8_t* __restrict__ dst,
-                                                            const uint64_t* __restrict__ addr,
-                                                            const uint32_t* __restrict__ val,
-                                                            uint32_t n) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[addr[i]] = val[i] != 0u ? 1 : 0;
+// The edits of a dense world: n records (Morton code, material).
+__global__ __launch_bounds__(256) void k_edit_dense(uint8_t* __restrict__ vox,
+                                                    const uint32_t* __restrict__ data,
+                                                    uint32_t n, uint32_t* __restrict__ changed) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i == 0u) *changed = 0u;  // for the kernels that follow
+  if (i < n) vox[data[2u * (size_t)i]] = (uint8_t)data[2u * (size_t)i + 1u];
 }
 
 // One wave per listed word: bit l of out[word] = (in[word * 64 + l] != 0).
+// Sets *changed (when not null) when a word stops or starts being zero.
 template <class T>
 __global__ __launch_bounds__(256) void k_rebuild_mask(const T* __restrict__ in,
                                                       uint64_t* __restrict__ out,
                                                       const uint32_t* __restrict__ words,
-                                                      uint32_t n) {
+                                                      uint32_t n, uint32_t* __restrict__ changed) {
   const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
   const uint32_t lane = threadIdx.x & 63u;
   if (wave >= n) return;  // whole waves leave together
   const uint32_t word = words[wave];
   const uint64_t m = __ballot(in[(size_t)word * 64u + lane] != 0);
-  if (lane == 0) out[word] = m;
+  if (lane == 0) {
+    if (changed && (out[word] == 0ull) != (m == 0ull)) *changed = 1u;
+    out[word] = m;
+  }
 }
 
 __global__ void k_gather_dense(const DenseWorld w, const uint32_t* __restrict__ xyz, uint32_t n,
@@ -160,10 +195,16 @@ __global__ void k_pick_brickmap(const BrickmapWorld w, ViewConsts v, int max_ste
   if (threadIdx.x != 0) return;
   float e[3], d[3];
   centre_ray(v, w.dim, e, d);
+  // one lane: bound by the latency of its lookups, so the empty blocks go
+  // through the loop that keeps several in flight (same steps, same count)
   GeneralHit g;
-  uint32_t chunk_reads = 0, pool_reads = 0;
-  trace_general<false>(w, e[0], e[1], e[2], d[0], d[1], d[2], max_steps, g, chunk_reads,
-                       pool_reads);
+  if (w.occ) {
+    trace_brickmap_fast<false, false>(w, e[0], e[1], e[2], d[0], d[1], d[2], max_steps, g);
+  } else {
+    uint32_t chunk_reads = 0, pool_reads = 0;
+    trace_general<false>(w, e[0], e[1], e[2], d[0], d[1], d[2], max_steps, g, chunk_reads,
+                         pool_reads);
+  }
   *out = pick_result(g.data != 0u, g.data, g.face, g.hx, g.hy, g.hz, g.steps);
 }
 
@@ -209,22 +250,39 @@ namespace {
 using vt::fail;
 using vt::hip_fail;
 
-// Device staging for one call; freed after the call's stream work is done.
-struct Staging {
-  std::vector<void*> bufs;
-  ~Staging() {
-    for (void* p : bufs) vt::dev_free(p);
+// The words of one call's lists where the device can read them: the
+// context's staging, or device memory for the call when they are more.
+// The destructor waits for the stream: the next call may use the staging.
+struct Lists {
+  vt_ctx* ctx;
+  hipStream_t s;
+  uint32_t* own = nullptr;
+  const uint32_t* dev = nullptr;
+  Lists(vt_ctx* c, hipStream_t st) : ctx(c), s(st) {}
+  ~Lists() {
+    if (dev) (void)hipStreamSynchronize(s);
+    vt::dev_free(own);
   }
-  template <class T>
-  hipError_t upload(const std::vector<T>& v, T** out, hipStream_t s) {
-    *out = nullptr;
-    if (v.empty()) return hipSuccess;
-    hipError_t e = hipMalloc((void**)out, v.size() * sizeof(T));
+  hipError_t put(const std::vector<uint32_t>& words) {
+    const size_t bytes = words.size() * 4u;
+    if (bytes <= kCtxStageBytes) {
+      std::memcpy(ctx->stage, words.data(), bytes);
+      dev = (const uint32_t*)ctx->stage_dev;
+      return hipSuccess;
+    }
+    hipError_t e = hipMalloc((void**)&own, bytes);
     if (e != hipSuccess) return e;
-    bufs.push_back(*out);
-    return hipMemcpyAsync(*out, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice, s);
+    e = hipMemcpyAsync(own, words.data(), bytes, hipMemcpyHostToDevice, s);
+    dev = own;
+    return e;
   }
 };
+
+// Sorted, each value once.
+void sort_unique(std::vector<uint32_t>& v) {
+  std::sort(v.begin(), v.end());
+  v.erase(std::unique(v.begin(), v.end()), v.end());
+}
 
 uint32_t part1by2_host(uint32_t v) {
   v &= 0x3FFu;
@@ -263,16 +321,16 @@ static void grow_box_by(vt_world* w, const uint32_t* xyz, const uint32_t* values
 int set_brickmap(vt_world* w, const uint32_t* xyz, const uint32_t* values, uint32_t n,
                  hipStream_t s) {
   const uint32_t M = w->dim / 8u;
-  std::vector<std::pair<uint64_t, uint32_t>> new_chunks;
-  std::unordered_map<uint64_t, uint32_t> last;  // pool word -> position in `writes`
-  std::vector<uint64_t> addr, oaddr;            // pool word, occupancy byte (Morton)
-  std::vector<uint32_t> val;
+  std::unordered_map<uint64_t, uint32_t> last;  // pool word -> its record
   // chunks this call allocates: kept here and entered into the host chunk
   // table only once the device holds them, so a failed call leaves the
   // world as it was
   std::unordered_map<uint64_t, uint32_t> fresh;
+  std::vector<uint32_t> words;  // records (pool word, value, Morton code), see k_edit_brickmap
+  std::vector<uint32_t> chunks, bricks;
   uint64_t used = w->pool_words / 512u;
   last.reserve(n);
+  words.reserve(3 * (size_t)n);
   grow_box_by(w, xyz, values, n);
   for (uint32_t i = 0; i < n; i++) {
     const uint32_t x = xyz[3 * (size_t)i], y = xyz[3 * (size_t)i + 1], z = xyz[3 * (size_t)i + 2];
@@ -283,58 +341,51 @@ int set_brickmap(vt_world* w, const uint32_t* xyz, const uint32_t* values, uint3
       if (f != fresh.end()) {
         entry = f->second;
       } else {  // get_block_for_chunk: allocate on first touch
-        if (used >= 0xFFFFFFFEull) return fail(VT_ERR_OUT_OF_MEMORY, "vt_world_set_voxels: pool");
-        entry = (uint32_t)(++used);
+        entry = (uint32_t)(++used);  // at most one block per chunk: (dim / 8)^3
         fresh.emplace(ci, entry);
-        new_chunks.emplace_back(ci, entry);
+        chunks.push_back((uint32_t)ci);
+        chunks.push_back(entry);
       }
     }
     const uint64_t a = (uint64_t)(entry - 1u) * 512u + (x % 8u) + 8u * ((y % 8u) + 8u * (z % 8u));
+    const uint32_t code = morton_code(x, y, z);
     auto it = last.find(a);
     if (it == last.end()) {
-      last.emplace(a, (uint32_t)addr.size());
-      addr.push_back(a);
-      val.push_back(values[i]);
-      if (w->occ) oaddr.push_back(morton_code(x, y, z));
+      last.emplace(a, (uint32_t)(words.size() / 3u));
+      words.insert(words.end(), {(uint32_t)a, values[i], code});
+      bricks.push_back(code >> 6);
     } else {
-      val[it->second] = values[i];
+      words[3 * (size_t)it->second + 1] = values[i];
     }
   }
   int st = vt::grow_pool(w, used, s, "vt_world_set_voxels: pool growth");
   if (st != VT_OK) return st;  // nothing written: the world is unchanged
-  std::vector<uint64_t> caddr;
-  std::vector<uint32_t> cval;
-  for (auto& c : new_chunks) {
-    caddr.push_back(c.first);
-    cval.push_back(c.second);
-  }
-  Staging stg;
-  uint64_t *d_addr, *d_caddr, *d_oaddr;
-  uint32_t *d_val, *d_cval;
-  VT_HIP(stg.upload(addr, &d_addr, s));
-  VT_HIP(stg.upload(val, &d_val, s));
-  VT_HIP(stg.upload(caddr, &d_caddr, s));
-  VT_HIP(stg.upload(cval, &d_cval, s));
-  VT_HIP(stg.upload(oaddr, &d_oaddr, s));
-  if (!addr.empty())
-    hipLaunchKernelGGL(vt::k_scatter_u32, dim3(blocks_for(addr.size(), 256)), dim3(256), 0, s,
-                       w->pool, d_addr, d_val, (uint32_t)addr.size());
-  if (!oaddr.empty())
-    hipLaunchKernelGGL(vt::k_scatter_nonzero_u8, dim3(blocks_for(oaddr.size(), 256)), dim3(256),
-                       0, s, w->occ, d_oaddr, d_val, (uint32_t)oaddr.size());
-  if (!caddr.empty())
-    hipLaunchKernelGGL(vt::k_scatter_u32, dim3(blocks_for(caddr.size(), 256)), dim3(256), 0, s,
-                       w->chunks, d_caddr, d_cval, (uint32_t)caddr.size());
+  sort_unique(bricks);
+  const uint32_t nw = (uint32_t)(words.size() / 3u), nc = (uint32_t)(chunks.size() / 2u),
+                 nb = (uint32_t)bricks.size();
+  words.insert(words.end(), chunks.begin(), chunks.end());
+  words.insert(words.end(), bricks.begin(), bricks.end());
+  Lists lists(w->ctx, s);
+  VT_HIP(lists.put(words));
+  const uint32_t* d_chunks = lists.dev + 3 * (size_t)nw;
+  hipLaunchKernelGGL(vt::k_edit_brickmap, dim3(blocks_for(std::max(nw, nc), 256)), dim3(256), 0, s,
+                     w->pool, w->occ, w->chunks, lists.dev, nw, nc, vt::freemap_changed(w));
   hipError_t e = hipGetLastError();
-  if (e == hipSuccess && !oaddr.empty()) e = vt::rebuild_freemap(w, s);
+  if (e == hipSuccess && w->occ) {
+    hipLaunchKernelGGL(vt::k_edit_bricks, dim3(blocks_for(nb, 4)), dim3(256), 0, s, w->occ,
+                       d_chunks + 2 * (size_t)nc, nb, (unsigned long long*)w->brick_bits,
+                       vt::freemap_changed(w));
+    e = hipGetLastError();
+    if (e == hipSuccess) e = vt::rebuild_freemap(w, s, vt::freemap_changed(w));
+  }
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) {
     // Undo what may have reached the device: new chunk entries back to 0
     // and the new blocks zero again (edits allocate zero blocks), so the
     // device agrees with the unchanged host chunk table and pool count.
-    if (!caddr.empty())
-      hipLaunchKernelGGL(vt::k_fill_u32, dim3(blocks_for(caddr.size(), 256)), dim3(256), 0, s,
-                         w->chunks, d_caddr, (uint32_t)caddr.size());
+    if (nc)
+      hipLaunchKernelGGL(vt::k_unset_chunks, dim3(blocks_for(nc, 256)), dim3(256), 0, s, w->chunks,
+                         d_chunks, nc);
     const uint64_t b0 = w->pool_words / 512u;
     if (used > b0)
       (void)hipMemsetAsync(w->pool + b0 * 512u, 0, (used - b0) * 512u * 4u, s);
@@ -342,9 +393,9 @@ int set_brickmap(vt_world* w, const uint32_t* xyz, const uint32_t* values, uint3
     (void)hipGetLastError();
     return hip_fail(e, "vt_world_set_voxels: scatter");
   }
-  for (auto& c : new_chunks) w->chunk_mirror[c.first] = c.second;
+  for (uint32_t k = 0; k < nc; k++) w->chunk_mirror[chunks[2 * k]] = chunks[2 * k + 1];
   w->pool_words = used * 512u;
-  if (!oaddr.empty()) VT_HIP(vt::finish_freemap(w));
+  if (w->occ) vt::finish_freemap(w);
   return VT_OK;
 }
 
@@ -355,65 +406,61 @@ int set_dense(vt_world* w, const uint32_t* xyz, const uint32_t* values, uint32_t
       return fail(VT_ERR_INVALID_ARGUMENT, "vt_world_set_voxels: dense value %u > 255 (edit %u)",
                   values[i], i);
   std::unordered_map<uint64_t, uint32_t> last;
-  std::vector<uint64_t> addr;
-  std::vector<uint32_t> val, bricks, regions, regions8;
+  std::vector<uint32_t> words, bricks, regions, regions8;
   last.reserve(n);
+  words.reserve(2 * (size_t)n);
   grow_box_by(w, xyz, values, n);
   for (uint32_t i = 0; i < n; i++) {
     const uint32_t code =
         morton_code(xyz[3 * (size_t)i], xyz[3 * (size_t)i + 1], xyz[3 * (size_t)i + 2]);
     auto it = last.find(code);
     if (it == last.end()) {
-      last.emplace(code, (uint32_t)addr.size());
-      addr.push_back(code);
-      val.push_back(values[i]);
+      last.emplace(code, (uint32_t)(words.size() / 2u));
+      words.insert(words.end(), {code, values[i]});
       bricks.push_back(code >> 6);
-      regions.push_back(code >> 12);
-      regions8.push_back(code >> 15);
     } else {
-      val[it->second] = values[i];
+      words[2 * (size_t)it->second + 1] = values[i];
     }
   }
-  std::sort(bricks.begin(), bricks.end());
-  bricks.erase(std::unique(bricks.begin(), bricks.end()), bricks.end());
-  std::sort(regions.begin(), regions.end());
-  regions.erase(std::unique(regions.begin(), regions.end()), regions.end());
-  std::sort(regions8.begin(), regions8.end());
-  regions8.erase(std::unique(regions8.begin(), regions8.end()), regions8.end());
-  Staging stg;
-  uint64_t* d_addr;
-  uint32_t *d_val, *d_bricks, *d_regions, *d_regions8;
-  VT_HIP(stg.upload(addr, &d_addr, s));
-  VT_HIP(stg.upload(val, &d_val, s));
-  VT_HIP(stg.upload(bricks, &d_bricks, s));
-  VT_HIP(stg.upload(regions, &d_regions, s));
-  VT_HIP(stg.upload(regions8, &d_regions8, s));
-  if (!addr.empty()) {
-    hipLaunchKernelGGL(vt::k_scatter_u8, dim3(blocks_for(addr.size(), 256)), dim3(256), 0, s,
-                       w->vox, d_addr, d_val, (uint32_t)addr.size());
-    hipLaunchKernelGGL((vt::k_rebuild_mask<uint8_t>), dim3(blocks_for(bricks.size(), 4)),
-                       dim3(256), 0, s, w->vox, w->l0, d_bricks, (uint32_t)bricks.size());
-    hipLaunchKernelGGL((vt::k_rebuild_mask<uint64_t>), dim3(blocks_for(regions.size(), 4)),
-                       dim3(256), 0, s, w->l0, w->l1, d_regions, (uint32_t)regions.size());
-    VT_HIP(vt::launch_build_l1b(w->l0, (uint64_t)w->dim * w->dim * w->dim / 64u, d_regions8,
-                                (uint32_t)regions8.size(), w->l1b, s));
-    VT_HIP(vt::rebuild_freemap(w, s));
+  sort_unique(bricks);
+  for (const uint32_t b : bricks) {  // sorted, so equal neighbours only
+    if (regions.empty() || regions.back() != b >> 6) regions.push_back(b >> 6);
+    if (regions8.empty() || regions8.back() != b >> 9) regions8.push_back(b >> 9);
   }
+  const uint32_t nw = (uint32_t)(words.size() / 2u), nb = (uint32_t)bricks.size(),
+                 nr = (uint32_t)regions.size(), nr8 = (uint32_t)regions8.size();
+  words.insert(words.end(), bricks.begin(), bricks.end());
+  words.insert(words.end(), regions.begin(), regions.end());
+  words.insert(words.end(), regions8.begin(), regions8.end());
+  Lists lists(w->ctx, s);
+  VT_HIP(lists.put(words));
+  const uint32_t* d_bricks = lists.dev + 2 * (size_t)nw;
+  hipLaunchKernelGGL(vt::k_edit_dense, dim3(blocks_for(nw, 256)), dim3(256), 0, s, w->vox,
+                     lists.dev, nw, vt::freemap_changed(w));
+  hipLaunchKernelGGL((vt::k_rebuild_mask<uint8_t>), dim3(blocks_for(nb, 4)), dim3(256), 0, s,
+                     w->vox, w->l0, d_bricks, nb, (uint32_t*)nullptr);
+  hipLaunchKernelGGL((vt::k_rebuild_mask<uint64_t>), dim3(blocks_for(nr, 4)), dim3(256), 0, s,
+                     w->l0, w->l1, d_bricks + nb, nr, vt::freemap_changed(w));
   VT_HIP(hipGetLastError());
-  if (w->prefix && !addr.empty()) {  // keep the compact index current
+  VT_HIP(vt::launch_build_l1b(w->l0, (uint64_t)w->dim * w->dim * w->dim / 64u,
+                              d_bricks + nb + nr, nr8, w->l1b, s));
+  VT_HIP(vt::rebuild_freemap(w, s, vt::freemap_changed(w)));
+  if (w->prefix) {  // keep the compact index current
     const uint64_t nwords = (uint64_t)w->dim * w->dim * w->dim / 64u;
     const uint64_t ntiles = (nwords + 1023) / 1024;
     uint32_t* scratch = nullptr;
     VT_HIP(hipMalloc((void**)&scratch, (ntiles + 1) * 4));
-    stg.bufs.push_back(scratch);
-    VT_HIP(vt::launch_compact_prefix(w->l0, nwords, w->prefix, scratch, s));
+    hipError_t e = vt::launch_compact_prefix(w->l0, nwords, w->prefix, scratch, s);
     uint32_t total = 0;
-    VT_HIP(hipMemcpyAsync(&total, scratch + ntiles, 4, hipMemcpyDeviceToHost, s));
-    VT_HIP(hipStreamSynchronize(s));
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(&total, scratch + ntiles, 4, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    vt::dev_free(scratch);
+    VT_HIP(e);
     w->n_occupied = total;
   }
   VT_HIP(hipStreamSynchronize(s));
-  if (!addr.empty()) VT_HIP(vt::finish_freemap(w));
+  vt::finish_freemap(w);
   return VT_OK;
 }
 
@@ -430,8 +477,12 @@ int vt_world_set_voxels(vt_ctx* ctx, vt_world* world, const uint32_t* xyz,
   if (st != VT_OK || n == 0) return st;
   VT_HIP(hipSetDevice(ctx->device));
   const hipStream_t s = (hipStream_t)stream;
-  return world->kind == WorldKind::Dense ? set_dense(world, xyz, values, n, s)
-                                         : set_brickmap(world, xyz, values, n, s);
+  try {
+    return world->kind == WorldKind::Dense ? set_dense(world, xyz, values, n, s)
+                                           : set_brickmap(world, xyz, values, n, s);
+  } catch (const std::bad_alloc&) {  // the host lists; nothing written yet
+    return fail(VT_ERR_OUT_OF_MEMORY, "vt_world_set_voxels: host lists of %u edits", n);
+  }
 }
 
 int vt_world_get_voxels(vt_ctx* ctx, const vt_world* world, const uint32_t* xyz, uint32_t n,
@@ -443,12 +494,14 @@ int vt_world_get_voxels(vt_ctx* ctx, const vt_world* world, const uint32_t* xyz,
   if (st != VT_OK || n == 0) return st;
   VT_HIP(hipSetDevice(ctx->device));
   const hipStream_t s = (hipStream_t)stream;
-  // the context's staging: coordinates, then values, kCtxStageVoxels at a time
-  uint32_t* d_xyz = (uint32_t*)ctx->stage;
-  uint32_t* d_out = d_xyz + 3u * (size_t)kCtxStageVoxels;
+  // the context's staging: coordinates, then values, kCtxStageVoxels at a
+  // time, read and written in place by the kernel
+  char* host = (char*)ctx->stage;
+  uint32_t* d_xyz = (uint32_t*)ctx->stage_dev;
   for (uint32_t i0 = 0; i0 < n; i0 += kCtxStageVoxels) {
     const uint32_t m = std::min(n - i0, kCtxStageVoxels);
-    VT_HIP(hipMemcpyAsync(d_xyz, xyz + 3 * (size_t)i0, 12 * (size_t)m, hipMemcpyHostToDevice, s));
+    std::memcpy(host, xyz + 3 * (size_t)i0, 12 * (size_t)m);
+    uint32_t* d_out = d_xyz + 3 * (size_t)m;
     if (world->kind == WorldKind::Dense)
       hipLaunchKernelGGL(vt::k_gather_dense, dim3(blocks_for(m, 256)), dim3(256), 0, s,
                          vt::dense_view(world), d_xyz, m, d_out);
@@ -456,8 +509,8 @@ int vt_world_get_voxels(vt_ctx* ctx, const vt_world* world, const uint32_t* xyz,
       hipLaunchKernelGGL(vt::k_gather_brickmap, dim3(blocks_for(m, 256)), dim3(256), 0, s,
                          vt::brickmap_view(world), d_xyz, m, d_out);
     VT_HIP(hipGetLastError());
-    VT_HIP(hipMemcpyAsync(values + i0, d_out, 4 * (size_t)m, hipMemcpyDeviceToHost, s));
     VT_HIP(hipStreamSynchronize(s));
+    std::memcpy(values + i0, host + 12 * (size_t)m, 4 * (size_t)m);
   }
   return VT_OK;
 }
@@ -517,18 +570,20 @@ int vt_pick(vt_ctx* ctx, const vt_world* world, const vt_camera* camera, int32_t
   VT_HIP(hipSetDevice(ctx->device));
   const hipStream_t s = (hipStream_t)stream;
   const vt::ViewConsts v = vt::view_consts(camera, 1, 1);
-  vt_pick_result* d = (vt_pick_result*)ctx->stage;  // the context's staging
+  vt_pick_result* d = (vt_pick_result*)ctx->stage_dev;  // the context's staging
   if (world->kind == WorldKind::Dense) {
     vt::DenseWorld dw = vt::dense_view(world);
     dw.free_bytes = 0;  // the result reports traceMap's step count
     hipLaunchKernelGGL(vt::k_pick_dense, dim3(1), dim3(64), 0, s, dw, v, (int)max_steps, d);
-  } else
-    hipLaunchKernelGGL(vt::k_pick_brickmap, dim3(1), dim3(64), 0, s, vt::brickmap_view(world), v,
-                       (int)max_steps, d);
+  } else {
+    vt::BrickmapWorld bw = vt::brickmap_view(world);
+    if (bw.dim < 2u * (uint32_t)vt::kSkipLong) bw.occ = nullptr;  // as launch_render_brickmap
+    hipLaunchKernelGGL(vt::k_pick_brickmap, dim3(1), dim3(64), 0, s, bw, v, (int)max_steps, d);
+  }
   hipError_t e = hipGetLastError();
-  if (e == hipSuccess) e = hipMemcpyAsync(result, d, sizeof *d, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) return hip_fail(e, "vt_pick");
+  std::memcpy(result, ctx->stage, sizeof *result);
   return VT_OK;
 }
 

@@ -9,19 +9,42 @@
 #include "../../include/vt.h"
 #include "vt_trace.hpp"
 
-// Device staging owned by a context, allocated once by vt_create: the pick
-// result and the coordinates / values of vt_world_get_voxels (in chunks of
-// kCtxStageVoxels), so neither allocates per call.  Calls that use it
-// return only after their stream work is done, so calls made one after
+// Staging owned by a context, allocated once by vt_create: page-locked host
+// memory that kernels read and write in place.  It carries the edit lists of
+// vt_world_set_voxels (larger ones take device memory for the call), the
+// coordinates and values of vt_world_get_voxels (in chunks of
+// kCtxStageVoxels), the pick result, and what the host needs to know of a
+// rebuilt free-region map, so that small calls make no copies and no
+// allocations: a copy of a few bytes costs 11-13 us of its own, a kernel
+// with a synchronisation 11 us with the bytes on either side.  Calls that use
+// it return only after their stream work is done, so calls made one after
 // another on the context's thread never overlap on it.
 constexpr size_t kCtxStageBytes = 256u * 1024u;
 constexpr uint32_t kCtxStageVoxels = (uint32_t)(kCtxStageBytes / 16u);  // 12 B xyz + 4 B value
+constexpr size_t kCtxReportBytes = 256;  // after the staging: CtxReport
+
+// What the map builders report to the host (written by the device into the
+// context's staging, valid once the stream has synchronised).
+struct CtxReport {
+  uint32_t free_built;       // 0: no region had changed, the map was left as it is
+  uint32_t free_regions[8];  // else: free regions of each octant
+  int32_t box_lo[3], box_hi[3];  // box of the nonempty voxels; lo > hi: none
+};
+static_assert(sizeof(CtxReport) <= kCtxReportBytes, "CtxReport");
 
 struct vt_ctx {
   int device;
   int compute_units;
   char name[256];
-  void* stage;  // kCtxStageBytes of device memory, 256-byte aligned
+  void* stage;        // kCtxStageBytes + kCtxReportBytes of page-locked host memory
+  void* stage_dev;    // its device address
+  // (the report follows the staging)
+  CtxReport* report() const {
+    return reinterpret_cast<CtxReport*>(static_cast<char*>(stage) + kCtxStageBytes);
+  }
+  CtxReport* report_dev() const {
+    return reinterpret_cast<CtxReport*>(static_cast<char*>(stage_dev) + kCtxStageBytes);
+  }
 };
 
 enum class WorldKind { Dense, Brickmap };
@@ -47,8 +70,8 @@ struct vt_world {
   uint8_t* occ;            // block occupancy in Morton order (power-of-two dim)
   uint64_t* brick_bits;    // brickmap: bit per 4^3 brick of blocks, from occ
   // free-region map (dense worlds and power-of-two brickmap worlds)
-  uint32_t* freemap;       // 8 octants x free_words_per_octant(dim) words
-  uint8_t* free_tmp;       // 8 x free_regions(dim)^3 bytes of build scratch
+  uint32_t* freemap;       // 8 octants x free_words_per_octant(dim) words, then a
+                           // word edits set when a region empties or fills
   bool free_valid;         // the map matches the occupancy (finish_freemap)
   float free_frac;         // largest share of free regions over the 8 octants
   // the box of the nonempty voxels (dense) or blocks (reference layout),
@@ -110,7 +133,6 @@ struct TileShape {
 };
 
 DenseWorld dense_view(const vt_world* w);
-void scan_dense_box(const uint8_t* grid, uint32_t dim, vt_world* w);
 void scan_brickmap_box(const uint32_t* chunks, const uint32_t* pool, uint32_t dim, vt_world* w);
 void grow_box(vt_world* w, int32_t x, int32_t y, int32_t z);
 void reach_of(const vt_world* w, float* lo, float* hi);
@@ -141,15 +163,21 @@ hipError_t launch_render_brickmap(const BrickmapWorld& w, const ViewConsts& v,
 
 // World construction kernels.
 // occ[morton(b)] = (map_getVoxel(b) != 0) for every block b of a brickmap
-// world with y < y_end (0: all layers).
-hipError_t launch_build_occupancy(const BrickmapWorld& w, uint8_t* occ, hipStream_t stream,
-                                  uint32_t y_end = 0);
+// world (power-of-two dim) with y < y_end (0: all layers), and the brick
+// bits of those layers' 4^3 bricks (bits of a partly covered word are set
+// only, never cleared: the other layers' bits must be right already).
+hipError_t launch_build_occupancy(const BrickmapWorld& w, uint8_t* occ, uint64_t* brick_bits,
+                                  hipStream_t stream, uint32_t y_end = 0);
 // Grows a brickmap world's block pool to at least `blocks` blocks by
 // doubling (GpuBlockAllocator.alloc, gpu_block_allocator.zig:20-30), keeping
 // the contents and zeroing the new blocks; `who` names the caller in errors.
 int grow_pool(vt_world* w, uint64_t blocks, hipStream_t s, const char* who);
+// The Morton-ordered voxels of a linear grid and their occupancy levels, and
+// the box of the nonempty voxels into *report (which holds an empty box
+// before).
 hipError_t launch_build_dense(const uint8_t* linear, uint32_t dim, uint8_t* vox, uint64_t* l0,
-                              uint64_t* l1, uint64_t* l1b, hipStream_t stream);
+                              uint64_t* l1, uint64_t* l1b, int32_t* box6, CtxReport* report,
+                              hipStream_t stream);
 // Words of the 8^3-brick level of a dim^3 world: one per 32^3 region (one
 // partial word for dim 16).
 inline uint64_t l1b_words(uint32_t dim) {
@@ -164,19 +192,24 @@ hipError_t launch_build_l1b(const uint64_t* l0, uint64_t n0, const uint32_t* wor
 // bit r of octant o's bitmap (free_words_per_octant(dim) words) is set when
 // no region at or ahead of r on every axis in o's travel direction holds a
 // nonempty block.  Built from the brick bits (a dense world's L1 words, a
-// brickmap world's brick_bits) with 8 R^3 bytes of scratch.
+// brickmap world's brick_bits), unless *changed (device, may be null) is 0;
+// reports whether it was and the free regions of each octant.
 uint32_t free_regions(uint32_t dim);
 uint32_t free_words_per_octant(uint32_t dim);
-hipError_t launch_build_freemap(const uint64_t* l1, uint32_t dim, uint8_t* tmp, uint32_t* fm,
-                                hipStream_t stream);
+hipError_t launch_build_freemap(const uint64_t* l1, uint32_t dim, uint32_t* fm,
+                                const uint32_t* changed, CtxReport* report, hipStream_t stream);
 // Rebuilds a world's free-region map from its current occupancy (a dense
-// world's L1 words; a brickmap world's occupancy bytes); no-op without one.
-// Clears free_valid: the caller calls finish_freemap once the stream has
+// world's L1 words; a brickmap world's brick bits); no-op without one.
+// `changed`: as launch_build_freemap (null: always).  Clears free_valid: the caller calls finish_freemap once the stream has
 // synchronised without error, and until then the renderers do not read it.
-hipError_t rebuild_freemap(vt_world* w, hipStream_t stream);
-// After a rebuild completed: reads the map back to learn the largest share
-// of free regions over the octants (free_frac) and marks it valid.
-hipError_t finish_freemap(vt_world* w);
+hipError_t rebuild_freemap(vt_world* w, hipStream_t stream, const uint32_t* changed = nullptr);
+// The word edits set when a region empties or fills.
+inline uint32_t* freemap_changed(const vt_world* w) {
+  return w->freemap ? w->freemap + 8u * free_words_per_octant(w->dim) : nullptr;
+}
+// After a rebuild completed: takes the largest share of free regions over the
+// octants (free_frac) from the context's report and marks the map valid.
+void finish_freemap(vt_world* w);
 // Whether a launch with these constants tests the free-region map: the map
 // is valid and has a free region, and VT_FLAG_FREE_MAP_ON, or neither
 // FREE_MAP flag, a step cap of at least VT_FREE_MIN_CAP and at least
@@ -189,11 +222,8 @@ bool use_free_map(const vt_world* w, const ShadeConsts& sc);
 // the steps executed); on the reference layout occupancy bytes and no
 // statistics.
 bool render_free_map(const vt_world* w, const vt_render_params& p, const vt_frame& f);
-// Brick bits (one uint64 per 4096 codes) of a Morton-ordered byte array of
-// dim^3 bytes; brick_bit_words(dim) words.
+// Words of a brickmap world's brick bits: one uint64 per 4096 codes.
 uint32_t brick_bit_words(uint32_t dim);
-hipError_t launch_brick_bits(const uint8_t* bytes, uint32_t dim, uint64_t* l1,
-                             hipStream_t stream);
 // Exclusive prefix sum of popcount(l0[i]) into prefix[0..nwords); scratch
 // holds ceil(nwords/1024) + 1 words; *total receives the sum (device).
 hipError_t launch_compact_prefix(const uint64_t* l0, uint64_t nwords, uint32_t* prefix,

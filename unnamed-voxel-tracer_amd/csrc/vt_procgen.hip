@@ -396,7 +396,7 @@ int vt_world_procgen(vt_ctx* ctx, vt_world* world, float offset_x, float offset_
   }
   // the empty map's occupancy bytes were zero; only the written layers change
   if (e == hipSuccess && world->occ)
-    e = vt::launch_build_occupancy(vt::brickmap_view(world), world->occ, s,
+    e = vt::launch_build_occupancy(vt::brickmap_view(world), world->occ, world->brick_bits, s,
                                    std::min(dim, (walk.y_end + 7u) & ~7u));
   if (e == hipSuccess) e = vt::rebuild_freemap(world, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
@@ -405,7 +405,10 @@ int vt_world_procgen(vt_ctx* ctx, vt_world* world, float offset_x, float offset_
     // blocks and occupancy bytes zero
     (void)hipMemsetAsync(world->chunks, 0, nchunks * 4, s);
     (void)hipMemsetAsync(world->pool, 0, walk.used * 512u * 4u, s);
-    if (world->occ) (void)hipMemsetAsync(world->occ, 0, (size_t)dim * dim * dim, s);
+    if (world->occ) {
+      (void)hipMemsetAsync(world->occ, 0, (size_t)dim * dim * dim, s);
+      (void)hipMemsetAsync(world->brick_bits, 0, (size_t)vt::brick_bit_words(dim) * 8u, s);
+    }
     (void)hipStreamSynchronize(s);
     (void)hipGetLastError();
     return vt::hip_fail(e, "vt_world_procgen: device writes");
@@ -413,7 +416,7 @@ int vt_world_procgen(vt_ctx* ctx, vt_world* world, float offset_x, float offset_
   std::memcpy(world->chunk_mirror, walk.mirror.data(), nchunks * 4);
   world->pool_words = walk.used * 512u;
   vt::scan_brickmap_box(world->chunk_mirror, nullptr, dim, world);  // chunk granularity
-  VT_HIP(vt::finish_freemap(world));
+  vt::finish_freemap(world);
   return VT_OK;
 }
 

@@ -7,47 +7,118 @@
 // 16^3 region, bit = brick index & 63 set when the brick has a solid voxel),
 // L1b = one uint64 per 32768 codes (a 32^3 region, bit per 8^3 brick).
 #include <algorithm>
-#include <vector>
 
 #include "vt_internal.hpp"
 
 namespace vt {
 
-// One thread per 4 consecutive codes (one 32-bit store).
-__global__ __launch_bounds__(256) void k_build_morton(const uint8_t* __restrict__ lin,
-                                                      uint32_t dim, uint8_t* __restrict__ vox) {
-  const uint64_t n = (uint64_t)dim * dim * dim;
-  const uint64_t c0 = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4u;
-  if (c0 >= n) return;
-  uint32_t word = 0;
-#pragma unroll
-  for (uint32_t k = 0; k < 4; k++) {
-    const uint32_t c = (uint32_t)c0 + k;
-    const uint32_t x = compact1by2(c), y = compact1by2(c >> 1), z = compact1by2(c >> 2);
-    const uint32_t b = lin[(uint64_t)x + (uint64_t)dim * ((uint64_t)y + (uint64_t)dim * z)];
-    word |= b << (8 * k);
-  }
-  *reinterpret_cast<uint32_t*>(vox + c0) = word;
-}
-
-// One thread per L0 word: 64 consecutive Morton bytes.
-__global__ __launch_bounds__(256) void k_build_l0(const uint8_t* __restrict__ vox, uint64_t nwords,
-                                                  uint64_t* __restrict__ l0) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nwords) return;
-  const uint4* src = reinterpret_cast<const uint4*>(vox + i * 64u);
+// The 64 Morton bytes of a 4^3 brick from its 16 rows of 4 voxels (row
+// [4 z + y], x in the byte order).  Byte code bits are x0 y0 z0 x1 y1 z1, so
+// the 32-bit word (z0, x1, y1, z1) takes two half words of rows 2 y1 and
+// 2 y1 + 1 of layer 2 z1 + z0.  Returns the brick's occupancy word.
+__device__ __forceinline__ uint64_t morton_brick(const uint32_t row[16], uint32_t out[16]) {
   uint64_t mask = 0;
 #pragma unroll
-  for (int q = 0; q < 4; q++) {
-    const uint4 v = src[q];
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int j = 0; j < 4; j++)
-#pragma unroll
-      for (int b = 0; b < 4; b++)
-        if ((w[j] >> (8 * b)) & 255u) mask |= 1ull << (q * 16 + j * 4 + b);
+  for (uint32_t w = 0; w < 16u; w++) {
+    const uint32_t z = (w & 1u) | ((w >> 3) << 1), x1 = (w >> 1) & 1u, y1 = (w >> 2) & 1u;
+    const uint32_t a = row[4u * z + 2u * y1], b = row[4u * z + 2u * y1 + 1u];
+    const uint32_t v = x1 ? (a >> 16) | (b & 0xFFFF0000u) : (a & 0xFFFFu) | (b << 16);
+    out[w] = v;
+    uint32_t y = v | (v >> 4);  // bit k = byte k is nonzero
+    y |= y >> 2;
+    y |= y >> 1;
+    y &= 0x01010101u;
+    mask |= (uint64_t)((y | (y >> 7) | (y >> 14) | (y >> 21)) & 15u) << (4u * w);
   }
-  l0[i] = mask;
+  return mask;
+}
+
+// One thread per 4^3 brick: 16 rows of 4 voxels in (a wave's rows are
+// contiguous along x), 64 Morton bytes and the L0 word out (two bricks a
+// 128-byte line).  Bound by HBM: 2 bytes a voxel and 1/8 byte of L0.  512^3:
+// 262 us as one thread per 4 codes (4-byte gathers of bytes) with a second
+// pass for L0, 64 us here.
+__global__ __launch_bounds__(256) void k_build_bricks(const uint8_t* __restrict__ lin,
+                                                      uint32_t log2n, uint8_t* __restrict__ vox,
+                                                      uint64_t* __restrict__ l0) {
+  const uint32_t n = 1u << log2n;  // bricks per axis
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= 1u << (3u * log2n)) return;
+  const uint32_t bx = i & (n - 1u), by = (i >> log2n) & (n - 1u), bz = i >> (2u * log2n);
+  const size_t dim = 4u * (size_t)n;
+  const uint8_t* src = lin + 4u * bx + dim * (4u * by + dim * (4u * (size_t)bz));
+  uint32_t row[16], out[16];
+#pragma unroll
+  for (uint32_t k = 0; k < 16u; k++)
+    row[k] = *reinterpret_cast<const uint32_t*>(src + dim * ((k & 3u) + dim * (k >> 2)));
+  const uint64_t mask = morton_brick(row, out);
+  const uint32_t c = morton3(bx, by, bz);
+  uint4* dst = reinterpret_cast<uint4*>(vox + 64u * (size_t)c);
+#pragma unroll
+  for (uint32_t q = 0; q < 4u; q++)
+    dst[q] = make_uint4(out[4 * q], out[4 * q + 1], out[4 * q + 2], out[4 * q + 3]);
+  l0[c] = mask;
+}
+
+// The box of the nonempty voxels from the L0 words: grid-stride, a sum over
+// the block first, so that the atomics on box6 (lo, then hi) stay few.
+__global__ __launch_bounds__(256) void k_box(const uint64_t* __restrict__ l0, uint32_t nwords,
+                                             int32_t* __restrict__ box6) {
+  // bits of a word whose voxel has x / y / z = k (x in code bits 0 and 3)
+  constexpr uint64_t X0 = 0x0055005500550055ull, Y0 = 0x0000333300003333ull,
+                     Z0 = 0x000000000F0F0F0Full;
+  constexpr uint64_t at[3][4] = {{X0, X0 << 1, X0 << 8, X0 << 9},
+                                 {Y0, Y0 << 2, Y0 << 16, Y0 << 18},
+                                 {Z0, Z0 << 4, Z0 << 32, Z0 << 36}};
+  int lo[3] = {1 << 20, 1 << 20, 1 << 20}, hi[3] = {-1, -1, -1};
+  for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < nwords; i += gridDim.x * 256u) {
+    const uint64_t w = l0[i];
+    if (w == 0ull) continue;
+    const int base[3] = {4 * (int)compact1by2(i), 4 * (int)compact1by2(i >> 1),
+                         4 * (int)compact1by2(i >> 2)};
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+#pragma unroll
+      for (int k = 0; k < 4; k++)
+        if (w & at[a][k]) {
+          lo[a] = min(lo[a], base[a] + k);
+          hi[a] = max(hi[a], base[a] + k);
+        }
+    }
+  }
+  __shared__ int32_t part[6];
+  if (threadIdx.x < 6u) part[threadIdx.x] = threadIdx.x < 3u ? 1 << 20 : -1;
+  __syncthreads();
+#pragma unroll
+  for (int a = 0; a < 3; a++) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      lo[a] = min(lo[a], __shfl_xor(lo[a], off, 64));
+      hi[a] = max(hi[a], __shfl_xor(hi[a], off, 64));
+    }
+    if ((threadIdx.x & 63u) == 0u && hi[a] >= 0) {
+      atomicMin(&part[a], lo[a]);
+      atomicMax(&part[3 + a], hi[a]);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 6u && part[3] >= 0) {
+    if (threadIdx.x < 3u)
+      atomicMin(&box6[threadIdx.x], part[threadIdx.x]);
+    else
+      atomicMax(&box6[threadIdx.x], part[threadIdx.x]);
+  }
+}
+
+__global__ void k_box_clear(int32_t* __restrict__ box6) {
+  if (threadIdx.x < 6u) box6[threadIdx.x] = threadIdx.x < 3u ? 1 << 20 : -1;
+}
+
+__global__ void k_box_report(const int32_t* __restrict__ box6, CtxReport* __restrict__ report) {
+  if (threadIdx.x < 3u) {
+    report->box_lo[threadIdx.x] = box6[threadIdx.x];
+    report->box_hi[threadIdx.x] = box6[3u + threadIdx.x];
+  }
 }
 
 // One thread per L1 word: 64 consecutive L0 words.
@@ -182,19 +253,24 @@ hipError_t launch_compact_prefix(const uint64_t* l0, uint64_t nwords, uint32_t* 
 }
 
 hipError_t launch_build_dense(const uint8_t* linear, uint32_t dim, uint8_t* vox, uint64_t* l0,
-                              uint64_t* l1, uint64_t* l1b, hipStream_t stream) {
+                              uint64_t* l1, uint64_t* l1b, int32_t* box6, CtxReport* report,
+                              hipStream_t stream) {
   const uint64_t n = (uint64_t)dim * dim * dim;  // a power of two >= 4096
-  const uint64_t n0 = n / 64u, n1 = n / 4096u;
-  hipLaunchKernelGGL(k_build_morton, dim3((uint32_t)((n / 4u + 255) / 256)), dim3(256), 0, stream,
-                     linear, dim, vox);
+  const uint32_t n0 = (uint32_t)(n / 64u), n1 = (uint32_t)(n / 4096u);
+  uint32_t log2n = 0;
+  while ((4u << log2n) < dim) log2n++;
+  hipLaunchKernelGGL(k_build_bricks, dim3((n0 + 255u) / 256u), dim3(256), 0, stream, linear, log2n,
+                     vox, l0);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_build_l0, dim3((uint32_t)((n0 + 255) / 256)), dim3(256), 0, stream, vox, n0,
-                     l0);
+  hipLaunchKernelGGL(k_build_l1, dim3((n1 + 255u) / 256u), dim3(256), 0, stream, l0, (uint64_t)n1,
+                     l1);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_build_l1, dim3((uint32_t)((n1 + 255) / 256)), dim3(256), 0, stream, l0, n1,
-                     l1);
+  hipLaunchKernelGGL(k_box_clear, dim3(1), dim3(64), 0, stream, box6);
+  hipLaunchKernelGGL(k_box, dim3(std::min((n0 + 255u) / 256u, 256u)), dim3(256), 0, stream, l0, n0,
+                     box6);
+  hipLaunchKernelGGL(k_box_report, dim3(1), dim3(64), 0, stream, box6, report);
   e = hipGetLastError();
   if (e != hipSuccess) return e;
   return launch_build_l1b(l0, n0, nullptr, (uint32_t)l1b_words(dim), l1b, stream);
@@ -208,70 +284,105 @@ hipError_t launch_build_dense(const uint8_t* linear, uint32_t dim, uint8_t* vox,
 // o's bitmap is free_o(r).  The traversal loops read it to end a ray that can
 // hit nothing more.
 
-// One thread per region (linear index rx + R (ry + R rz)); writes whether the
-// region holds a nonempty brick into all 8 octant planes of tmp.
-__global__ __launch_bounds__(256) void k_free_regions(const uint64_t* __restrict__ l1, uint32_t R,
-                                                      uint8_t* __restrict__ tmp) {
-  const uint32_t n = R * R * R;
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t rx = i % R, ry = (i / R) % R, rz = i / (R * R);
-  const uint8_t v = l1[morton3(rx, ry, rz)] != 0ull ? 1 : 0;
-  for (uint32_t o = 0; o < 8; o++) tmp[(size_t)o * n + i] = v;
-}
-
-// One thread per (octant, line along `axis`): each region becomes the OR of
-// itself and every region ahead of it on that axis in the octant's travel
-// direction.  Three passes (x, y, z) give the forward-orthant OR.
-__global__ __launch_bounds__(256) void k_free_scan(uint8_t* __restrict__ tmp, uint32_t R,
-                                                   int axis) {
-  const uint32_t lines = R * R, n = lines * R;
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= 8u * lines) return;
-  const uint32_t o = t / lines, l = t % lines;
-  const uint32_t u = l % R, v = l / R;
-  size_t base, stride;
-  if (axis == 0) {
-    base = (size_t)R * (u + (size_t)R * v);
-    stride = 1;
-  } else if (axis == 1) {
-    base = u + (size_t)lines * v;
-    stride = R;
-  } else {
-    base = u + (size_t)R * v;
-    stride = lines;
-  }
-  uint8_t* p = tmp + (size_t)o * n + base;
-  uint8_t acc = 0;
-  if (((o >> axis) & 1u) == 0u) {  // positive: ahead = higher index
-    for (int k = (int)R - 1; k >= 0; --k) {
-      acc |= p[(size_t)k * stride];
-      p[(size_t)k * stride] = acc;
+// One block per octant, the regions as bit rows along x in LDS (R = 1 << lg,
+// at most 64 rows of 64 bits a layer, 32 KiB).  A row's bit x becomes the OR
+// of the regions at or ahead of x by shifts; along y and z the rows take the
+// OR of rows 1, 2, 4, ... ahead.  Then bit j of word w of the octant's bitmap
+// = the region with Morton code 32 w + j is free.  Bound by the one CU a block
+// has: 16 us at 512^3 (five kernels over byte planes: 36).  An edit rarely
+// empties or fills a whole region, so it passes `changed` (device word: a
+// region did) and the launch ends at once, in 3 us, when none did.
+__global__ __launch_bounds__(1024) void k_free_map(const uint64_t* __restrict__ l1, uint32_t lg,
+                                                   uint32_t words, uint32_t* __restrict__ fm,
+                                                   const uint32_t* __restrict__ changed,
+                                                   CtxReport* __restrict__ report) {
+  const bool run = !changed || *changed != 0u;
+  if (blockIdx.x == 0u && threadIdx.x == 0u) report->free_built = run ? 1u : 0u;
+  if (!run) return;  // the same for every thread
+  __shared__ uint64_t row[4096];
+  __shared__ uint32_t total;
+  const uint32_t R = 1u << lg, rows = R << lg, n = rows << lg;
+  const uint32_t o = blockIdx.x, t = threadIdx.x;
+  if (t == 0u) total = 0u;
+  const uint64_t full = R == 64u ? ~0ull : (1ull << R) - 1ull;
+  for (uint32_t r = t; r < rows; r += 1024u) row[r] = 0ull;
+  __syncthreads();
+  // eight consecutive codes (2^3 regions) a thread: two bits of four rows
+  uint32_t* half = reinterpret_cast<uint32_t*>(row);
+  for (uint32_t g = t; g < (n >= 8u ? n / 8u : 1u); g += 1024u) {
+    uint32_t any = 0u;
+    if (n >= 8u) {
+      const uint4* p = reinterpret_cast<const uint4*>(l1 + 8u * (size_t)g);
+#pragma unroll
+      for (uint32_t k = 0; k < 4u; k++) {
+        const uint4 q = p[k];
+        any |= ((q.x | q.y) ? 1u : 0u) << (2u * k) | ((q.z | q.w) ? 2u : 0u) << (2u * k);
+      }
+    } else {
+      any = l1[0] != 0ull ? 1u : 0u;  // R = 1
     }
-  } else {
-    for (uint32_t k = 0; k < R; ++k) {
-      acc |= p[(size_t)k * stride];
-      p[(size_t)k * stride] = acc;
+    const uint32_t x = 2u * compact1by2(g), y = 2u * compact1by2(g >> 1),
+                   z = 2u * compact1by2(g >> 2);
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; k++) {
+      const uint32_t two = (any >> (2u * k)) & 3u;
+      if (two) {
+        const uint32_t r = (y + (k & 1u)) + ((z + (k >> 1)) << lg);
+        atomicOr(&half[2u * r + (x >> 5)], two << (x & 31u));
+      }
     }
   }
-}
-
-// One thread per (octant, bitmap word): bit j of word w = free_o(region with
-// Morton code 32 w + j).
-__global__ __launch_bounds__(256) void k_free_pack(const uint8_t* __restrict__ tmp, uint32_t R,
-                                                   uint32_t words, uint32_t* __restrict__ fm) {
-  const uint32_t n = R * R * R;
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= 8u * words) return;
-  const uint32_t o = t / words, wi = t % words;
-  uint32_t bits = 0;
-  for (uint32_t j = 0; j < 32; j++) {
-    const uint32_t rc = wi * 32u + j;
-    if (rc >= n) break;
-    const uint32_t x = compact1by2(rc), y = compact1by2(rc >> 1), z = compact1by2(rc >> 2);
-    if (!tmp[(size_t)o * n + x + (size_t)R * (y + (size_t)R * z)]) bits |= 1u << j;
+  __syncthreads();
+  // along x: each row by itself
+  for (uint32_t r = t; r < rows; r += 1024u) {
+    uint64_t v = row[r];
+#pragma unroll
+    for (uint32_t s = 1; s < 64u; s <<= 1) v |= (o & 1u) ? v << s : v >> s;
+    row[r] = v & full;
   }
-  fm[t] = bits;
+  __syncthreads();
+  for (uint32_t axis = 1; axis < 3u; axis++) {
+    const uint32_t sh = axis == 1u ? 0u : lg;  // log2 of the row stride
+    const bool neg = ((o >> axis) & 1u) != 0u;
+    for (uint32_t s = 1; s < R; s <<= 1) {
+      uint64_t v[4] = {0, 0, 0, 0};
+#pragma unroll
+      for (uint32_t k = 0; k < 4u; k++) {
+        const uint32_t r = t + 1024u * k, c = (r >> sh) & (R - 1u);
+        if (r < rows && (neg ? c >= s : c + s < R))
+          v[k] = row[neg ? r - (s << sh) : r + (s << sh)];
+      }
+      __syncthreads();
+#pragma unroll
+      for (uint32_t k = 0; k < 4u; k++)
+        if (t + 1024u * k < rows) row[t + 1024u * k] |= v[k];
+      __syncthreads();
+    }
+  }
+  uint32_t sum = 0;
+  for (uint32_t w = t; w < words; w += 1024u) {
+    // 32 regions: x 4, y 4, z 2 of them (code bits x0 y0 z0 x1 y1); fewer in
+    // the one word of a map with R < 4
+    const uint32_t c = w * 32u;
+    const uint32_t x = compact1by2(c), y = compact1by2(c >> 1), z = compact1by2(c >> 2);
+    uint32_t bits = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < 8u; k++) {
+      const uint32_t dy = (k & 1u) | (k & 2u), dz = k >> 2;
+      if (y + dy >= R || z + dz >= R) continue;
+      const uint32_t q = (uint32_t)(~row[(y + dy) + ((z + dz) << lg)] >> x);
+#pragma unroll
+      for (uint32_t dx = 0; dx < 4u; dx++)
+        if (x + dx < R)
+          bits |= ((q >> dx) & 1u)
+                  << ((dx & 1u) | ((dy & 1u) << 1) | (dz << 2) | ((dx >> 1) << 3) | ((dy >> 1) << 4));
+    }
+    fm[o * words + w] = bits;
+    sum += (uint32_t)__popc(bits);
+  }
+  if (sum) atomicAdd(&total, sum);
+  __syncthreads();
+  if (t == 0u) report->free_regions[o] = total;
 }
 
 uint32_t free_regions(uint32_t dim) { return dim >= 16u ? dim / 16u : 1u; }
@@ -281,43 +392,13 @@ uint32_t free_words_per_octant(uint32_t dim) {
   return (R * R * R + 31u) / 32u;
 }
 
-hipError_t launch_build_freemap(const uint64_t* l1, uint32_t dim, uint8_t* tmp, uint32_t* fm,
-                                hipStream_t stream) {
-  const uint32_t R = free_regions(dim), n = R * R * R, words = free_words_per_octant(dim);
-  hipLaunchKernelGGL(k_free_regions, dim3((n + 255u) / 256u), dim3(256), 0, stream, l1, R, tmp);
-  hipError_t e = hipGetLastError();
-  for (int axis = 0; axis < 3 && e == hipSuccess; axis++) {
-    hipLaunchKernelGGL(k_free_scan, dim3((8u * R * R + 255u) / 256u), dim3(256), 0, stream, tmp,
-                       R, axis);
-    e = hipGetLastError();
-  }
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_free_pack, dim3((8u * words + 255u) / 256u), dim3(256), 0, stream, tmp, R,
-                     words, fm);
+hipError_t launch_build_freemap(const uint64_t* l1, uint32_t dim, uint32_t* fm,
+                                const uint32_t* changed, CtxReport* report, hipStream_t stream) {
+  uint32_t lg = 0;
+  while ((1u << lg) < free_regions(dim)) lg++;
+  hipLaunchKernelGGL(k_free_map, dim3(8), dim3(1024), 0, stream, l1, lg,
+                     free_words_per_octant(dim), fm, changed, report);
   return hipGetLastError();
-}
-
-// Brick bits of a Morton-ordered byte array (the brickmap occupancy bytes):
-// one uint64 per 4096 codes, bit j set when bytes [64 (64 w + j), +64) hold
-// a nonzero byte.  One wave per word; an 8^3 map has one partial word.
-__global__ __launch_bounds__(256) void k_brick_bits(const uint8_t* __restrict__ bytes,
-                                                    uint64_t nbytes, uint32_t nwords,
-                                                    uint64_t* __restrict__ l1) {
-  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const uint32_t lane = threadIdx.x & 63u;
-  if (wave >= nwords) return;  // whole waves leave together
-  const uint64_t first = ((uint64_t)wave * 64u + lane) * 64u;
-  bool any = false;
-  if (first < nbytes) {
-    const uint4* s = reinterpret_cast<const uint4*>(bytes + first);
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const uint4 v = s[q];
-      any |= (v.x | v.y | v.z | v.w) != 0u;
-    }
-  }
-  const uint64_t m = __ballot(any);
-  if (lane == 0) l1[wave] = m;
 }
 
 uint32_t brick_bit_words(uint32_t dim) {
@@ -325,39 +406,25 @@ uint32_t brick_bit_words(uint32_t dim) {
   return n >= 4096u ? (uint32_t)(n / 4096u) : 1u;
 }
 
-hipError_t launch_brick_bits(const uint8_t* bytes, uint32_t dim, uint64_t* l1,
-                             hipStream_t stream) {
-  const uint32_t nwords = brick_bit_words(dim);
-  hipLaunchKernelGGL(k_brick_bits, dim3((nwords + 3u) / 4u), dim3(256), 0, stream, bytes,
-                     (uint64_t)dim * dim * dim, nwords, l1);
-  return hipGetLastError();
-}
-
-hipError_t rebuild_freemap(vt_world* w, hipStream_t stream) {
+hipError_t rebuild_freemap(vt_world* w, hipStream_t stream, const uint32_t* changed) {
+  if (!w->free_valid) changed = nullptr;  // whatever the map holds is not current
   w->free_valid = false;
   if (!w->freemap) return hipSuccess;
-  if (w->kind == WorldKind::Dense) return launch_build_freemap(w->l1, w->dim, w->free_tmp,
-                                                               w->freemap, stream);
-  hipError_t e = launch_brick_bits(w->occ, w->dim, w->brick_bits, stream);
-  if (e != hipSuccess) return e;
-  return launch_build_freemap(w->brick_bits, w->dim, w->free_tmp, w->freemap, stream);
+  return launch_build_freemap(w->kind == WorldKind::Dense ? w->l1 : w->brick_bits, w->dim,
+                              w->freemap, changed, w->ctx->report_dev(), stream);
 }
 
-hipError_t finish_freemap(vt_world* w) {
+void finish_freemap(vt_world* w) {
   w->free_valid = false;
-  w->free_frac = 0.0f;
-  if (!w->freemap) return hipSuccess;
-  const uint32_t words = free_words_per_octant(w->dim), R = free_regions(w->dim);
-  std::vector<uint32_t> h(8u * (size_t)words);
-  const hipError_t e = hipMemcpy(h.data(), w->freemap, h.size() * 4, hipMemcpyDeviceToHost);
-  if (e != hipSuccess) return e;
-  for (uint32_t o = 0; o < 8; o++) {
-    uint64_t n = 0;
-    for (uint32_t i = 0; i < words; i++) n += (uint64_t)__builtin_popcount(h[o * words + i]);
-    w->free_frac = std::max(w->free_frac, (float)((double)n / ((double)R * R * R)));
+  if (!w->freemap) return;
+  const CtxReport* r = w->ctx->report();
+  if (r->free_built) {
+    const double R = free_regions(w->dim);
+    w->free_frac = 0.0f;
+    for (uint32_t o = 0; o < 8; o++)
+      w->free_frac = std::max(w->free_frac, (float)((double)r->free_regions[o] / (R * R * R)));
   }
   w->free_valid = true;
-  return hipSuccess;
 }
 
 bool use_free_map(const vt_world* w, const ShadeConsts& sc) {
@@ -368,24 +435,60 @@ bool use_free_map(const vt_world* w, const ShadeConsts& sc) {
          w->free_frac * VT_FREE_MIN_SHARE >= 1.0f;
 }
 
-// One thread per block of the layers y < y_end of a brickmap world (linear
-// order x + dim*(y + y_end*z)).
+// One thread per 4^3 brick of the layers y < 4 ny: a brick lies in one chunk,
+// so one chunk-table read and 16 rows of 4 pool words make its 64 occupancy
+// bytes (Morton order).  A whole 512^3 map, mostly empty chunks: 384 us as
+// one thread per block, 45 us here.
 __global__ __launch_bounds__(256) void k_build_occupancy(BrickmapWorld w, uint8_t* __restrict__ occ,
-                                                         uint32_t y_end) {
+                                                         uint64_t* __restrict__ brick_bits,
+                                                         uint32_t ny) {
+  const uint32_t nb = w.dim / 4u;
   const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const uint64_t n = (uint64_t)w.dim * y_end * w.dim;
-  if (i >= n) return;
-  const uint32_t x = (uint32_t)(i % w.dim), y = (uint32_t)((i / w.dim) % y_end),
-                 z = (uint32_t)(i / ((uint64_t)w.dim * y_end));
-  occ[morton3(x, y, z)] = bm_block(w, (int)x, (int)y, (int)z) != 0u ? 1 : 0;
+  if (i >= (uint64_t)nb * ny * nb) return;
+  const uint32_t bx = (uint32_t)(i % nb), by = (uint32_t)(i / nb % ny),
+                 bz = (uint32_t)(i / ((uint64_t)nb * ny));
+  const uint32_t M = w.dim / 8u;
+  const uint32_t c = morton3(bx, by, bz);
+  const uint32_t e = w.chunks[bx / 2u + M * (by / 2u + (size_t)(bz / 2u) * M)];
+  uint32_t out[16] = {};
+  uint64_t mask = 0;
+  if (e != 0u) {
+    const uint32_t* src = w.pool + (size_t)(e - 1u) * 512u + 4u * (bx & 1u) + 32u * (by & 1u) +
+                          256u * (bz & 1u);
+    uint32_t row[16];
+#pragma unroll
+    for (uint32_t k = 0; k < 16u; k++) {
+      const uint4 v = *reinterpret_cast<const uint4*>(src + 8u * (k & 3u) + 64u * (k >> 2));
+      row[k] = (v.x ? 1u : 0u) | (v.y ? 0x100u : 0u) | (v.z ? 0x10000u : 0u) |
+               (v.w ? 0x1000000u : 0u);
+    }
+    mask = morton_brick(row, out);
+  }
+  uint4* dst = reinterpret_cast<uint4*>(occ + 64u * (size_t)c);
+#pragma unroll
+  for (uint32_t q = 0; q < 4u; q++)
+    dst[q] = make_uint4(out[4 * q], out[4 * q + 1], out[4 * q + 2], out[4 * q + 3]);
+  if (mask)
+    atomicOr(reinterpret_cast<unsigned long long*>(brick_bits + (c >> 6)), 1ull << (c & 63u));
 }
 
-hipError_t launch_build_occupancy(const BrickmapWorld& w, uint8_t* occ, hipStream_t stream,
-                                  uint32_t y_end) {
+__global__ __launch_bounds__(256) void k_clear_words(uint64_t* __restrict__ p, uint32_t n) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i < n) p[i] = 0ull;
+}
+
+hipError_t launch_build_occupancy(const BrickmapWorld& w, uint8_t* occ, uint64_t* brick_bits,
+                                  hipStream_t stream, uint32_t y_end) {
   if (y_end == 0 || y_end > w.dim) y_end = w.dim;
-  const uint64_t n = (uint64_t)w.dim * y_end * w.dim;
+  if (y_end == w.dim) {
+    const uint32_t nwords = brick_bit_words(w.dim);
+    hipLaunchKernelGGL(k_clear_words, dim3((nwords + 255u) / 256u), dim3(256), 0, stream,
+                       brick_bits, nwords);
+  }
+  const uint32_t ny = (y_end + 3u) / 4u;
+  const uint64_t n = (uint64_t)(w.dim / 4u) * ny * (w.dim / 4u);
   hipLaunchKernelGGL(k_build_occupancy, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, stream, w,
-                     occ, y_end);
+                     occ, brick_bits, ny);
   return hipGetLastError();
 }
 
