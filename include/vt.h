@@ -84,19 +84,23 @@ typedef struct vt_camera {
                                       /* vignette of blit.fragment.glsl:32-35 */
                                       /* (not with LAMBERT); frame.display,   */
                                       /* when set, gets it as RGBA8           */
-/* Free-region test (flat traversal of dense worlds; brickmap worlds with a
- * power-of-two dim).  The library keeps, per world, a bitmap of the 16^3
- * regions from which no ray of a given direction octant can meet a nonempty
- * block (every region ahead of it on all three axes is empty: traceMap's
- * blocks only move in the travel direction), and ends a ray as a miss when
- * it stands in such a region.  Every output is unchanged except the step
- * counts, so the test is never made for a frame that stores them
- * (frame.steps).  Statistics (frame.stats) count traceMap's steps; with
- * VT_FLAG_FREE_MAP_ON on a dense world they count the steps executed (rays
- * ending early).  Default: made when a step cap is at least VT_FREE_MIN_CAP
- * and some octant has at least 1/VT_FREE_MIN_SHARE of the world's regions
- * free (below either, the test costs more than it saves); these flags force
- * it either way (not both).                                                */
+/* Rays that end early (flat traversal of dense worlds; brickmap worlds with a
+ * power-of-two dim).  The library keeps, per world, a clearance map of the
+ * space around the nonempty blocks: a ray crosses clear stretches without
+ * lookups and ends as a miss when its line meets nothing more (before its
+ * step cap).  Every output is unchanged except the step counts, so it is
+ * never done for a frame that stores them (frame.steps).  Default: done in
+ * worlds open enough for it to pay; these flags force it either way (not
+ * both).
+ * The library also keeps the free-region map, a bitmap of the 16^3 regions
+ * from which no ray of a given direction octant can meet a nonempty block
+ * (every region ahead of it on all three axes is empty: traceMap's blocks
+ * only move in the travel direction).  Statistics (frame.stats) count
+ * traceMap's steps; with VT_FLAG_FREE_MAP_ON on a dense world with a free
+ * region they count the steps executed (rays ending early): then, and for
+ * frames without statistics when a step cap is at least VT_FREE_MIN_CAP and
+ * some octant has at least 1/VT_FREE_MIN_SHARE of the world's regions free,
+ * vt_free_map_used says 1.                                                 */
 #define VT_FLAG_FREE_MAP_ON (1u << 5)
 #define VT_FLAG_FREE_MAP_OFF (1u << 6)
 #define VT_FREE_MIN_CAP 512
@@ -154,9 +158,8 @@ enum {
   VT_STAT_L1_FETCHES = 4,    /* bitmask traversal: 16^3 region words loaded; */
                              /* brickmap worlds: chunk-table reads; flat    */
                              /* traversal with VT_FLAG_FREE_MAP_ON: steps   */
-                             /* taken without a lookup (a primary ray's     */
-                             /* steps before its line can reach the box of  */
-                             /* the nonempty voxels)                        */
+                             /* taken without a lookup (stretches the       */
+                             /* clearance map shows clear)                  */
   VT_STAT_L0_FETCHES = 5,    /* bitmask traversal: 4^3 brick words loaded;  */
                              /* brickmap worlds: block-pool + atlas reads   */
   VT_STAT_LEAF_READS = 6,    /* bitmask traversal: material bytes read at   */
@@ -338,11 +341,11 @@ int vt_world_info(const vt_world* world, uint32_t* dim, size_t* device_bytes);
 int vt_render(vt_ctx* ctx, const vt_world* world, const vt_camera* camera,
               const vt_render_params* params, const vt_frame* frame, void* stream);
 
-/* Whether vt_render with these arguments makes the free-region test
- * (VT_FLAG_FREE_MAP_ON above): *used = 1 when its rays end early in free
- * regions, 0 when every ray runs to its end.  No counterpart in the
- * reference, whose traceMap runs every ray to its end; for callers that
- * need to know whether a frame's statistics are traceMap's step counts.   */
+/* The free-region rule above for vt_render with these arguments: *used = 1
+ * when the caps, the world's free regions and the flags let rays end early
+ * in free regions, and a frame's statistics then count the steps executed;
+ * 0 when its statistics are traceMap's step counts.  No counterpart in the
+ * reference, whose traceMap runs every ray to its end.                     */
 int vt_free_map_used(const vt_world* world, const vt_render_params* params,
                      const vt_frame* frame, int* used);
 

@@ -58,6 +58,8 @@ void free_world(vt_world* w) {
   dev_free(w->occ);
   dev_free(w->brick_bits);
   dev_free(w->freemap);
+  dev_free(w->clear);
+  dev_free(w->clear_tmp);
   delete[] w->chunk_mirror;
   delete w;
 }
@@ -84,10 +86,14 @@ int dev_alloc(vt_world* w, void** p, size_t bytes, const char* what) {
   return VT_OK;
 }
 
-// The free-region map (built by vt::rebuild_freemap).
-int alloc_freemap(vt_world* w) {
-  return dev_alloc(w, (void**)&w->freemap, (8u * vt::free_words_per_octant(w->dim) + 1u) * 4u,
-                   "free-region map");
+// The free-region and clearance maps (built by vt::rebuild_maps).
+int alloc_maps(vt_world* w) {
+  int st = dev_alloc(w, (void**)&w->freemap, (8u * vt::free_words_per_octant(w->dim) + 2u) * 4u,
+                     "free-region map");
+  if (st != VT_OK || w->dim < 32u) return st;  // (a 16^3 map has 2 cells a side)
+  st = dev_alloc(w, (void**)&w->clear, 16u * (size_t)vt::clear_cells(w->dim), "clearance map");
+  if (st != VT_OK) return st;
+  return dev_alloc(w, (void**)&w->clear_tmp, vt::clear_tmp_bytes(w->dim), "clearance scratch");
 }
 
 }  // namespace
@@ -111,9 +117,9 @@ DenseWorld dense_view(const vt_world* w) {
   d.mz = (0x09249249u << 2) & low;
   d.nvox = w->dim * w->dim * w->dim;
   d.prefix = w->prefix;
-  d.freemap = w->freemap;
-  d.free_oct_bytes = free_words_per_octant(w->dim) * 4u;
-  d.free_bytes = w->freemap && w->free_valid ? 8u * d.free_oct_bytes : 0u;
+  d.clear = w->clear;
+  d.clear_oct_bytes = clear_cells(w->dim);
+  d.clear_bytes = w->clear && w->maps_valid ? 16u * d.clear_oct_bytes : 0u;
   reach_of(w, d.reach_lo, d.reach_hi);
   return d;
 }
@@ -137,30 +143,6 @@ void grow_box(vt_world* w, int32_t x, int32_t y, int32_t z) {
   w->box_any = true;
 }
 
-// The box of the nonzero blocks of a reference-layout map: exact from the
-// pool when `pool` is given, else the box of the nonzero chunk-table entries
-// (8^3 blocks each).
-void scan_brickmap_box(const uint32_t* chunks, const uint32_t* pool, uint32_t dim, vt_world* w) {
-  w->box_any = false;
-  const uint32_t M = dim / 8u;
-  for (uint32_t cz = 0; cz < M; cz++)
-    for (uint32_t cy = 0; cy < M; cy++)
-      for (uint32_t cx = 0; cx < M; cx++) {
-        const uint32_t e = chunks[cx + M * (cy + M * cz)];
-        if (!e) continue;
-        if (!pool) {
-          grow_box(w, (int32_t)(8u * cx), (int32_t)(8u * cy), (int32_t)(8u * cz));
-          grow_box(w, (int32_t)(8u * cx + 7u), (int32_t)(8u * cy + 7u), (int32_t)(8u * cz + 7u));
-          continue;
-        }
-        const uint32_t* b = pool + (size_t)(e - 1u) * 512u;  // in-block x + 8y + 64z
-        for (uint32_t i = 0; i < 512u; i++)
-          if (b[i])
-            grow_box(w, (int32_t)(8u * cx + (i & 7u)), (int32_t)(8u * cy + ((i >> 3) & 7u)),
-                     (int32_t)(8u * cz + (i >> 6)));
-      }
-}
-
 BrickmapWorld brickmap_view(const vt_world* w) {
   BrickmapWorld b;
   b.chunks = w->chunks;
@@ -175,10 +157,9 @@ BrickmapWorld brickmap_view(const vt_world* w) {
   b.mx = 0x09249249u & low;
   b.my = (0x09249249u << 1) & low;
   b.mz = (0x09249249u << 2) & low;
-  b.freemap = w->freemap;
-  b.free_oct_bytes = free_words_per_octant(w->dim) * 4u;
-  b.free_bytes = w->freemap && w->free_valid ? 8u * b.free_oct_bytes : 0u;
-  reach_of(w, b.reach_lo, b.reach_hi);
+  b.clear = w->clear;
+  b.clear_oct_bytes = clear_cells(w->dim);
+  b.clear_bytes = w->clear && w->maps_valid ? 16u * b.clear_oct_bytes : 0u;
   return b;
 }
 
@@ -295,6 +276,14 @@ bool render_free_map(const vt_world* w, const vt_render_params& p, const vt_fram
     return false;
   }
   return use_free_map(w, shade_consts(p));
+}
+
+bool render_clear_map(const vt_world* w, const vt_render_params& p, const vt_frame& f) {
+  if (f.steps) return false;
+  if (w->kind == WorldKind::Dense ? p.traversal != VT_TRAVERSAL_FLAT : !w->occ) return false;
+  // statistics count traceMap's steps exactly when vt_free_map_used says so
+  if (f.stats && !render_free_map(w, p, f)) return false;
+  return use_clear_map(w, p.flags);
 }
 
 FrameOut frame_out(const vt_frame* frame) {
@@ -419,7 +408,7 @@ int vt_world_create_dense_u8(vt_ctx* ctx, const uint8_t* grid, uint32_t dim,
       (st = dev_alloc(w, (void**)&w->l1, n / 512, "L1 masks")) != VT_OK ||
       (st = dev_alloc(w, (void**)&w->l1b, vt::l1b_words(dim) * 8, "8^3-brick masks")) != VT_OK ||
       (st = dev_alloc(w, (void**)&w->palette, 256 * 4, "palette")) != VT_OK ||
-      (st = alloc_freemap(w)) != VT_OK) {
+      (st = alloc_maps(w)) != VT_OK) {
     free_world(w);
     return st;
   }
@@ -434,16 +423,16 @@ int vt_world_create_dense_u8(vt_ctx* ctx, const uint8_t* grid, uint32_t dim,
   if (e == hipSuccess) e = hipMemcpy(w->palette, palette_rgba8, 256 * 4, hipMemcpyHostToDevice);
   // (the box is summed up in the free-region map's memory, which is built after)
   if (e == hipSuccess)
-    e = vt::launch_build_dense(lin, dim, w->vox, w->l0, w->l1, w->l1b, (int32_t*)w->freemap,
-                               ctx->report_dev(), nullptr);
-  if (e == hipSuccess) e = vt::rebuild_freemap(w, nullptr);
+    e = vt::launch_build_dense(lin, dim, w->vox, w->l0, w->l1, w->l1b, w->clear_tmp,
+                               (int32_t*)w->freemap, ctx->report_dev(), nullptr);
+  if (e == hipSuccess) e = vt::rebuild_maps(w, nullptr);
   if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
   dev_free(lin);
   if (e != hipSuccess) {
     free_world(w);
     return hip_fail(e, "vt_world_create_dense_u8: upload/build");
   }
-  vt::finish_freemap(w);
+  vt::finish_maps(w);
   std::memcpy(w->box_lo, ctx->report()->box_lo, sizeof w->box_lo);
   std::memcpy(w->box_hi, ctx->report()->box_hi, sizeof w->box_hi);
   w->box_any = w->box_lo[0] <= w->box_hi[0];
@@ -491,7 +480,6 @@ int vt_world_create_brickmap(vt_ctx* ctx, uint32_t dim, const uint32_t* chunks,
     return fail(VT_ERR_OUT_OF_MEMORY, "vt_world_create_brickmap: host chunk table");
   }
   std::memcpy(w->chunk_mirror, chunks, nchunks * 4);
-  vt::scan_brickmap_box(chunks, pool, dim, w);
   hipError_t e = hipMemcpy(w->chunks, chunks, nchunks * 4, hipMemcpyHostToDevice);
   if (e == hipSuccess && pool_words)
     e = hipMemcpy(w->pool, pool, pool_words * 4, hipMemcpyHostToDevice);
@@ -507,18 +495,19 @@ int vt_world_create_brickmap(vt_ctx* ctx, uint32_t dim, const uint32_t* chunks,
     if ((st = dev_alloc(w, (void**)&w->occ, n, "block occupancy")) != VT_OK ||
         (st = dev_alloc(w, (void**)&w->brick_bits, (size_t)vt::brick_bit_words(dim) * 8,
                         "block brick bits")) != VT_OK ||
-        (st = alloc_freemap(w)) != VT_OK) {
+        (st = alloc_maps(w)) != VT_OK) {
       free_world(w);
       return st;
     }
-    e = vt::launch_build_occupancy(vt::brickmap_view(w), w->occ, w->brick_bits, nullptr);
-    if (e == hipSuccess) e = vt::rebuild_freemap(w, nullptr);
+    e = vt::launch_build_occupancy(vt::brickmap_view(w), w->occ, w->brick_bits, w->clear_tmp,
+                                   nullptr);
+    if (e == hipSuccess) e = vt::rebuild_maps(w, nullptr);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess) {
       free_world(w);
       return hip_fail(e, "vt_world_create_brickmap: occupancy");
     }
-    vt::finish_freemap(w);
+    vt::finish_maps(w);
   }
   *out = w;
   return VT_OK;
@@ -571,15 +560,15 @@ int vt_render(vt_ctx* ctx, const vt_world* world, const vt_camera* camera,
   const uint32_t blocks_8x8 = ((p.width + 15u) / 16u) * ((p.height + 15u) / 16u);
   vt::TileShape tile{blocks_8x8 >= 8u * (uint32_t)ctx->compute_units ? 4u : 3u};
   hipError_t e;
-  const bool free_map = vt::render_free_map(world, p, *frame);
+  const bool clear = vt::render_clear_map(world, p, *frame);
   if (world->kind == WorldKind::Dense) {
     vt::DenseWorld dw = vt::dense_view(world);
-    if (!free_map) dw.free_bytes = 0;
+    if (!clear) dw.clear_bytes = 0;
     e = vt::launch_render_dense(dw, p.traversal, v, sc, o, frame->schedule, tile,
                                 (uint32_t)ctx->compute_units, (hipStream_t)stream);
   } else {
     vt::BrickmapWorld bw = vt::brickmap_view(world);
-    if (!free_map) bw.free_bytes = 0;
+    if (!clear) bw.clear_bytes = 0;
     e = vt::launch_render_brickmap(bw, v, sc, o, frame->schedule, tile,
                                    (uint32_t)ctx->compute_units, (hipStream_t)stream);
   }

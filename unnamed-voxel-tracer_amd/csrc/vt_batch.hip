@@ -37,17 +37,10 @@ __global__ void k_batch_reset(uint32_t* __restrict__ queues) {
   if (threadIdx.x < kQueues) queues[threadIdx.x * kQueueLine] = 0u;
 }
 
-// 7 waves per SIMD (72 VGPRs): the view record and queue state push the
-// kernel to ~94 VGPRs (5 waves); capping it spills values that live outside
-// the traversal loops and hides the gathers' latency far better (C2: 19.5 ->
-// 16.3 ms per 64-view batch at 8 waves).  With the free-region test seven
-// waves measure 3.81 / 3.84 ms against 4.01 / 3.91 at eight (fewer spills:
-// 132 vs 176 B per lane).
-#ifndef VT_BATCH_WAVES_PER_SIMD
-#define VT_BATCH_WAVES_PER_SIMD 7
-#endif
+// Six waves per SIMD (80 VGPRs) with the clearance map: 64 views over 1024^3
+// 2.26 ms against 2.33 at seven and 2.28 at five; seven without it.
 template <class L, bool kStats, int kShade>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VT_BATCH_WAVES_PER_SIMD))) void k_render_batch(DenseWorld w, ShadeConsts sc,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(L::kClear ? 6 : 7))) void k_render_batch(DenseWorld w, ShadeConsts sc,
                                                       const BatchView* __restrict__ views,
                                                       uint32_t n_views, uint32_t total_tiles,
                                                       uint32_t* __restrict__ queues,
@@ -173,14 +166,14 @@ using vt::fail;
 using vt::hip_fail;
 
 // Queue reset + persistent launch over a device view table.
-// steps_out: some view stores step counts, which the free-region map's early
-// end of a ray would change, so the map is not read.
+// steps_out: some view stores step counts, which the early end of a ray would
+// change, so the clearance map is not read.
 hipError_t launch_batch(const vt_world* world, const vt::ShadeConsts& sc_in,
                         const vt::BatchView* d_views, uint32_t n_views, uint32_t total_tiles,
                         uint32_t* d_queues, const vt_tuning& tuning, uint32_t nblocks,
                         unsigned long long* stats, bool steps_out, hipStream_t s) {
   vt::DenseWorld w = vt::dense_view(world);
-  if (steps_out || stats || !vt::use_free_map(world, sc_in)) w.free_bytes = 0;
+  if (steps_out || stats || !vt::use_clear_map(world, sc_in.flags)) w.clear_bytes = 0;
   // rays end early at the reach box unless their step counts are observed
   if (steps_out || stats) vt::reach_everywhere(w.reach_lo, w.reach_hi);
   vt::ShadeConsts sc = sc_in;
@@ -207,7 +200,7 @@ hipError_t launch_batch(const vt_world* world, const vt::ShadeConsts& sc_in,
     else VT_BATCH_SHADE(BitmaskLookup8, false)
   } else {
     if (stats) VT_BATCH_SHADE(FlatLookup, true)
-    else if (w.free_bytes) VT_BATCH_SHADE(FlatLookupFree, false)
+    else if (w.clear_bytes) VT_BATCH_SHADE(FlatLookupClear, false)
     else if (sc.max_primary >= vt::kLongCap || sc.max_shadow >= vt::kLongCap)
       VT_BATCH_SHADE(FlatLookupLong, false)
     else VT_BATCH_SHADE(FlatLookup, false)

@@ -38,7 +38,7 @@ __global__ __launch_bounds__(256) void k_edit_brickmap(uint32_t* __restrict__ po
                                                        uint32_t n, uint32_t m,
                                                        uint32_t* __restrict__ changed) {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-  if (i == 0u && changed) *changed = 0u;  // for the kernels that follow
+  if (i < 2u && changed) changed[i] = 0u;  // for the kernels that follow
   if (i < n) {
     const uint3 r = reinterpret_cast<const uint3*>(data)[i];
     pool[r.x] = r.y;
@@ -50,25 +50,40 @@ __global__ __launch_bounds__(256) void k_edit_brickmap(uint32_t* __restrict__ po
   }
 }
 
+// The clearance map's byte of brick b (null: a world without the map), from
+// its occupancy word; sets changed[1] when it is another one.
+__device__ __forceinline__ void put_sub(uint8_t* sub, uint32_t b, uint64_t word,
+                                        uint32_t* changed) {
+  if (!sub) return;
+  const uint8_t v = (uint8_t)nonzero_bytes(word);
+  if (sub[b] != v) {
+    sub[b] = v;
+    changed[1] = 1u;
+  }
+}
+
 // The brick bits of the listed 4^3 bricks, from their 64 occupancy bytes
-// (one wave per brick; several bricks of a word: atomics on its bits).  Sets
-// *changed when a word (a 16^3 region) stops or starts being zero.
+// (one wave per brick; several bricks of a word: atomics on its bits), and
+// their sub-block bits.  Sets changed[0] when a word (a 16^3 region) stops
+// or starts being zero.
 __global__ __launch_bounds__(256) void k_edit_bricks(const uint8_t* __restrict__ occ,
                                                      const uint32_t* __restrict__ bricks,
                                                      uint32_t n,
                                                      unsigned long long* __restrict__ bits,
+                                                     uint8_t* __restrict__ sub,
                                                      uint32_t* __restrict__ changed) {
   const uint32_t wave = (blockIdx.x * 256u + threadIdx.x) >> 6, lane = threadIdx.x & 63u;
   if (wave >= n) return;  // whole waves leave together
   const uint32_t b = bricks[wave];
-  const bool any = __ballot(occ[(size_t)b * 64u + lane] != 0) != 0ull;
+  const uint64_t m = __ballot(occ[(size_t)b * 64u + lane] != 0);
   if (lane != 0u) return;
+  put_sub(sub, b, m, changed);
   const unsigned long long bit = 1ull << (b & 63u);
-  if (any) {
-    if (atomicOr(bits + (b >> 6), bit) == 0ull) *changed = 1u;
+  if (m) {
+    if (atomicOr(bits + (b >> 6), bit) == 0ull) changed[0] = 1u;
   } else {
     const unsigned long long old = atomicAnd(bits + (b >> 6), ~bit);
-    if (old != 0ull && (old & ~bit) == 0ull) *changed = 1u;
+    if (old != 0ull && (old & ~bit) == 0ull) changed[0] = 1u;
   }
 }
 
@@ -85,25 +100,41 @@ __global__ __launch_bounds__(256) void k_edit_dense(uint8_t* __restrict__ vox,
                                                     const uint32_t* __restrict__ data,
                                                     uint32_t n, uint32_t* __restrict__ changed) {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-  if (i == 0u) *changed = 0u;  // for the kernels that follow
+  if (i < 2u) changed[i] = 0u;  // for the kernels that follow
   if (i < n) vox[data[2u * (size_t)i]] = (uint8_t)data[2u * (size_t)i + 1u];
 }
 
-// One wave per listed word: bit l of out[word] = (in[word * 64 + l] != 0).
-// Sets *changed (when not null) when a word stops or starts being zero.
-template <class T>
-__global__ __launch_bounds__(256) void k_rebuild_mask(const T* __restrict__ in,
-                                                      uint64_t* __restrict__ out,
-                                                      const uint32_t* __restrict__ words,
-                                                      uint32_t n, uint32_t* __restrict__ changed) {
-  const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const uint32_t lane = threadIdx.x & 63u;
+// The L0 words of the listed 4^3 bricks (one wave per word: ballot over its
+// 64 bytes) and their sub-block bits.
+__global__ __launch_bounds__(256) void k_edit_l0(const uint8_t* __restrict__ vox,
+                                                 uint64_t* __restrict__ l0,
+                                                 const uint32_t* __restrict__ bricks, uint32_t n,
+                                                 uint8_t* __restrict__ sub,
+                                                 uint32_t* __restrict__ changed) {
+  const uint32_t wave = (blockIdx.x * 256u + threadIdx.x) >> 6, lane = threadIdx.x & 63u;
   if (wave >= n) return;  // whole waves leave together
-  const uint32_t word = words[wave];
-  const uint64_t m = __ballot(in[(size_t)word * 64u + lane] != 0);
+  const uint32_t b = bricks[wave];
+  const uint64_t m = __ballot(vox[(size_t)b * 64u + lane] != 0);
   if (lane == 0) {
-    if (changed && (out[word] == 0ull) != (m == 0ull)) *changed = 1u;
-    out[word] = m;
+    l0[b] = m;
+    put_sub(sub, b, m, changed);
+  }
+}
+
+// The L1 words of the listed 16^3 regions, one wave per word: bit l =
+// (l0[region * 64 + l] != 0).  Sets changed[0] when a word stops or starts
+// being zero.
+__global__ __launch_bounds__(256) void k_edit_l1(const uint64_t* __restrict__ l0,
+                                                 uint64_t* __restrict__ l1,
+                                                 const uint32_t* __restrict__ regions, uint32_t n,
+                                                 uint32_t* __restrict__ changed) {
+  const uint32_t wave = (blockIdx.x * 256u + threadIdx.x) >> 6, lane = threadIdx.x & 63u;
+  if (wave >= n) return;  // whole waves leave together
+  const uint32_t r = regions[wave];
+  const uint64_t m = __ballot(l0[(size_t)r * 64u + lane] != 0ull);
+  if (lane == 0) {
+    if ((l1[r] == 0ull) != (m == 0ull)) changed[0] = 1u;
+    l1[r] = m;
   }
 }
 
@@ -331,7 +362,6 @@ int set_brickmap(vt_world* w, const uint32_t* xyz, const uint32_t* values, uint3
   uint64_t used = w->pool_words / 512u;
   last.reserve(n);
   words.reserve(3 * (size_t)n);
-  grow_box_by(w, xyz, values, n);
   for (uint32_t i = 0; i < n; i++) {
     const uint32_t x = xyz[3 * (size_t)i], y = xyz[3 * (size_t)i + 1], z = xyz[3 * (size_t)i + 2];
     const uint64_t ci = (uint64_t)(x / 8u) + M * ((uint64_t)(y / 8u) + (uint64_t)M * (z / 8u));
@@ -369,14 +399,14 @@ int set_brickmap(vt_world* w, const uint32_t* xyz, const uint32_t* values, uint3
   VT_HIP(lists.put(words));
   const uint32_t* d_chunks = lists.dev + 3 * (size_t)nw;
   hipLaunchKernelGGL(vt::k_edit_brickmap, dim3(blocks_for(std::max(nw, nc), 256)), dim3(256), 0, s,
-                     w->pool, w->occ, w->chunks, lists.dev, nw, nc, vt::freemap_changed(w));
+                     w->pool, w->occ, w->chunks, lists.dev, nw, nc, vt::maps_changed(w));
   hipError_t e = hipGetLastError();
   if (e == hipSuccess && w->occ) {
     hipLaunchKernelGGL(vt::k_edit_bricks, dim3(blocks_for(nb, 4)), dim3(256), 0, s, w->occ,
                        d_chunks + 2 * (size_t)nc, nb, (unsigned long long*)w->brick_bits,
-                       vt::freemap_changed(w));
+                       w->clear_tmp, vt::maps_changed(w));
     e = hipGetLastError();
-    if (e == hipSuccess) e = vt::rebuild_freemap(w, s, vt::freemap_changed(w));
+    if (e == hipSuccess) e = vt::rebuild_maps(w, s, vt::maps_changed(w));
   }
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) {
@@ -395,7 +425,7 @@ int set_brickmap(vt_world* w, const uint32_t* xyz, const uint32_t* values, uint3
   }
   for (uint32_t k = 0; k < nc; k++) w->chunk_mirror[chunks[2 * k]] = chunks[2 * k + 1];
   w->pool_words = used * 512u;
-  if (w->occ) vt::finish_freemap(w);
+  if (w->occ) vt::finish_maps(w);
   return VT_OK;
 }
 
@@ -436,15 +466,15 @@ int set_dense(vt_world* w, const uint32_t* xyz, const uint32_t* values, uint32_t
   VT_HIP(lists.put(words));
   const uint32_t* d_bricks = lists.dev + 2 * (size_t)nw;
   hipLaunchKernelGGL(vt::k_edit_dense, dim3(blocks_for(nw, 256)), dim3(256), 0, s, w->vox,
-                     lists.dev, nw, vt::freemap_changed(w));
-  hipLaunchKernelGGL((vt::k_rebuild_mask<uint8_t>), dim3(blocks_for(nb, 4)), dim3(256), 0, s,
-                     w->vox, w->l0, d_bricks, nb, (uint32_t*)nullptr);
-  hipLaunchKernelGGL((vt::k_rebuild_mask<uint64_t>), dim3(blocks_for(nr, 4)), dim3(256), 0, s,
-                     w->l0, w->l1, d_bricks + nb, nr, vt::freemap_changed(w));
+                     lists.dev, nw, vt::maps_changed(w));
+  hipLaunchKernelGGL(vt::k_edit_l0, dim3(blocks_for(nb, 4)), dim3(256), 0, s, w->vox, w->l0,
+                     d_bricks, nb, w->clear_tmp, vt::maps_changed(w));
+  hipLaunchKernelGGL(vt::k_edit_l1, dim3(blocks_for(nr, 4)), dim3(256), 0, s, w->l0, w->l1,
+                     d_bricks + nb, nr, vt::maps_changed(w));
   VT_HIP(hipGetLastError());
   VT_HIP(vt::launch_build_l1b(w->l0, (uint64_t)w->dim * w->dim * w->dim / 64u,
                               d_bricks + nb + nr, nr8, w->l1b, s));
-  VT_HIP(vt::rebuild_freemap(w, s, vt::freemap_changed(w)));
+  VT_HIP(vt::rebuild_maps(w, s, vt::maps_changed(w)));
   if (w->prefix) {  // keep the compact index current
     const uint64_t nwords = (uint64_t)w->dim * w->dim * w->dim / 64u;
     const uint64_t ntiles = (nwords + 1023) / 1024;
@@ -460,7 +490,7 @@ int set_dense(vt_world* w, const uint32_t* xyz, const uint32_t* values, uint32_t
     w->n_occupied = total;
   }
   VT_HIP(hipStreamSynchronize(s));
-  vt::finish_freemap(w);
+  vt::finish_maps(w);
   return VT_OK;
 }
 
@@ -547,7 +577,7 @@ int vt_world_read_free_map(vt_ctx* ctx, const vt_world* world, uint32_t* words,
   if (world->ctx != ctx) return fail(VT_ERR_WRONG_CONTEXT, "vt_world_read_free_map");
   const uint32_t wpo = vt::free_words_per_octant(world->dim);
   *words_per_octant = wpo;
-  *valid = world->freemap && world->free_valid ? 1 : 0;
+  *valid = world->freemap && world->maps_valid ? 1 : 0;
   if (!words || !world->freemap) return VT_OK;
   if (capacity_words < 8u * (size_t)wpo)
     return fail(VT_ERR_INVALID_ARGUMENT,
@@ -573,7 +603,7 @@ int vt_pick(vt_ctx* ctx, const vt_world* world, const vt_camera* camera, int32_t
   vt_pick_result* d = (vt_pick_result*)ctx->stage_dev;  // the context's staging
   if (world->kind == WorldKind::Dense) {
     vt::DenseWorld dw = vt::dense_view(world);
-    dw.free_bytes = 0;  // the result reports traceMap's step count
+    dw.clear_bytes = 0;  // the result reports traceMap's step count
     hipLaunchKernelGGL(vt::k_pick_dense, dim3(1), dim3(64), 0, s, dw, v, (int)max_steps, d);
   } else {
     vt::BrickmapWorld bw = vt::brickmap_view(world);

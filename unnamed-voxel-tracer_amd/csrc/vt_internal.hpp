@@ -28,6 +28,7 @@ constexpr size_t kCtxReportBytes = 256;  // after the staging: CtxReport
 struct CtxReport {
   uint32_t free_built;       // 0: no region had changed, the map was left as it is
   uint32_t free_regions[8];  // else: free regions of each octant
+  uint32_t near_cells;       // near cells of the clearance map
   int32_t box_lo[3], box_hi[3];  // box of the nonempty voxels; lo > hi: none
 };
 static_assert(sizeof(CtxReport) <= kCtxReportBytes, "CtxReport");
@@ -71,12 +72,17 @@ struct vt_world {
   uint64_t* brick_bits;    // brickmap: bit per 4^3 brick of blocks, from occ
   // free-region map (dense worlds and power-of-two brickmap worlds)
   uint32_t* freemap;       // 8 octants x free_words_per_octant(dim) words, then a
-                           // word edits set when a region empties or fills
-  bool free_valid;         // the map matches the occupancy (finish_freemap)
+                           // two words edits set: when a region empties or
+                           // fills, when a 2^3 sub-block does
+  // clearance map (the same worlds, dim >= 32)
+  uint8_t* clear;          // 2 orders x 8 octants x clear_cells(dim) bytes
+  uint8_t* clear_tmp;      // clear_tmp_bytes(dim): the sub-block bits of every
+                           // 4^3 brick (kept current), then build scratch
+  bool maps_valid;         // both maps match the occupancy (finish_maps)
+  float near_frac;         // share of near cells in the clearance map
   float free_frac;         // largest share of free regions over the 8 octants
-  // the box of the nonempty voxels (dense) or blocks (reference layout),
-  // inclusive; grown by edits, never shrunk; box_any = false while the
-  // world has none
+  // the box of a dense world's nonempty voxels, inclusive; grown by edits,
+  // never shrunk; box_any = false while the world has none
   int32_t box_lo[3], box_hi[3];
   bool box_any;
   // compact albedo index of a dense world (built on request)
@@ -132,8 +138,16 @@ struct TileShape {
   uint32_t log2_w;  // 3 (8x8), 4 (16x4) or 5 (32x2)
 };
 
+// Bit k = byte k of v is nonzero.
+__device__ __forceinline__ uint32_t nonzero_bytes(uint64_t v) {
+  uint64_t y = v | (v >> 4);
+  y |= y >> 2;
+  y |= y >> 1;
+  y &= 0x0101010101010101ull;
+  return (uint32_t)((y * 0x0102040810204080ull) >> 56);
+}
+
 DenseWorld dense_view(const vt_world* w);
-void scan_brickmap_box(const uint32_t* chunks, const uint32_t* pool, uint32_t dim, vt_world* w);
 void grow_box(vt_world* w, int32_t x, int32_t y, int32_t z);
 void reach_of(const vt_world* w, float* lo, float* hi);
 BrickmapWorld brickmap_view(const vt_world* w);
@@ -166,18 +180,19 @@ hipError_t launch_render_brickmap(const BrickmapWorld& w, const ViewConsts& v,
 // world (power-of-two dim) with y < y_end (0: all layers), and the brick
 // bits of those layers' 4^3 bricks (bits of a partly covered word are set
 // only, never cleared: the other layers' bits must be right already).
+// sub (may be null): the clearance map's byte of each of those bricks.
 hipError_t launch_build_occupancy(const BrickmapWorld& w, uint8_t* occ, uint64_t* brick_bits,
-                                  hipStream_t stream, uint32_t y_end = 0);
+                                  uint8_t* sub, hipStream_t stream, uint32_t y_end = 0);
 // Grows a brickmap world's block pool to at least `blocks` blocks by
 // doubling (GpuBlockAllocator.alloc, gpu_block_allocator.zig:20-30), keeping
 // the contents and zeroing the new blocks; `who` names the caller in errors.
 int grow_pool(vt_world* w, uint64_t blocks, hipStream_t s, const char* who);
 // The Morton-ordered voxels of a linear grid and their occupancy levels, and
 // the box of the nonempty voxels into *report (which holds an empty box
-// before).
+// before); sub: the clearance map's byte of each 4^3 brick.
 hipError_t launch_build_dense(const uint8_t* linear, uint32_t dim, uint8_t* vox, uint64_t* l0,
-                              uint64_t* l1, uint64_t* l1b, int32_t* box6, CtxReport* report,
-                              hipStream_t stream);
+                              uint64_t* l1, uint64_t* l1b, uint8_t* sub, int32_t* box6,
+                              CtxReport* report, hipStream_t stream);
 // Words of the 8^3-brick level of a dim^3 world: one per 32^3 region (one
 // partial word for dim 16).
 inline uint64_t l1b_words(uint32_t dim) {
@@ -198,29 +213,47 @@ uint32_t free_regions(uint32_t dim);
 uint32_t free_words_per_octant(uint32_t dim);
 hipError_t launch_build_freemap(const uint64_t* l1, uint32_t dim, uint32_t* fm,
                                 const uint32_t* changed, CtxReport* report, hipStream_t stream);
-// Rebuilds a world's free-region map from its current occupancy (a dense
-// world's L1 words; a brickmap world's brick bits); no-op without one.
-// `changed`: as launch_build_freemap (null: always).  Clears free_valid: the caller calls finish_freemap once the stream has
-// synchronised without error, and until then the renderers do not read it.
-hipError_t rebuild_freemap(vt_world* w, hipStream_t stream, const uint32_t* changed = nullptr);
-// The word edits set when a region empties or fills.
-inline uint32_t* freemap_changed(const vt_world* w) {
+// Clearance map (ClearMap in vt_trace.hpp): 2 x 8 octant planes of
+// clear_cells(dim) bytes, built from one byte per 4^3 brick (a bit per 2^3
+// sub-block) at the start of tmp, unless *changed (device, may be null) is 0;
+// reports the near cells.
+uint32_t clear_cells(uint32_t dim);
+size_t clear_tmp_bytes(uint32_t dim);
+hipError_t launch_build_clear(uint8_t* tmp, uint32_t dim, uint8_t* map, const uint32_t* changed,
+                              CtxReport* report, hipStream_t stream);
+// Whether launches with these flags use the clearance map: it is valid and
+// VT_FLAG_FREE_MAP_ON, or neither FREE_MAP flag and a world open enough for
+// it to pay.
+bool use_clear_map(const vt_world* w, uint32_t flags);
+// Whether vt_render uses it for this world, parameters and frame: no stored
+// step counts (they would lack the steps of rays that end early); on dense
+// worlds the flat traversal, and statistics only with VT_FLAG_FREE_MAP_ON
+// (they then count the steps executed); on the reference layout occupancy
+// bytes and no statistics.
+bool render_clear_map(const vt_world* w, const vt_render_params& p, const vt_frame& f);
+// Rebuilds a world's free-region and clearance maps from its current
+// occupancy (L1 words or brick bits, and the sub-block bits); no-op without
+// them.  `changed`: the two words of maps_changed (null: rebuild always).
+// Clears maps_valid: the caller calls finish_maps once the stream has
+// synchronised without error, and until then the renderers read neither.
+hipError_t rebuild_maps(vt_world* w, hipStream_t stream, const uint32_t* changed = nullptr);
+// The words edits set: [0] a 16^3 region emptied or filled, [1] a 2^3
+// sub-block did.
+inline uint32_t* maps_changed(const vt_world* w) {
   return w->freemap ? w->freemap + 8u * free_words_per_octant(w->dim) : nullptr;
 }
-// After a rebuild completed: takes the largest share of free regions over the
-// octants (free_frac) from the context's report and marks the map valid.
-void finish_freemap(vt_world* w);
-// Whether a launch with these constants tests the free-region map: the map
-// is valid and has a free region, and VT_FLAG_FREE_MAP_ON, or neither
-// FREE_MAP flag, a step cap of at least VT_FREE_MIN_CAP and at least
-// 1/VT_FREE_MIN_SHARE of the regions free in some octant.  (Frames that
-// store step counts or statistics are excluded by the launchers.)
+// After a rebuild completed: takes what the context's report says (free_frac,
+// near_frac) and marks the maps valid.
+void finish_maps(vt_world* w);
+// The free-region rule (vt.h): the map is valid and has a free region, and
+// VT_FLAG_FREE_MAP_ON, or neither FREE_MAP flag, a step cap of at least
+// VT_FREE_MIN_CAP and at least 1/VT_FREE_MIN_SHARE of the regions free in
+// some octant.
 bool use_free_map(const vt_world* w, const ShadeConsts& sc);
-// Whether vt_render makes the test for this world, parameters and frame:
-// use_free_map, and no stored step counts; on dense worlds the flat
-// traversal, and statistics only with VT_FLAG_FREE_MAP_ON (they then count
-// the steps executed); on the reference layout occupancy bytes and no
-// statistics.
+// vt_free_map_used: use_free_map, and no stored step counts; on dense worlds
+// the flat traversal, and statistics only with VT_FLAG_FREE_MAP_ON (they
+// then count the steps executed); on the reference layout occupancy bytes
+// and no statistics.
 bool render_free_map(const vt_world* w, const vt_render_params& p, const vt_frame& f);
 // Words of a brickmap world's brick bits: one uint64 per 4096 codes.
 uint32_t brick_bit_words(uint32_t dim);

@@ -653,19 +653,20 @@ __device__ __forceinline__ void trace_pixel_dense(const DenseWorld& w, const Vie
   float ey = (v.pos[1] + dy * tc) - 0.001f;
   float ez = (v.pos[2] + dz * tc) - 0.001f;
   const RayConsts pk = make_ray_consts(dx, dy, dz, w.mx, w.my, w.mz);
-  if (!line_meets_reach(w, ex, ey, ez, pk)) {
+  if (!L::kClear && !line_meets_reach(w, ex, ey, ez, pk)) {
     // this ray cannot reach a nonempty voxel: a miss, no steps (launches
-    // whose step counts are observed pass a reach every line meets)
+    // whose step counts are observed pass a reach every line meets; the
+    // clearance map finds such rays by itself)
     h.hit = false;
     h.steps = 0;
   } else if (!dense_begin_k<kStats>(r, lk, w, ex, ey, ez, pk, sc.max_primary, h, cnt.l1f,
                                     cnt.l0f)) {
-    r.blind = blind_steps(w, ex, ey, ez, pk);
+    if constexpr (!L::kClear) r.blind = blind_steps(w, ex, ey, ez, pk);
     dense_run<kStats>(r, lk, w, h, cnt.l1f, cnt.l0f);
-    // statistics of the steps executed (flat, free-region test): count
-    // those taken without a lookup (VT_STAT_L1_FETCHES, unused by the flat
-    // lookups otherwise)
-    if constexpr (kStats && L::kPrefetch && L::kFree) cnt.l1f += (uint32_t)r.blind;
+    // statistics of the steps executed (flat, clearance map): count those
+    // taken without a lookup (VT_STAT_L1_FETCHES, unused by the flat lookups
+    // otherwise)
+    if constexpr (kStats && L::kClear) cnt.l1f += (uint32_t)r.blind;
   }
   p.hit = h.hit;
   p.steps = h.steps;
@@ -690,12 +691,13 @@ __device__ __forceinline__ void trace_pixel_dense(const DenseWorld& w, const Vie
     const int psteps = p.steps;
     if (!dense_begin_k<kStats>(r, lk, w, sox, soy, soz, sc.shadow, sc.max_shadow, h, cnt.l1f,
                                cnt.l0f)) {
-      if constexpr (L::kPrefetch && (!kStats || L::kFree)) {
+      if constexpr (L::kPrefetch && (!kStats || L::kClear)) {
         // the sun is the same for every lane: a uniform branch
         if (sc.sun[0] >= 0.0f && sc.sun[1] >= 0.0f && sc.sun[2] >= 0.0f)
-          dense_run_prefetch<L, true>(r, lk, w, h);
+          dense_run_prefetch<L, true, true>(r, lk, w, h);
         else
-          dense_run_prefetch<L, false>(r, lk, w, h);
+          dense_run_prefetch<L, false, true>(r, lk, w, h);
+        if constexpr (kStats && L::kClear) cnt.l1f += (uint32_t)r.blind;
       } else {
         dense_run<kStats>(r, lk, w, h, cnt.l1f, cnt.l0f);
       }

@@ -396,9 +396,9 @@ int vt_world_procgen(vt_ctx* ctx, vt_world* world, float offset_x, float offset_
   }
   // the empty map's occupancy bytes were zero; only the written layers change
   if (e == hipSuccess && world->occ)
-    e = vt::launch_build_occupancy(vt::brickmap_view(world), world->occ, world->brick_bits, s,
-                                   std::min(dim, (walk.y_end + 7u) & ~7u));
-  if (e == hipSuccess) e = vt::rebuild_freemap(world, s);
+    e = vt::launch_build_occupancy(vt::brickmap_view(world), world->occ, world->brick_bits,
+                                   world->clear_tmp, s, std::min(dim, (walk.y_end + 7u) & ~7u));
+  if (e == hipSuccess) e = vt::rebuild_maps(world, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) {
     // back to the empty map the call was given: chunk table, written pool
@@ -408,6 +408,8 @@ int vt_world_procgen(vt_ctx* ctx, vt_world* world, float offset_x, float offset_
     if (world->occ) {
       (void)hipMemsetAsync(world->occ, 0, (size_t)dim * dim * dim, s);
       (void)hipMemsetAsync(world->brick_bits, 0, (size_t)vt::brick_bit_words(dim) * 8u, s);
+      if (world->clear_tmp)
+        (void)hipMemsetAsync(world->clear_tmp, 0, 8u * (size_t)vt::clear_cells(dim), s);
     }
     (void)hipStreamSynchronize(s);
     (void)hipGetLastError();
@@ -415,8 +417,7 @@ int vt_world_procgen(vt_ctx* ctx, vt_world* world, float offset_x, float offset_
   }
   std::memcpy(world->chunk_mirror, walk.mirror.data(), nchunks * 4);
   world->pool_words = walk.used * 512u;
-  vt::scan_brickmap_box(world->chunk_mirror, nullptr, dim, world);  // chunk granularity
-  vt::finish_freemap(world);
+  vt::finish_maps(world);
   return VT_OK;
 }
 

@@ -14,31 +14,25 @@
 // no XCD is left with the costliest rows.  Each lane traces its primary ray,
 // then (on a hit) its shadow ray.
 //
-// Rays end early where nothing is left to hit: with the free-region test
-// (a per-world bitmap of the 16^3 regions from which every region ahead in a
-// direction octant is empty) a ray standing in such a region is a miss.  Lit
-// shadow rays, which otherwise run to the edge of the grid, mostly end a few
-// regions after their start, so the lanes of a wave finish close together.
+// Rays end early where nothing is left to hit and cross clear space without
+// lookups: with the clearance map (ClearMap in vt_trace.hpp) the line is
+// followed from clear cube to clear cube first.  Lit shadow rays, which
+// otherwise run to the edge of the grid, mostly end a few cells after their
+// start, so the lanes of a wave finish close together.
 #include "vt_pixel.hpp"
 
 namespace vt {
 
-// amdgpu_waves_per_eu: at most 72 VGPRs (seven waves per SIMD) for every
-// shading mode.  The reference composite needs no scratch at 72 (56 B per
-// lane of spills at 64 with the free-region test, ~100 MB of spill stores
-// per 1080p frame); C1 at 1080p measures the same at eight, seven and six
-// waves (0.2785 / 0.2791 / 0.2789 ms), C3's 512x512 views 2% faster at
-// seven (0.1113 vs 0.1137 ms per view).  Before the free-region test eight
-// waves were faster (1080p 0.785 vs 0.804 ms): the traversal loop then held
-// most of the time and its gathers needed the waves.
-#ifndef VT_REF_WAVES_PER_SIMD
-#define VT_REF_WAVES_PER_SIMD 7
-#endif
+// amdgpu_waves_per_eu: with the clearance map six waves per SIMD (80 VGPRs)
+// -- six views of the 512^3 world at 1080p 290 us on average, 301 at seven
+// (spills), 295 at five -- without it seven (72 VGPRs, no spills).
+constexpr int kClearWaves = 6;
+constexpr int kPlainWaves = 7;
 // kSched: the launch order comes from the frame's tile schedule (`sched`);
 // the kernels without it carry none of its code.
 template <class L, bool kStats, int kShade, bool kSched>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(kShade == kShadeRef ? VT_REF_WAVES_PER_SIMD : 7))) void k_render_dense(
+__attribute__((amdgpu_waves_per_eu(L::kClear ? kClearWaves : kPlainWaves))) void k_render_dense(
     DenseWorld w, ViewConsts v, ShadeConsts sc, FrameOut out, uint32_t* sched, uint32_t log2_tw,
     uint32_t blocks_x) {
   __shared__ SchedBlock sb;
@@ -63,18 +57,14 @@ __attribute__((amdgpu_waves_per_eu(kShade == kShadeRef ? VT_REF_WAVES_PER_SIMD :
   if constexpr (kSched) sched_end(sb, lane);
 }
 
-// Seven waves per SIMD (at most 72 VGPRs): the engine's own frame 0.373 vs
-// 0.460 ms at eight (fewer spills around its many literal-loop iterations),
-// the C1 world in this layout 0.823 vs 0.820 ms; five waves (90 VGPRs) were
-// slower on both.  The free-region variants take six (80 VGPRs, 64 B of
-// scratch per lane against 112 at seven): with the reach box and the blind
-// prefix the C1 world in this layout measured 204.4 us at six against 212.5
-// at seven, 206.6 at five and 225.9 at eight; the engine's frame (no
-// free-region test) measures the same at six (275.7 against 275.4 us).
-// kFree: the empty-space loops test the free-region map.
+// Seven waves per SIMD (72 VGPRs) without the clearance map; with it five (96
+// VGPRs): the engine's map with long caps at 1600x900, six views, 245 us on
+// average, 272 at six, 316 at seven; its own frame 138, 143 and 152 (fewer
+// spills around its many literal-loop iterations).
+// kClear: the empty-space runs take the clearance map.
 // kSched: as k_render_dense.
-template <bool kStats, bool kFree, bool kSched>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kFree ? 6 : 7))) void k_render_brickmap(
+template <bool kStats, bool kClear, bool kSched>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kClear ? 5 : 7))) void k_render_brickmap(
     BrickmapWorld w, ViewConsts v, ShadeConsts sc, FrameOut out, uint32_t* sched,
     uint32_t log2_tw, uint32_t blocks_x) {
   __shared__ SchedBlock sb;
@@ -100,17 +90,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kFree ? 6 :
     float ey = (v.pos[1] + dy * tc) - 0.001f;
     float ez = (v.pos[2] + dz * tc) - 0.001f;
     GeneralHit g;
-    int blind = 0;
-    if (kFree && !kStats && !line_meets_reach_bm(w, ex, ey, ez, dx, dy, dz, blind)) {
-      // with the free-region test: this ray cannot reach a nonempty block (a
-      // miss, no steps).  Without the test the check is left out: the
-      // engine's own frame (caps 192/48, its camera inside the box, where
-      // no ray can end) measured 0.304 ms with it against 0.274 without.
-      g.data = 0u;
-      g.hx = g.hy = g.hz = -1.0f;
-      g.steps = 0;
-    } else if (!kStats && w.occ)
-      trace_brickmap_fast<false, kFree>(w, ex, ey, ez, dx, dy, dz, sc.max_primary, g, blind);
+    if (!kStats && w.occ)
+      trace_brickmap_fast<false, kClear, false>(w, ex, ey, ez, dx, dy, dz, sc.max_primary, g);
     else
       trace_general<kStats>(w, ex, ey, ez, dx, dy, dz, sc.max_primary, g, cnt.l1f, cnt.l0f);
     Primary p;
@@ -137,11 +118,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kFree ? 6 :
       if (!kStats && w.occ) {
         // the sun is the same for every lane: a uniform branch
         if (sc.sun[0] >= 0.0f && sc.sun[1] >= 0.0f && sc.sun[2] >= 0.0f)
-          trace_brickmap_fast<true, kFree>(w, sox, soy, soz, sc.sun[0], sc.sun[1], sc.sun[2],
-                                           sc.max_shadow, s);
+          trace_brickmap_fast<true, kClear, true>(w, sox, soy, soz, sc.sun[0], sc.sun[1],
+                                                  sc.sun[2], sc.max_shadow, s);
         else
-          trace_brickmap_fast<false, kFree>(w, sox, soy, soz, sc.sun[0], sc.sun[1], sc.sun[2],
-                                            sc.max_shadow, s);
+          trace_brickmap_fast<false, kClear, true>(w, sox, soy, soz, sc.sun[0], sc.sun[1],
+                                                   sc.sun[2], sc.max_shadow, s);
       } else {
         trace_general<kStats>(w, sox, soy, soz, sc.sun[0], sc.sun[1], sc.sun[2], sc.max_shadow,
                               s, cnt.l1f, cnt.l0f);
@@ -211,12 +192,12 @@ static void launch_dense_select(const DenseWorld& w, uint32_t traversal, const V
       launch_dense_shade<BitmaskLookup8, false, kSched>(w, v, sc, out, sd, lw, blocks_x, grid, stream);
   } else {
     const bool long_caps = sc.max_primary >= kLongCap || sc.max_shadow >= kLongCap;
-    if (stats && w.free_bytes)  // statistics of the steps executed
-      launch_dense_shade<FlatLookupFree, true, kSched>(w, v, sc, out, sd, lw, blocks_x, grid, stream);
+    if (stats && w.clear_bytes)  // statistics of the steps executed
+      launch_dense_shade<FlatLookupClear, true, kSched>(w, v, sc, out, sd, lw, blocks_x, grid, stream);
     else if (stats)
       launch_dense_shade<FlatLookup, true, kSched>(w, v, sc, out, sd, lw, blocks_x, grid, stream);
-    else if (w.free_bytes)
-      launch_dense_shade<FlatLookupFree, false, kSched>(w, v, sc, out, sd, lw, blocks_x, grid, stream);
+    else if (w.clear_bytes)
+      launch_dense_shade<FlatLookupClear, false, kSched>(w, v, sc, out, sd, lw, blocks_x, grid, stream);
     else if (long_caps)
       launch_dense_shade<FlatLookupLong, false, kSched>(w, v, sc, out, sd, lw, blocks_x, grid, stream);
     else
@@ -238,10 +219,11 @@ hipError_t launch_render_dense(const DenseWorld& w_in, uint32_t traversal, const
                                TileShape tile, uint32_t compute_units, hipStream_t stream) {
   (void)compute_units;
   DenseWorld w = w_in;
-  if (out.steps) w.free_bytes = 0;  // step counts are stored: no early end of rays
-  // nor where they are stored, or counted as traceMap's (statistics without
-  // the free-region test), for the reach box
-  if (out.steps || (out.stats && !w.free_bytes)) reach_everywhere(w.reach_lo, w.reach_hi);
+  // Where step counts are observed (stored, or counted as traceMap's by
+  // statistics without the clearance map) no ray ends early, at the reach box
+  // neither.
+  if (out.steps) w.clear_bytes = 0;
+  if (out.steps || (out.stats && !w.clear_bytes)) reach_everywhere(w.reach_lo, w.reach_hi);
   ShadeConsts sc = sc_in;
   sc.shadow = make_ray_consts(sc.sun[0], sc.sun[1], sc.sun[2], w.mx, w.my, w.mz);
   uint32_t blocks_x, nblocks;
@@ -257,15 +239,15 @@ hipError_t launch_render_dense(const DenseWorld& w_in, uint32_t traversal, const
   return hipGetLastError();
 }
 
-template <bool kStats, bool kFree>
+template <bool kStats, bool kClear>
 static void launch_brickmap(bool sched, const BrickmapWorld& w, const ViewConsts& v,
                             const ShadeConsts& sc, const FrameOut& out, uint32_t* schedule,
                             uint32_t lw, uint32_t blocks_x, dim3 grid, hipStream_t stream) {
   if (sched)
-    hipLaunchKernelGGL((k_render_brickmap<kStats, kFree, true>), grid, dim3(256), 0, stream, w, v,
+    hipLaunchKernelGGL((k_render_brickmap<kStats, kClear, true>), grid, dim3(256), 0, stream, w, v,
                        sc, out, schedule, lw, blocks_x);
   else
-    hipLaunchKernelGGL((k_render_brickmap<kStats, kFree, false>), grid, dim3(256), 0, stream, w,
+    hipLaunchKernelGGL((k_render_brickmap<kStats, kClear, false>), grid, dim3(256), 0, stream, w,
                        v, sc, out, nullptr, lw, blocks_x);
 }
 
@@ -279,10 +261,7 @@ hipError_t launch_render_brickmap(const BrickmapWorld& w_in, const ViewConsts& v
   if (w.dim < 2u * (uint32_t)kSkipLong) w.occ = nullptr;
   // step counts stored, or statistics (of traceMap's steps on this layout):
   // no early end of rays
-  if (out.steps || out.stats) {
-    w.free_bytes = 0;
-    reach_everywhere(w.reach_lo, w.reach_hi);
-  }
+  if (out.steps || out.stats) w.clear_bytes = 0;
   uint32_t blocks_x, nblocks;
   grid_shape(v, tile, blocks_x, nblocks);
   if (schedule && nblocks > VT_SCHEDULE_BLOCKS(v.W, v.H)) return hipErrorInvalidValue;
@@ -291,7 +270,7 @@ hipError_t launch_render_brickmap(const BrickmapWorld& w_in, const ViewConsts& v
   const uint32_t lw = tile.log2_w;
   if (out.stats)
     launch_brickmap<true, false>(sched, w, v, sc, out, schedule, lw, blocks_x, grid, stream);
-  else if (w.occ && w.free_bytes)
+  else if (w.occ && w.clear_bytes)
     launch_brickmap<false, true>(sched, w, v, sc, out, schedule, lw, blocks_x, grid, stream);
   else
     launch_brickmap<false, false>(sched, w, v, sc, out, schedule, lw, blocks_x, grid, stream);

@@ -207,9 +207,9 @@ struct DenseWorld {
   uint32_t nvox;            // dim^3 (bytes of vox)
   const uint32_t* prefix;   // compact albedo index: occupied voxels before each
                             // L0 word (null until built)
-  // free-region map (see FreeMap below); free_bytes 0 = rays are not ended early
-  const uint32_t* freemap;
-  uint32_t free_bytes, free_oct_bytes;
+  // clearance map (see ClearMap below); clear_bytes 0 = not used
+  const uint8_t* clear;
+  uint32_t clear_bytes, clear_oct_bytes;
   // the box of the nonempty voxels widened by the traversal's reach
   // (line_meets_reach); the whole grid when the world is empty; everywhere
   // (reach_everywhere) when step counts are observed
@@ -247,15 +247,20 @@ __device__ __forceinline__ bool in_dim(const DenseWorld& w, int bx, int by, int 
 // world in the reference layout 0.2858 (6) / 0.2892 (7) / 0.292 (8) against
 // 0.2869 (5); the engine's own frame (caps 192/48, short runs between model
 // blocks) 0.2747 at 5 against 0.2972 at 6 and 0.335 at 7.
+// With the clearance map (near something only) 5: the batch 2.32 ms against
+// 2.38 at 6, the engine's map with long caps 272 us against 275.
 constexpr int kSkipShort = 5;
 constexpr int kSkipLong = 6;
+constexpr int kSkipClear = 5;
 constexpr int kLongCap = 512;
+// Steps per turn of the loop without lookups (clear_advance).
+constexpr int kClearSteps = 4;
 
 // Occupancy probe strategies (identical answers by contract).
 struct FlatLookup {
   // one byte gather per probe; returns the material (0 = empty)
   static constexpr bool kPrefetch = true;  // probes have no state: run ahead
-  static constexpr bool kFree = false;     // no free-region test
+  static constexpr bool kClear = false;    // no clearance map
   static constexpr int kSkip = kSkipShort;  // empty-space iteration length
   __device__ __forceinline__ void reset() {}
   template <bool kStats>
@@ -283,7 +288,7 @@ template <uint32_t kBrick>
 struct BitmaskLookupT {
   static_assert(kBrick == 4 || kBrick == 8, "4^3 or 8^3 bricks");
   static constexpr bool kPrefetch = false;
-  static constexpr bool kFree = false;
+  static constexpr bool kClear = false;
   static constexpr int kSkip = kSkipShort;  // (the plain loop has no empty-space phase)
   static constexpr uint32_t kBrickShift = kBrick == 8 ? 9u : 6u;  // log2 codes per brick
   uint32_t brick, region, leaf;
@@ -331,15 +336,16 @@ struct BitmaskLookupT {
 using BitmaskLookup = BitmaskLookupT<4>;
 using BitmaskLookup8 = BitmaskLookupT<8>;
 
-// The flat lookup whose empty-space loops also test the free-region map (see
-// free_rsrc below) and end a ray that can hit nothing more.
-struct FlatLookupFree : FlatLookup {
-  static constexpr bool kFree = true;
-  static constexpr int kSkip = kSkipLong;
+// The flat lookup with the clearance map (see ClearMap below): empty stretches
+// of a ray are crossed without lookups, and a ray whose line meets nothing
+// more ends.
+struct FlatLookupClear : FlatLookup {
+  static constexpr bool kClear = true;
+  static constexpr int kSkip = kSkipClear;
 };
 
 // The flat lookup for frames with long step caps: the longer empty-space
-// iteration, no free-region test.
+// iteration, no clearance map.
 struct FlatLookupLong : FlatLookup {
   static constexpr int kSkip = kSkipLong;
 };
@@ -759,45 +765,170 @@ __device__ __forceinline__ void dense_loop_prefetch(
 enum SkipStatus : int {
   kSkipLimit = 0,    // reached its step limit; every lookup so far empty
   kSkipBlocked = 1,  // an iteration met a nonzero byte or left the grid
-  kSkipFree = 2,     // the ray is in a free region: it can hit nothing more
+  kSkipFree = 2,     // nothing ahead of the ray on all three axes: a miss
+  kSkipOpen = 3,     // the wave's rays stand clear of everything: clear_advance
 };
 
-// The free-region map (built by launch_build_freemap): regions of 16^3
-// blocks, region code = block Morton code >> 12; bit r of the bitmap of
-// direction octant o is set when no region at or ahead of r on every axis in
-// o's travel direction (r included) holds a nonempty block.
+// ---- ClearMap: the clearance map (built by launch_build_clear) ----
+// Cells of 8^3 blocks, R = dim / 8 per axis.  A cell is near when the cell
+// widened by 2 blocks a side holds a nonempty block.  For each direction
+// octant (bit k = travelling negatively on axis k) the byte of a cell is the
+// side m, in cells, of the largest cube of cells none of them near that has
+// this cell as its corner and extends in the octant's travel direction (parts
+// outside the grid count as clear): 0 = the cell is near; 255 = no near cell
+// at or ahead of this one on all three axes.  Each octant's cells are
+// numbered with its negative axes complemented, as the traversal's codes are,
+// twice: in Morton order (8 planes of R^3 bytes, byte c >> 9 for a flipped
+// block code c) and, after those, x + R (y + R z).
 //
-// Why a ray standing in such a region can hit nothing more, so that ending
-// it as a miss changes no output but its step count: a step of traceMap's
-// block-level recurrence moves the crossed axis one block in the travel
-// direction and no axis the other way, and a lookup probes the state's block
-// G or, on a positive axis whose within reached 8, the block after it.  So
-// every later lookup is a block at or ahead of G on every axis -- inside the
-// forward orthant of G's region, or outside the grid, which reads as empty --
-// whatever the rounding and the 0.999 re-anchoring do to within.  With that
-// orthant empty every later lookup reads 0, and traceMap ends by leaving the
-// grid or at its step cap: a miss either way.  Octant bit k = the ray
-// travels negatively on axis k; free_bytes 0 reads as "never free" through
-// the bounds-checked load.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t free_rsrc(const uint32_t* fm, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc((void*)fm, (short)0, (int)bytes, 0x00020000);
+// What it is exact for.  A step of traceMap's block-level recurrence moves
+// the position p = G + within / 8 along the direction by the crossing time tm
+// (p += d tm / 8) up to binary32 rounding (< 1e-6 block), and a crossing of
+// a negative axis re-anchors within at A = 8 x 0.999 instead of 8, 1 - A / 8 =
+// 0.001 block ahead.  After crossing times summing to T the position is
+// therefore p0 + d T / 8 to within 0.001 block per negative crossing (at most
+// dim of them: 1.03 blocks) and the rounding of the sum (< 0.2 block over
+// 3 x 1024 steps), and the block a lookup probes contains the position or
+// touches it.  So while the line p0 + d T / 8 runs through cells that are not
+// near, every probe is at least 2 - 1.3 blocks from the nearest nonempty
+// block: the lookups read empty and need not be made.  Where the line leaves
+// the grid through such cells, or the cell's byte is 255, the ray is a miss.
+//
+// clear_walk follows the line from cube to cube; the walk itself is then
+// taken step by step (its float state must be traceMap's), without lookups
+// and without tracking the block, until the sum of its crossing times says
+// that the line comes near something: 20 VALU a step against 29 with its
+// lookup, and no memory latency.  The block at the end follows from T: axis
+// i crossed n_i = round(((within0 - within) + d T) / 8) boundaries (negative
+// axes: / -A).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t clear_rsrc(const uint8_t* map, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)map, (short)0, (int)bytes, 0x00020000);
 }
 
-// Byte offset of the octant bitmap of a ray whose complemented (negative)
+// Byte offset of the octant plane of a ray whose complemented (negative)
 // axes are `flip`.
-__device__ __forceinline__ uint32_t free_octant_offset(uint32_t flip, uint32_t mx, uint32_t my,
-                                                       uint32_t mz, uint32_t oct_bytes) {
+__device__ __forceinline__ uint32_t clear_octant_offset(uint32_t flip, uint32_t mx, uint32_t my,
+                                                        uint32_t mz, uint32_t oct_bytes) {
   const uint32_t o = ((flip & mx) ? 1u : 0u) | ((flip & my) ? 2u : 0u) | ((flip & mz) ? 4u : 0u);
   return o * oct_bytes;
 }
 
-// The free-map word holding region (block code >> 12) of real block code g.
-__device__ __forceinline__ uint32_t free_word(__amdgpu_buffer_rsrc_t fm, uint32_t fofs,
-                                             uint32_t g) {
-  return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(fm, (int)(fofs + ((g >> 17) << 2)), 0, 0);
+// The map's byte for the cell of flipped block code c.
+__device__ __forceinline__ uint32_t clear_byte(__amdgpu_buffer_rsrc_t cm, uint32_t cofs,
+                                               uint32_t c) {
+  return (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(cm, (int)(cofs + (c >> 9)), 0, 0);
 }
-__device__ __forceinline__ bool free_bit(uint32_t word, uint32_t g) {
-  return ((word >> ((g >> 12) & 31u)) & 1u) != 0u;
+
+// Directions the line argument holds for: every component and reciprocal
+// within 1e-30 .. 1e30 (no product of the walk overflows or turns NaN).
+__device__ __forceinline__ bool clear_usable(float ix, float iy, float iz) {
+  const float a = fabsf(ix), b = fabsf(iy), c = fabsf(iz);
+  return fmaxf(fmaxf(a, b), c) < 1.0e30f && fminf(fminf(a, b), c) > 1.0e-30f;
+}
+
+// From the flipped cell (cx, cy, cz) of the point q (flipped, cell units),
+// follows the line q + |d| T / 64 until it comes to a near cell: true, T =
+// where (0: at once).  False: nothing near ahead.  Each turn takes the
+// largest clear cube from the cell and moves on to the cell behind its far
+// face: at least one axis moves on and none back, so the walk ends within 3 R
+// turns.  Rounding can put the line in a cell next to its own, within 1e-3
+// block of it: the 2-block widening has room for that.  Cell numbers are kept
+// as floats (exact), the index by two fused multiply-adds: a turn is about
+// 45 VALU and one load.
+__device__ __forceinline__ bool clear_walk(__amdgpu_buffer_rsrc_t cm, uint32_t lofs, float R,
+                                           float cx, float cy, float cz, float qx, float qy,
+                                           float qz, float ax, float ay, float az, float bx,
+                                           float by, float bz, float& T) {
+  // a = |d| / 64, b = 64 / |d|
+  T = 0.0f;
+  for (;;) {
+    const uint32_t i = (uint32_t)fmaf(R, fmaf(R, cz, cy), cx);
+    const uint32_t m =
+        (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(cm, (int)(lofs + i), 0, 0);
+    if (m == 0u) return true;
+    if (m == 255u) return false;
+    const float side = (float)m;
+    const float fx = cx + side, fy = cy + side, fz = cz + side;  // behind the far faces
+    const float tx = (fx - qx) * bx, ty = (fy - qy) * by, tz = (fz - qz) * bz;
+    const float t = fminf(fminf(tx, ty), tz);
+    T = fmaxf(T, t);
+    cx = tx > t ? fmaxf(floorf(qx + ax * T), cx) : fx;
+    cy = ty > t ? fmaxf(floorf(qy + ay * T), cy) : fy;
+    cz = tz > t ? fmaxf(floorf(qz + az * T), cz) : fz;
+    if (!(fmaxf(fmaxf(cx, cy), cz) < R)) return false;
+  }
+}
+
+// Takes the ray from state s as far as the clearance map shows its lookups
+// to read empty (steps advanced by as many).  False: the ray is a miss --
+// nothing near ahead, or the walk left the grid or reached max_steps
+// meanwhile.  After crossing times summing to T the walk has crossed at least
+// (|dx| + |dy| + |dz|) T / 8 - 3 boundaries, one a step (each axis at least its
+// line's, the drift being ahead), so a line that comes near something only
+// after max_steps + 5 of them does so past the cap.
+template <int K>
+__device__ __forceinline__ bool clear_advance(float Px, float Py, float Pz, float Ax, float Ay,
+                                              float Az, float dx, float dy, float dz, float ix,
+                                              float iy, float iz, uint32_t flip, uint32_t mx,
+                                              uint32_t my, uint32_t mz, uint32_t dim,
+                                              DenseCell& s, int& steps, int max_steps,
+                                              __amdgpu_buffer_rsrc_t cm, uint32_t cofs,
+                                              uint32_t oct_bytes) {
+  const bool nx = (flip & mx) != 0u, ny = (flip & my) != 0u, nz = (flip & mz) != 0u;
+  uint32_t hx = compact1by2(s.c), hy = compact1by2(s.c >> 1), hz = compact1by2(s.c >> 2);
+  float T;
+  if (!clear_walk(cm, 8u * oct_bytes + cofs, (float)(dim >> 3), (float)(hx >> 3),
+                  (float)(hy >> 3), (float)(hz >> 3),
+                  ((float)hx + (nx ? 8.0f - s.wx : s.wx) * 0.125f) * 0.125f,
+                  ((float)hy + (ny ? 8.0f - s.wy : s.wy) * 0.125f) * 0.125f,
+                  ((float)hz + (nz ? 8.0f - s.wz : s.wz) * 0.125f) * 0.125f,
+                  fabsf(dx) * 0.015625f, fabsf(dy) * 0.015625f, fabsf(dz) * 0.015625f,
+                  fabsf(ix) * 64.0f, fabsf(iy) * 64.0f, fabsf(iz) * 64.0f, T))
+    return false;
+  if ((fabsf(dx) + fabsf(dy) + fabsf(dz)) * T >= 8.0f * (float)(max_steps - steps + 5))
+    return false;  // the cap comes first
+  // K steps take at most K crossing times of the fastest axis
+  const float lim = T - (8.0f * K) * fminf(fminf(fabsf(ix), fabsf(iy)), fabsf(iz));
+  // The wave's rays go on together while all of them can (a wave-uniform
+  // loop): a ray that could go further alone would have the others wait for
+  // it now and wait for them later.
+  if (__ballot(!(lim >= 0.0f)) != 0ull) return true;
+  float wx = s.wx, wy = s.wy, wz = s.wz, t = 0.0f;
+  do {
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      // dense_advance without the block.  No crossing time is NaN here
+      // (clear_usable), so minIdx is z when tz <= min(tx, ty), else x when
+      // tx < ty: traceMap's nested compares.
+      const float tx = (Px - wx) * ix;
+      const float ty = (Py - wy) * iy;
+      const float tz = (Pz - wz) * iz;
+      const float txy = fminf(tx, ty);
+      const bool z = tz <= txy, xy = tx < ty;
+      const float tm = fminf(txy, tz);
+      const float nwx = wx + dx * tm;
+      const float nwy = wy + dy * tm;
+      const float nwz = wz + dz * tm;
+      wx = (xy & !z) ? Ax : nwx;
+      wy = (xy | z) ? nwy : Ay;
+      wz = z ? Az : nwz;
+      t += tm;
+    }
+  } while (__ballot(!(t <= lim)) == 0ull);
+  const float kp = 0.125f, kn = -1.0f / (8.0f * 0.999f);
+  const uint32_t cx = (uint32_t)(int)rintf(((s.wx - wx) + dx * t) * (nx ? kn : kp));
+  const uint32_t cy = (uint32_t)(int)rintf(((s.wy - wy) + dy * t) * (ny ? kn : kp));
+  const uint32_t cz = (uint32_t)(int)rintf(((s.wz - wz) + dz * t) * (nz ? kn : kp));
+  hx += cx;
+  hy += cy;
+  hz += cz;
+  steps += (int)(cx + cy + cz);
+  if ((hx >= dim) | (hy >= dim) | (hz >= dim)) return false;  // left the grid, all empty
+  s.wx = wx;
+  s.wy = wy;
+  s.wz = wz;
+  s.c = morton3(hx, hy, hz);
+  return true;
 }
 
 // Steps K at a time from s while steps + K <= lim without their lookups:
@@ -844,35 +975,36 @@ __device__ __forceinline__ void dense_skip_blind(float Px, float Py, float Pz, f
 // K steps instead of one per step, and with it none of the per-step copies of
 // the exit state that a divergent exit costs.  An iteration only starts when
 // steps + K < limit (limit <= max_steps), so the step cap falls inside the
-// replay.  Each iteration also requests the free-map word of its start
-// block and, when that region is free for the ray's octant (bitmap at byte
-// `fofs` of `fm`), ends the run with kSkipFree: the ray can hit nothing
-// more.  Returns kSkipBlocked when it stopped at an iteration that met a
-// nonzero byte or left the grid, kSkipLimit at the limit; either way `s` is
-// a state the exact loop (or another call) continues from.
+// replay.  With kClear each iteration also requests the clearance map's byte
+// of its start block (octant plane at `cofs` of `cm`): 255 ends the run with
+// kSkipFree, the ray can hit nothing more; when the cells of all the wave's
+// rays in the loop have clear neighbours ahead (>= 2) they leave together
+// with kSkipOpen for clear_advance (one ray at a time would have the wave
+// alternate between the loops).  Returns kSkipBlocked when it stopped at an
+// iteration that met a nonzero byte or left the grid, kSkipLimit at the
+// limit; either way `s` is a state the exact loop (or another call)
+// continues from.
 //
 // The lookup of a state with within >= 8 probes the next block.  Instead of
 // a branch at every step the iteration is taken without that correction and
 // taken again with it when a crossing time says that such a state was among
-// them (4% of the rays of a terrain frame meet one), and the grid's edge is
-// tested once an iteration: 29 VALU + 8 SALU a step against 31 + 15 and the
-// branch.  Frames of the 128^3 world at 256x256 42.8 -> 36.8 us, the engine's
-// world with long caps at 1600x900 199 -> 178.
-template <int K, bool kFree>
+// them (4% of the rays of a terrain frame meet one): 29 VALU + 8 SALU a step
+// against 39 + 19.
+template <int K, bool kClear>
 __device__ __forceinline__ int dense_skip_empty(float Px, float Py, float Pz, float Ax, float Ay,
                                                 float Az, float dx, float dy, float dz, float ix,
                                                 float iy, float iz, uint32_t mx, uint32_t my,
                                                 uint32_t mz, uint32_t flip, DenseCell& s,
                                                 int& steps, int limit,
                                                 __amdgpu_buffer_rsrc_t bytes,
-                                                __amdgpu_buffer_rsrc_t fm, uint32_t fofs) {
+                                                __amdgpu_buffer_rsrc_t cm, uint32_t cofs,
+                                                bool usable) {
   float bx = s.wx, by = s.wy, bz = s.wz;
   uint32_t bc = s.c;
   int sb = steps;
   int status = kSkipLimit;
   while (sb + K < limit) {
-    const uint32_t g = bc ^ flip;
-    const uint32_t fw = kFree ? free_word(fm, fofs, g) : 0u;
+    const uint32_t m = kClear ? clear_byte(cm, cofs, bc) : 0u;
     float wx = bx, wy = by, wz = bz;
     uint32_t c = bc, any = 0u;
     float mn = 1.0f;  // smallest crossing time of the steps from S_1 .. S_K-1
@@ -898,7 +1030,7 @@ __device__ __forceinline__ int dense_skip_empty(float Px, float Py, float Pz, fl
         any |= (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(bytes, (int)n.a, 0, 0);
       }
     }
-    if (kFree && free_bit(fw, g)) {
+    if (kClear && m == 255u) {
       status = kSkipFree;
       break;
     }
@@ -911,6 +1043,10 @@ __device__ __forceinline__ int dense_skip_empty(float Px, float Py, float Pz, fl
     bz = wz;
     bc = c;
     sb += K;
+    if (kClear && __ballot(!((m >= 2u) & usable)) == 0ull) {
+      status = kSkipOpen;
+      break;
+    }
   }
   s.wx = bx;
   s.wy = by;
@@ -937,19 +1073,19 @@ __device__ __forceinline__ int dense_skip_empty(float Px, float Py, float Pz, fl
 // iteration and takes the general branch (dense_step's).  Shadow rays start
 // on lattice points, so this correction is frequent for them: as a branch it
 // ran in about half of the wave-steps.
-// The free-map test is dense_skip_empty's, on octant 0's bitmap (`fm`).
-template <int K, bool kFree>
+// The clearance map's part is dense_skip_empty's, on octant 0's plane.
+template <int K, bool kClear>
 __device__ __forceinline__ int dense_skip_positive(float dx, float dy, float dz, float ix,
                                                    float iy, float iz, uint32_t mx, uint32_t my,
                                                    uint32_t mz, DenseCell& s, int& steps,
                                                    int limit, __amdgpu_buffer_rsrc_t bytes,
-                                                   __amdgpu_buffer_rsrc_t fm) {
+                                                   __amdgpu_buffer_rsrc_t cm, bool usable) {
   float bx = s.wx, by = s.wy, bz = s.wz;
   uint32_t bc = s.c;
   int sb = steps;
   int status = kSkipLimit;
   while (sb + K < limit) {
-    const uint32_t fw = kFree ? free_word(fm, 0u, bc) : 0u;
+    const uint32_t m = kClear ? clear_byte(cm, 0u, bc) : 0u;
     float wx = bx, wy = by, wz = bz;
     uint32_t c = bc;
     uint32_t any = 0u;
@@ -989,7 +1125,7 @@ __device__ __forceinline__ int dense_skip_positive(float dx, float dy, float dz,
       }
       any |= (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(bytes, (int)a, 0, 0);
     }
-    if (kFree && free_bit(fw, bc)) {
+    if (kClear && m == 255u) {
       status = kSkipFree;
       break;
     }
@@ -1002,6 +1138,10 @@ __device__ __forceinline__ int dense_skip_positive(float dx, float dy, float dz,
     bz = wz;
     bc = c;
     sb += K;
+    if (kClear && __ballot(!((m >= 2u) & usable)) == 0ull) {
+      status = kSkipOpen;
+      break;
+    }
   }
   s.wx = bx;
   s.wy = by;
@@ -1013,9 +1153,10 @@ __device__ __forceinline__ int dense_skip_positive(float dx, float dy, float dz,
 
 // The flat lookup's traversal from r's block-level state: the empty-space
 // phase, then the exact loop to the ray's end.
-// kPositive: the caller guarantees a direction positive on every axis (after
-// the zero substitution), and the empty-space phase is dense_skip_positive.
-template <class L, bool kPositive = false>
+// kShadow: the ray starts next to a nonempty voxel.  kPositive: the caller
+// guarantees a direction positive on every axis (after the zero
+// substitution), and the empty-space phase is dense_skip_positive.
+template <class L, bool kPositive = false, bool kShadow = false>
 __device__ __forceinline__ void dense_run_prefetch(DenseRay& r, L& lk, const DenseWorld& w,
                                                    DenseHit& h) {
   const uint32_t mx = in_vgpr(w.mx), my = in_vgpr(w.my), mz = in_vgpr(w.mz), flip = r.flip;
@@ -1028,28 +1169,58 @@ __device__ __forceinline__ void dense_run_prefetch(DenseRay& r, L& lk, const Den
   const __amdgpu_buffer_rsrc_t vox =
       __builtin_amdgcn_make_buffer_rsrc((void*)w.vox, (short)0, (int)w.nvox, 0x00020000);
   int steps0 = r.steps;
-  const __amdgpu_buffer_rsrc_t fm = free_rsrc(w.freemap, w.free_bytes);
   int status;
-  if constexpr (kPositive)
-    status = dense_skip_positive<L::kSkip, L::kFree>(r.dx, r.dy, r.dz, r.ix, r.iy, r.iz, mx,
-                                                          my, mz, s0, steps0, max_steps, vox, fm);
-  else {
+  if constexpr (L::kClear) {
+    // clear stretches without lookups and stretches near something with
+    // them, in turn; a primary ray starts with the former, a shadow ray (it
+    // starts at a nonempty voxel) with the latter
+    const __amdgpu_buffer_rsrc_t cm = clear_rsrc(w.clear, w.clear_bytes);
+    const uint32_t cofs =
+        kPositive ? 0u : clear_octant_offset(flip, mx, my, mz, w.clear_oct_bytes);
+    const bool usable = clear_usable(r.ix, r.iy, r.iz);
+    bool open = !kShadow;
+    int blind = 0;
+    for (;;) {
+      if (open & usable) {
+        const int s1 = steps0;
+        const bool on = clear_advance<kClearSteps>(
+            r.Px, r.Py, r.Pz, r.Ax, r.Ay, r.Az, r.dx, r.dy, r.dz, r.ix, r.iy, r.iz, flip, mx, my,
+            mz, w.dim, s0, steps0, max_steps, cm, cofs, w.clear_oct_bytes);
+        blind += steps0 - s1;
+        if (!on || steps0 >= max_steps) {
+          status = kSkipFree;
+          break;
+        }
+      }
+      if constexpr (kPositive)
+        status = dense_skip_positive<L::kSkip, true>(r.dx, r.dy, r.dz, r.ix, r.iy, r.iz, mx, my,
+                                                     mz, s0, steps0, max_steps, vox, cm, usable);
+      else
+        status = dense_skip_empty<L::kSkip, true>(
+            r.Px, r.Py, r.Pz, r.Ax, r.Ay, r.Az, r.dx, r.dy, r.dz, r.ix, r.iy, r.iz, mx, my, mz,
+            flip, s0, steps0, max_steps, vox, cm, cofs, usable);
+      if (status != kSkipOpen) break;
+      open = true;
+    }
+    r.blind = blind;  // the steps taken without lookups
+    if (status == kSkipFree) {  // a miss: no later lookup can be nonzero
+      h.hit = false;
+      h.steps = min(steps0, max_steps);
+      return;
+    }
+  } else if constexpr (kPositive) {
+    dense_skip_positive<L::kSkip, false>(r.dx, r.dy, r.dz, r.ix, r.iy, r.iz, mx, my, mz, s0,
+                                         steps0, max_steps, vox, vox, false);
+  } else {
     // the lookups that can only read empty first (primary rays), the
     // iteration that reaches the cap left to the loops below
-    const int sblind = steps0;
     if (r.blind > steps0)
       dense_skip_blind<L::kSkip>(r.Px, r.Py, r.Pz, r.Ax, r.Ay, r.Az, r.dx, r.dy, r.dz, r.ix,
                                  r.iy, r.iz, mx, my, mz, s0, steps0,
                                  min(r.blind, max_steps - 1));
-    r.blind = steps0 - sblind;  // the steps taken without lookups
-    status = dense_skip_empty<L::kSkip, L::kFree>(
-        r.Px, r.Py, r.Pz, r.Ax, r.Ay, r.Az, r.dx, r.dy, r.dz, r.ix, r.iy, r.iz, mx, my, mz, flip,
-        s0, steps0, max_steps, vox, fm, free_octant_offset(flip, mx, my, mz, w.free_oct_bytes));
-  }
-  if (L::kFree && status == kSkipFree) {  // a miss: no later lookup can be nonzero
-    h.hit = false;
-    h.steps = steps0 + L::kSkip;  // the steps executed, the last iteration's included
-    return;
+    dense_skip_empty<L::kSkip, false>(r.Px, r.Py, r.Pz, r.Ax, r.Ay, r.Az, r.dx, r.dy, r.dz, r.ix,
+                                      r.iy, r.iz, mx, my, mz, flip, s0, steps0, max_steps, vox,
+                                      vox, 0u, false);
   }
   float fwx, fwy, fwz;
   uint32_t fc, fM, fa, fv;
@@ -1083,12 +1254,12 @@ __device__ __forceinline__ void dense_run_prefetch(DenseRay& r, L& lk, const Den
   h.steps = sF + 1;
 }
 
-// kStats with the free-region lookup keeps the fast loops: its statistics
-// count the steps executed, rays ending early included.
+// kStats with the clearance map keeps the fast loops: its statistics count
+// the steps executed, rays ending early included.
 template <bool kStats, class L>
 __device__ __forceinline__ void dense_run(DenseRay& r, L& lk, const DenseWorld& w, DenseHit& h,
                                           uint32_t& l1f, uint32_t& l0f) {
-  if constexpr (L::kPrefetch && (!kStats || L::kFree)) {
+  if constexpr (L::kPrefetch && (!kStats || L::kClear)) {
     dense_run_prefetch(r, lk, w, h);
     return;
   }
@@ -1166,27 +1337,11 @@ struct BrickmapWorld {
   const uint8_t* occ;
   uint32_t nvox;           // dim^3
   uint32_t mx, my, mz;     // dilated Morton masks of x, y, z
-  // free-region map of the occupancy bytes; free_bytes 0 = none
-  const uint32_t* freemap;
-  uint32_t free_bytes, free_oct_bytes;
-  // the box of the nonempty blocks widened by the traversal's reach (as
-  // DenseWorld's: line_meets_reach)
-  float reach_lo[3], reach_hi[3];
+  // clearance map of the occupancy bytes (as DenseWorld's); clear_bytes 0 =
+  // not used
+  const uint8_t* clear;
+  uint32_t clear_bytes, clear_oct_bytes;
 };
-
-// line_meets_reach of a reference-layout world: the same exactness argument
-// (every probe before the first nonempty block is a block-level step of the
-// same recurrence); d is the direction before the zero substitution.  Also
-// the ray's blind_steps.
-__device__ __forceinline__ bool line_meets_reach_bm(const BrickmapWorld& w, float ex, float ey,
-                                                    float ez, float dx, float dy, float dz,
-                                                    int& blind) {
-  const float d[3] = {dx == 0.0f ? 0.001f : dx, dy == 0.0f ? 0.001f : dy,
-                      dz == 0.0f ? 0.001f : dz};
-  const float inv[3] = {1.0f / d[0], 1.0f / d[1], 1.0f / d[2]};
-  blind = blind_steps_box(w.reach_lo, w.reach_hi, ex, ey, ez, d, inv);
-  return line_meets_box(w.reach_lo, w.reach_hi, ex, ey, ez, inv);
-}
 
 // map_getVoxel (map.glsl:38-47) of block coordinates b; counts the chunk-table
 // and pool reads it makes.
@@ -1322,16 +1477,15 @@ __device__ bool trace_general(const BrickmapWorld& w, float ox, float oy, float 
 // kPositive: the caller guarantees a direction with no negative component (the
 // zero substitution below makes it positive), and the empty-space steps take
 // dense_skip_positive.
-// kFree: the empty-space loop tests the free-region map of the occupancy
-// bytes and ends a ray that can hit nothing more; the launcher takes it for
-// long step caps, so it also takes the longer empty-space iteration.
-// blind: leading steps whose lookups can only read empty (blind_steps; 0
-// for none).
-template <bool kPositive = false, bool kFree = false>
+// kClear: the empty-space runs take the clearance map of the occupancy bytes.
+// It holds here too: block-level lookups only descend into nonempty blocks,
+// so a stretch whose block-level lookups all read empty is walked at the
+// block level, and each run starts its line from the walk's own position.
+// kShadow: the ray starts next to a nonempty block.
+template <bool kPositive = false, bool kClear = false, bool kShadow = false>
 __device__ bool trace_brickmap_fast(const BrickmapWorld& w, float ox, float oy, float oz, float dx,
-                                    float dy, float dz, int max_steps, GeneralHit& h,
-                                    int blind = 0) {
-  constexpr int kSkip = kFree ? kSkipLong : kSkipShort;
+                                    float dy, float dz, int max_steps, GeneralHit& h) {
+  constexpr int kSkip = kClear ? kSkipClear : kSkipShort;
   if (dx == 0.0f) dx = 0.001f;
   if (dy == 0.0f) dy = 0.001f;
   if (dz == 0.0f) dz = 0.001f;
@@ -1357,6 +1511,11 @@ __device__ bool trace_brickmap_fast(const BrickmapWorld& w, float ox, float oy, 
   h.hx = h.hy = h.hz = -1.0f;
   int step = 0;
   bool hit = false;
+  // the map's plane and whether the direction allows it; a primary ray's
+  // first run starts with a stretch without lookups
+  const __amdgpu_buffer_rsrc_t cm = clear_rsrc(w.clear, w.clear_bytes);
+  const bool usable = kClear && clear_usable(inv[0], inv[1], inv[2]);
+  bool open = kClear && !kShadow;
   for (;;) {
     // The literal loop (both levels) until the lane stands at an empty
     // block at the block level, hits, leaves the map or reaches the cap.
@@ -1432,26 +1591,35 @@ __device__ bool trace_brickmap_fast(const BrickmapWorld& w, float ox, float oy, 
     s0.c = morton3((uint32_t)g[0] >> 3, (uint32_t)g[1] >> 3, (uint32_t)g[2] >> 3) ^ flip;
     const uint32_t mx = in_vgpr(w.mx), my = in_vgpr(w.my), mz = in_vgpr(w.mz);
     int s0steps = step;
-    const int lim = max_steps;
-    // the free-region map of the occupancy bytes: block-level lookups only
-    // descend into nonempty blocks, so a ray whose block-level lookups all
-    // read empty from here on is a miss
-    const __amdgpu_buffer_rsrc_t fm = free_rsrc(w.freemap, w.free_bytes);
     int status;
-    if constexpr (kPositive)
-      status = dense_skip_positive<kSkip, kFree>(d[0], d[1], d[2], inv[0], inv[1], inv[2],
-                                                         mx, my, mz, s0, s0steps, lim, occ, fm);
-    else {
-      if (blind > s0steps)
-        dense_skip_blind<kSkip>(P3[0], P3[1], P3[2], A3[0], A3[1], A3[2], d[0], d[1], d[2],
-                                inv[0], inv[1], inv[2], mx, my, mz, s0, s0steps,
-                                min(blind, max_steps - 1));
-      status = dense_skip_empty<kSkip, kFree>(
-          P3[0], P3[1], P3[2], A3[0], A3[1], A3[2], d[0], d[1], d[2], inv[0], inv[1], inv[2], mx,
-          my, mz, flip, s0, s0steps, lim, occ, fm,
-          free_octant_offset(flip, mx, my, mz, w.free_oct_bytes));
+    const uint32_t cofs =
+        kPositive || !kClear ? 0u : clear_octant_offset(flip, mx, my, mz, w.clear_oct_bytes);
+    for (;;) {
+      if constexpr (kClear) {
+        if (open & usable) {
+          if (!clear_advance<kClearSteps>(P3[0], P3[1], P3[2], A3[0], A3[1], A3[2], d[0], d[1],
+                                          d[2], inv[0], inv[1], inv[2], flip, mx, my, mz, w.dim,
+                                          s0, s0steps, max_steps, cm, cofs, w.clear_oct_bytes) ||
+              s0steps >= max_steps) {
+            status = kSkipFree;
+            break;
+          }
+        }
+      }
+      if constexpr (kPositive)
+        status = dense_skip_positive<kSkip, kClear>(d[0], d[1], d[2], inv[0], inv[1], inv[2], mx,
+                                                    my, mz, s0, s0steps, max_steps, occ, cm,
+                                                    usable);
+      else
+        status = dense_skip_empty<kSkip, kClear>(P3[0], P3[1], P3[2], A3[0], A3[1], A3[2], d[0],
+                                                 d[1], d[2], inv[0], inv[1], inv[2], mx, my, mz,
+                                                 flip, s0, s0steps, max_steps, occ, cm, cofs,
+                                                 usable);
+      if (status != kSkipOpen) break;
+      open = true;
     }
-    if (kFree && status == kSkipFree) {
+    open = false;  // the next run starts at a nonempty block
+    if (kClear && status == kSkipFree) {
       step = s0steps;
       break;
     }
