@@ -246,6 +246,9 @@ ViewConsts view_consts(const vt_camera* camera, uint32_t W, uint32_t H) {
   v.tan_half = (float)std::tan((double)(camera->fov / 2.0f));
   v.W = W;
   v.H = H;
+  v.aspect = (float)H / (float)W;
+  v.inv_w = 1.0 / (double)(float)W;
+  v.inv_h = 1.0 / (double)(float)H;
   return v;
 }
 
@@ -254,6 +257,19 @@ ShadeConsts shade_consts(const vt_render_params& p) {
   std::memcpy(sc.sun, p.sun, sizeof sc.sun);
   // the dense launchers redo this with the world's axis masks
   sc.shadow = make_ray_consts(p.sun[0], p.sun[1], p.sun[2], 0u, 0u, 0u);
+  sc.sun_len = len3(p.sun[0], p.sun[1], p.sun[2]);
+  const bool unorm = (p.flags & VT_FLAG_GBUF_UNORM8) != 0u;
+  sc.cull_entities = true;
+  for (int i = 0; i < 3; i++) {
+    sc.sun_n[i] = p.sun[i] / sc.sun_len;
+    sc.illum[i] = unorm ? unorm8(p.sun[i]) : p.sun[i];
+    sc.cull_entities &= std::fabs(p.sun[i]) > 1.0e-20f && std::fabs(p.sun[i]) < 1.0e20f;
+  }
+  sc.illum_lit = unorm ? unorm8(0.3f) : 0.3f;
+  sc.illum_occ = unorm ? unorm8(-0.3f) : -0.3f;
+  const float li = len3(sc.illum[0], sc.illum[1], sc.illum[2]);
+  sky_dome(sc.sun_n, sc.illum[0] / li, sc.illum[1] / li, sc.illum[2] / li, sc.illum[1], sc.sky[0],
+           sc.sky[1], sc.sky[2]);
   sc.max_primary = p.max_steps_primary;
   sc.max_shadow = p.max_steps_shadow;
   sc.flags = p.flags;

@@ -230,7 +230,10 @@ __global__ void k_pick_brickmap(const BrickmapWorld w, ViewConsts v, int max_ste
   // through the loop that keeps several in flight (same steps, same count)
   GeneralHit g;
   if (w.occ) {
-    trace_brickmap_fast<false, false>(w, e[0], e[1], e[2], d[0], d[1], d[2], max_steps, g);
+    const float inv[3] = {1.0f / (d[0] == 0.0f ? 0.001f : d[0]),
+                          1.0f / (d[1] == 0.0f ? 0.001f : d[1]),
+                          1.0f / (d[2] == 0.0f ? 0.001f : d[2])};
+    trace_brickmap_fast<false, false>(w, e[0], e[1], e[2], d[0], d[1], d[2], inv, max_steps, g);
   } else {
     uint32_t chunk_reads = 0, pool_reads = 0;
     trace_general<false>(w, e[0], e[1], e[2], d[0], d[1], d[2], max_steps, g, chunk_reads,

@@ -109,6 +109,12 @@ void dev_free(void* p);
 struct ShadeConsts {
   float sun[3];
   RayConsts shadow;  // the shadow rays' direction constants (set by the dense launchers)
+  // what every hit has in common (the illumination image holds the sun):
+  float sun_n[3], sun_len;     // sun / |sun| and |sun|
+  float illum[3];              // illumination.xyz, through rgba8 if the G-buffer is
+  float illum_lit, illum_occ;  // illumination.w
+  float sky[3];                // the sky's colour along illumination.xyz
+  bool cull_entities;          // may_meet_entities holds for the sun
   int max_primary, max_shadow;
   uint32_t flags;
   float ambient;

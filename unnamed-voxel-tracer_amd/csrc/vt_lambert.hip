@@ -37,7 +37,7 @@ __global__ __launch_bounds__(256) void k_lambert_shade(DenseWorld w, ShadeConsts
   if (record_hit(w, voxel)) {
     const int face = (int)(info & 7u);
     const bool occl = ((info >> 3) & 1u) != 0u;
-    const LambertSun ls = lambert_sun(sc.sun);
+    const LambertSun ls = lambert_sun(sc);
     const float nd = lambert_nd(face, ls);
     const float fct = lambert_factor(sc.ambient, nd, occl);
     const uint32_t code = (sc.flags & VT_FLAG_ALBEDO_COMPACT) ? voxel_code(w, voxel) : 0u;
@@ -59,7 +59,7 @@ __global__ __launch_bounds__(256) void k_lambert_backward(DenseWorld w, ShadeCon
                                                           const float4* __restrict__ up,
                                                           uint32_t kind) {
   GradAcc acc = grad_acc();
-  const LambertSun ls = lambert_sun(sc.sun);
+  const LambertSun ls = lambert_sun(sc);
   const bool compact = (sc.flags & VT_FLAG_ALBEDO_COMPACT) != 0u;
   const uint32_t span = 256u * kBwdUnroll;
   // grid-stride over block spans of 256 x kBwdUnroll pixels, the wave's

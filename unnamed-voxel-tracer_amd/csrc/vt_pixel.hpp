@@ -265,12 +265,12 @@ struct LambertSun {
   float lx, ly, lz, ls;  // sun / |sun| and |sun|
 };
 
-__device__ __forceinline__ LambertSun lambert_sun(const float sun[3]) {
+__device__ __forceinline__ LambertSun lambert_sun(const ShadeConsts& sc) {
   LambertSun s;
-  s.ls = len3(sun[0], sun[1], sun[2]);
-  s.lx = sun[0] / s.ls;
-  s.ly = sun[1] / s.ls;
-  s.lz = sun[2] / s.ls;
+  s.ls = sc.sun_len;
+  s.lx = sc.sun_n[0];
+  s.ly = sc.sun_n[1];
+  s.lz = sc.sun_n[2];
   return s;
 }
 
@@ -415,10 +415,10 @@ __device__ __forceinline__ void shadow_origin(const Primary& p, uint32_t flags, 
   float px = ceilf(p.hx) / 8.0f, py = ceilf(p.hy) / 8.0f, pz = ceilf(p.hz) / 8.0f;
   float nx, ny, nz;
   face_normal(p.face, nx, ny, nz);
-  if (flags & VT_FLAG_GBUF_UNORM8) {
-    nx = unorm8(nx);
-    ny = unorm8(ny);
-    nz = unorm8(nz);
+  if (flags & VT_FLAG_GBUF_UNORM8) {  // unorm8 of -1, 0 and 1
+    nx = fmaxf(nx, 0.0f);
+    ny = fmaxf(ny, 0.0f);
+    nz = fmaxf(nz, 0.0f);
   }
   sox = px + nx * 0.001f;
   soy = py + ny * 0.001f;
@@ -437,11 +437,10 @@ __host__ __device__ constexpr int shade_mode(uint32_t flags) {
 }
 
 // Colour image of a hit: unpackUnorm4x8(data) (primary.comp.glsl:58-60).
-__device__ __forceinline__ float4 hit_color(uint32_t data, bool unorm) {
-  float4 col = make_float4((float)(data & 255u) / 255.0f, (float)((data >> 8) & 255u) / 255.0f,
-                           (float)((data >> 16) & 255u) / 255.0f, (float)(data >> 24) / 255.0f);
-  if (unorm) col = make_float4(unorm8(col.x), unorm8(col.y), unorm8(col.z), unorm8(col.w));
-  return col;
+__device__ __forceinline__ float4 hit_color(uint32_t data) {
+  // through rgba8 and back it is the same: round((b / 255) 255) = b
+  return make_float4(over255((float)(data & 255u)), over255((float)((data >> 8) & 255u)),
+                     over255((float)((data >> 16) & 255u)), over255((float)(data >> 24)));
 }
 
 // Normal and position images and the hit distance of a primary hit
@@ -452,23 +451,26 @@ __device__ __forceinline__ void hit_normal_position(const ViewConsts& v, const P
   float nx, ny, nz;
   face_normal(p.face, nx, ny, nz);
   nrm = make_float4(nx, ny, nz, 1.0f);
-  if (unorm) nrm = make_float4(unorm8(nrm.x), unorm8(nrm.y), unorm8(nrm.z), unorm8(nrm.w));
+  if (unorm) nrm = make_float4(fmaxf(nx, 0.0f), fmaxf(ny, 0.0f), fmaxf(nz, 0.0f), 1.0f);
   pos = make_float4(ceilf(p.hx) / 8.0f, ceilf(p.hy) / 8.0f, ceilf(p.hz) / 8.0f, 1.0f);
   t = len3(p.hx / 8.0f - v.pos[0], p.hy / 8.0f - v.pos[1], p.hz / 8.0f - v.pos[2]);
 }
 
 // traceEntities(rayOrigin, rayDir, distance(rayOrigin, inter.hit_pos / 8.))
-// and the illumination image of a hit (secondary.comp.glsl:36-50).
-__device__ __forceinline__ float4 shadow_illum(const ShadeConsts& sc, bool unorm, bool shit,
-                                               float shx, float shy, float shz, float sox,
-                                               float soy, float soz, bool& ent, bool& occl) {
-  float hx8 = shx / 8.0f, hy8 = shy / 8.0f, hz8 = shz / 8.0f;
-  float maxd = len3(sox - hx8, soy - hy8, soz - hz8);
-  ent = trace_entities(sox, soy, soz, sc.sun[0], sc.sun[1], sc.sun[2], maxd);
+// and the illumination image of a hit (secondary.comp.glsl:36-50).  Whether an
+// entity occludes a pixel that a voxel already does is only counted (kStats).
+template <bool kStats>
+__device__ __forceinline__ float4 shadow_illum(const ShadeConsts& sc, bool shit, float shx,
+                                               float shy, float shz, float sox, float soy,
+                                               float soz, bool& ent, bool& occl) {
+  ent = false;
+  if (kStats || (!shit && (!sc.cull_entities || may_meet_entities(sox, soy, soz, sc.shadow.inv)))) {
+    float hx8 = shx / 8.0f, hy8 = shy / 8.0f, hz8 = shz / 8.0f;
+    float maxd = len3(sox - hx8, soy - hy8, soz - hz8);
+    ent = trace_entities(sox, soy, soz, sc.sun[0], sc.sun[1], sc.sun[2], maxd);
+  }
   occl = ent || shit;
-  float4 ill = make_float4(sc.sun[0], sc.sun[1], sc.sun[2], occl ? -0.3f : 0.3f);
-  if (unorm) ill = make_float4(unorm8(ill.x), unorm8(ill.y), unorm8(ill.z), unorm8(ill.w));
-  return ill;
+  return make_float4(sc.illum[0], sc.illum[1], sc.illum[2], occl ? sc.illum_occ : sc.illum_lit);
 }
 
 // Hit-record info word: face | shadow << 3 | sub-voxel << 4 | material << 16.
@@ -485,10 +487,8 @@ __device__ __forceinline__ void store_ref_composite(const ViewConsts& v, const S
                                                     bool hit) {
   float4 s;
   if (hit) {
-    float r, g, b;
-    sky(sc.sun, ill.x, ill.y, ill.z, r, g, b);
-    s = make_float4(col.x + ill.w * r, col.y + ill.w * g, col.z + ill.w * b,
-                    col.w + ill.w * 1.0f);
+    s = make_float4(col.x + ill.w * sc.sky[0], col.y + ill.w * sc.sky[1],
+                    col.z + ill.w * sc.sky[2], col.w + ill.w * 1.0f);
   } else {
     s = col;
   }
@@ -499,7 +499,7 @@ __device__ __forceinline__ void store_ref_composite(const ViewConsts& v, const S
   out.shaded[pix] = s;
 }
 
-template <int kShade>
+template <int kShade, bool kStats>
 __device__ __forceinline__ void write_pixel(const ViewConsts& v, const ShadeConsts& sc,
                                             const FrameOut& out, uint32_t px, uint32_t py,
                                             const Primary& p, bool shit, float shx, float shy,
@@ -512,10 +512,10 @@ __device__ __forceinline__ void write_pixel(const ViewConsts& v, const ShadeCons
   float t;
   bool occl = false;
   if (p.hit) {
-    col = hit_color(p.data, unorm);
+    col = hit_color(p.data);
     hit_normal_position(v, p, unorm, nrm, pos, t);
     bool ent;
-    ill = shadow_illum(sc, unorm, shit, shx, shy, shz, sox, soy, soz, ent, occl);
+    ill = shadow_illum<kStats>(sc, shit, shx, shy, shz, sox, soy, soz, ent, occl);
     cnt.hits++;
     cnt.occluded += occl ? 1u : 0u;
     cnt.ent += ent ? 1u : 0u;
@@ -524,7 +524,7 @@ __device__ __forceinline__ void write_pixel(const ViewConsts& v, const ShadeCons
     float dx, dy, dz;
     raygen(v, px, py, dx, dy, dz);
     float r, g, b;
-    sky(sc.sun, dx, dy, dz, r, g, b);
+    sky(sc.sun_n, dx, dy, dz, r, g, b);
     col = make_float4(r, g, b, 1.0f);
     if (unorm) col = make_float4(unorm8(r), unorm8(g), unorm8(b), 1.0f);
     nrm = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
@@ -551,7 +551,7 @@ __device__ __forceinline__ void write_pixel(const ViewConsts& v, const ShadeCons
     float4 T = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     if constexpr (grad) T = out.target[pix];
     if (p.hit) {
-      const LambertSun ls = lambert_sun(sc.sun);
+      const LambertSun ls = lambert_sun(sc);
       const float nd = lambert_nd(p.face, ls);
       const float fct = lambert_factor(sc.ambient, nd, occl);
       const uint32_t ai = albedo_index(*dw, sc.flags, p.voxel, p.code);
@@ -583,7 +583,7 @@ __device__ __forceinline__ void store_hit_primary(const ViewConsts& v, const Sha
   float4 nrm, pos;
   float t;
   hit_normal_position(v, p, unorm, nrm, pos, t);
-  if (out.color) out.color[pix] = hit_color(p.data, unorm);
+  if (out.color) out.color[pix] = hit_color(p.data);
   if (out.normal) out.normal[pix] = nrm;
   if (out.position) out.position[pix] = pos;
   if (out.hits) {
@@ -594,6 +594,7 @@ __device__ __forceinline__ void store_hit_primary(const ViewConsts& v, const Sha
 
 // Second half, once the shadow ray (shit, sh*, ssteps) is done: data = the
 // primary colour, info0 = its hit-record info word without the shadow bit.
+template <bool kStats>
 __device__ __forceinline__ void store_hit_shadow_ref(const ViewConsts& v, const ShadeConsts& sc,
                                                      const FrameOut& out, uint32_t px,
                                                      uint32_t py, uint32_t data, uint32_t info0,
@@ -601,9 +602,8 @@ __device__ __forceinline__ void store_hit_shadow_ref(const ViewConsts& v, const 
                                                      float shy, float shz, float sox, float soy,
                                                      float soz, int ssteps, Counters& cnt) {
   const size_t pix = (size_t)py * v.W + px;
-  const bool unorm = (sc.flags & VT_FLAG_GBUF_UNORM8) != 0u;
   bool ent, occl;
-  const float4 ill = shadow_illum(sc, unorm, shit, shx, shy, shz, sox, soy, soz, ent, occl);
+  const float4 ill = shadow_illum<kStats>(sc, shit, shx, shy, shz, sox, soy, soz, ent, occl);
   cnt.hits++;
   cnt.occluded += occl ? 1u : 0u;
   cnt.ent += ent ? 1u : 0u;
@@ -613,7 +613,7 @@ __device__ __forceinline__ void store_hit_shadow_ref(const ViewConsts& v, const 
   if (out.steps) out.steps[pix] = (uint32_t)psteps | ((uint32_t)ssteps << 16);
   if (out.hits) out.hits[3 * pix + 2] = info0 | ((occl ? 1u : 0u) << 3);
   if (out.shaded)
-    store_ref_composite(v, sc, out, pix, px, py, hit_color(data, unorm), ill, true);
+    store_ref_composite(v, sc, out, pix, px, py, hit_color(data), ill, true);
 }
 
 __device__ __forceinline__ uint32_t wave_sum(uint32_t x) {
@@ -643,16 +643,10 @@ __device__ __forceinline__ void trace_pixel_dense(const DenseWorld& w, const Vie
   DenseHit h;
   Primary p;
   // ---- primary ray (primary.comp.glsl:31-43) ----
-  float dx, dy, dz;
-  raygen(v, px, py, dx, dy, dz);
-  float tn, tf;
-  const float D = (float)w.dim;
-  intersect_aabb(v.pos[0], v.pos[1], v.pos[2], dx, dy, dz, 0.0f, 0.0f, 0.0f, D, D, D, tn, tf);
-  float tc = fmaxf(tn, 0.0f);
-  float ex = (v.pos[0] + dx * tc) - 0.001f;
-  float ey = (v.pos[1] + dy * tc) - 0.001f;
-  float ez = (v.pos[2] + dz * tc) - 0.001f;
-  const RayConsts pk = make_ray_consts(dx, dy, dz, w.mx, w.my, w.mz);
+  float d[3], e[3], inv[3];
+  primary_ray(v, (float)w.dim, px, py, d, e, inv);
+  const float ex = e[0], ey = e[1], ez = e[2];
+  const RayConsts pk = ray_consts(d, inv, w.mx, w.my, w.mz);
   if (!L::kClear && !line_meets_reach(w, ex, ey, ez, pk)) {
     // this ray cannot reach a nonempty voxel: a miss, no steps (launches
     // whose step counts are observed pass a reach every line meets; the
@@ -710,12 +704,12 @@ __device__ __forceinline__ void trace_pixel_dense(const DenseWorld& w, const Vie
     }
     ssteps = h.steps;
     if constexpr (kShade == kShadeRef) {
-      store_hit_shadow_ref(v, sc, out, px, py, data, info0, psteps, shit, shx, shy, shz, sox, soy,
+      store_hit_shadow_ref<kStats>(v, sc, out, px, py, data, info0, psteps, shit, shx, shy, shz, sox, soy,
                            soz, ssteps, cnt);
       return;
     }
   }
-  write_pixel<kShade>(v, sc, out, px, py, p, shit, shx, shy, shz, sox, soy, soz, ssteps, cnt, &w,
+  write_pixel<kShade, kStats>(v, sc, out, px, py, p, shit, shx, shy, shz, sox, soy, soz, ssteps, cnt, &w,
                      gacc);
 }
 

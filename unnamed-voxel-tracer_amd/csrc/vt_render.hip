@@ -80,20 +80,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kClear ? 5 
   const bool active = px < v.W && py < v.H;
   Counters cnt = {0, 0, 0, 0, 0, 0, 0, 0};
   if (active) {
-    float dx, dy, dz;
-    raygen(v, px, py, dx, dy, dz);
-    float tn, tf;
-    const float D = (float)w.dim;
-    intersect_aabb(v.pos[0], v.pos[1], v.pos[2], dx, dy, dz, 0.0f, 0.0f, 0.0f, D, D, D, tn, tf);
-    float tc = fmaxf(tn, 0.0f);
-    float ex = (v.pos[0] + dx * tc) - 0.001f;
-    float ey = (v.pos[1] + dy * tc) - 0.001f;
-    float ez = (v.pos[2] + dz * tc) - 0.001f;
+    float d[3], e[3], inv[3];
+    primary_ray(v, (float)w.dim, px, py, d, e, inv);
     GeneralHit g;
     if (!kStats && w.occ)
-      trace_brickmap_fast<false, kClear, false>(w, ex, ey, ez, dx, dy, dz, sc.max_primary, g);
+      trace_brickmap_fast<false, kClear, false>(w, e[0], e[1], e[2], d[0], d[1], d[2], inv,
+                                                sc.max_primary, g);
     else
-      trace_general<kStats>(w, ex, ey, ez, dx, dy, dz, sc.max_primary, g, cnt.l1f, cnt.l0f);
+      trace_general<kStats>(w, e[0], e[1], e[2], d[0], d[1], d[2], sc.max_primary, g, cnt.l1f,
+                            cnt.l0f);
     Primary p;
     p.hit = g.data != 0u;
     p.steps = g.steps;
@@ -119,10 +114,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kClear ? 5 
         // the sun is the same for every lane: a uniform branch
         if (sc.sun[0] >= 0.0f && sc.sun[1] >= 0.0f && sc.sun[2] >= 0.0f)
           trace_brickmap_fast<true, kClear, true>(w, sox, soy, soz, sc.sun[0], sc.sun[1],
-                                                  sc.sun[2], sc.max_shadow, s);
+                                                  sc.sun[2], sc.shadow.inv, sc.max_shadow, s);
         else
           trace_brickmap_fast<false, kClear, true>(w, sox, soy, soz, sc.sun[0], sc.sun[1],
-                                                   sc.sun[2], sc.max_shadow, s);
+                                                   sc.sun[2], sc.shadow.inv, sc.max_shadow, s);
       } else {
         trace_general<kStats>(w, sox, soy, soz, sc.sun[0], sc.sun[1], sc.sun[2], sc.max_shadow,
                               s, cnt.l1f, cnt.l0f);
@@ -134,12 +129,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kClear ? 5 
         shz = s.hz;
       }
       ssteps = s.steps;
-      store_hit_shadow_ref(v, sc, out, px, py, data, info0, psteps, shit, shx, shy, shz, sox, soy,
+      store_hit_shadow_ref<kStats>(v, sc, out, px, py, data, info0, psteps, shit, shx, shy, shz, sox, soy,
                            soz, ssteps, cnt);
     }
     if (!p.hit) {  // a hit's stores are made above
       GradAcc gacc = grad_acc();
-      write_pixel<kShadeRef>(v, sc, out, px, py, p, shit, shx, shy, shz, sox, soy, soz, ssteps,
+      write_pixel<kShadeRef, kStats>(v, sc, out, px, py, p, shit, shx, shy, shz, sox, soy, soz, ssteps,
                              cnt, nullptr, gacc);
     }
   }
