@@ -28,11 +28,16 @@ namespace vt {
 // (spills), 295 at five -- without it seven (72 VGPRs, no spills).
 constexpr int kClearWaves = 6;
 constexpr int kPlainWaves = 7;
+// Launches without the clearance map of at most five waves per SIMD (96 VGPRs
+// hold the iteration in flight) run ahead (dense_skip_ahead): all their waves
+// are resident at once.
+constexpr int kAheadWaves = 5;
 // kSched: the launch order comes from the frame's tile schedule (`sched`);
 // the kernels without it carry none of its code.
 template <class L, bool kStats, int kShade, bool kSched>
 __global__ __launch_bounds__(256)
-__attribute__((amdgpu_waves_per_eu(L::kClear ? kClearWaves : kPlainWaves))) void k_render_dense(
+__attribute__((amdgpu_waves_per_eu(L::kClear ? kClearWaves : (L::kAhead ? kAheadWaves : kPlainWaves))))
+void k_render_dense(
     DenseWorld w, ViewConsts v, ShadeConsts sc, FrameOut out, uint32_t* sched, uint32_t log2_tw,
     uint32_t blocks_x) {
   __shared__ SchedBlock sb;
@@ -173,7 +178,8 @@ static void launch_dense_shade(const DenseWorld& w, const ViewConsts& v, const S
 template <bool kSched>
 static void launch_dense_select(const DenseWorld& w, uint32_t traversal, const ViewConsts& v,
                                 const ShadeConsts& sc, const FrameOut& out, uint32_t* sd,
-                                uint32_t lw, uint32_t blocks_x, dim3 grid, hipStream_t stream) {
+                                uint32_t lw, uint32_t blocks_x, dim3 grid, uint32_t compute_units,
+                                hipStream_t stream) {
   const bool stats = out.stats != nullptr;
   if (traversal == VT_TRAVERSAL_BITMASK) {
     if (stats)
@@ -193,6 +199,8 @@ static void launch_dense_select(const DenseWorld& w, uint32_t traversal, const V
       launch_dense_shade<FlatLookup, true, kSched>(w, v, sc, out, sd, lw, blocks_x, grid, stream);
     else if (w.clear_bytes)
       launch_dense_shade<FlatLookupClear, false, kSched>(w, v, sc, out, sd, lw, blocks_x, grid, stream);
+    else if (grid.x <= kAheadWaves * compute_units)
+      launch_dense_shade<FlatLookupAhead, false, kSched>(w, v, sc, out, sd, lw, blocks_x, grid, stream);
     else if (long_caps)
       launch_dense_shade<FlatLookupLong, false, kSched>(w, v, sc, out, sd, lw, blocks_x, grid, stream);
     else
@@ -212,7 +220,6 @@ static bool sched_taken(const uint32_t* schedule, const ShadeConsts& sc) {
 hipError_t launch_render_dense(const DenseWorld& w_in, uint32_t traversal, const ViewConsts& v,
                                const ShadeConsts& sc_in, const FrameOut& out, uint32_t* schedule,
                                TileShape tile, uint32_t compute_units, hipStream_t stream) {
-  (void)compute_units;
   DenseWorld w = w_in;
   // Where step counts are observed (stored, or counted as traceMap's by
   // statistics without the clearance map) no ray ends early, at the reach box
@@ -227,10 +234,10 @@ hipError_t launch_render_dense(const DenseWorld& w_in, uint32_t traversal, const
   const dim3 grid(nblocks);
   if (sched_taken(schedule, sc))
     launch_dense_select<true>(w, traversal, v, sc, out, schedule, tile.log2_w, blocks_x, grid,
-                              stream);
+                              compute_units, stream);
   else
     launch_dense_select<false>(w, traversal, v, sc, out, nullptr, tile.log2_w, blocks_x, grid,
-                               stream);
+                               compute_units, stream);
   return hipGetLastError();
 }
 

@@ -369,6 +369,7 @@ struct FlatLookup {
   // one byte gather per probe; returns the material (0 = empty)
   static constexpr bool kPrefetch = true;  // probes have no state: run ahead
   static constexpr bool kClear = false;    // no clearance map
+  static constexpr bool kAhead = false;    // no iteration ahead
   static constexpr int kSkip = kSkipShort;  // empty-space iteration length
   __device__ __forceinline__ void reset() {}
   template <bool kStats>
@@ -397,6 +398,7 @@ struct BitmaskLookupT {
   static_assert(kBrick == 4 || kBrick == 8, "4^3 or 8^3 bricks");
   static constexpr bool kPrefetch = false;
   static constexpr bool kClear = false;
+  static constexpr bool kAhead = false;
   static constexpr int kSkip = kSkipShort;  // (the plain loop has no empty-space phase)
   static constexpr uint32_t kBrickShift = kBrick == 8 ? 9u : 6u;  // log2 codes per brick
   uint32_t brick, region, leaf;
@@ -456,6 +458,12 @@ struct FlatLookupClear : FlatLookup {
 // iteration, no clearance map.
 struct FlatLookupLong : FlatLookup {
   static constexpr int kSkip = kSkipLong;
+};
+
+// For launches whose waves are all resident at once (dense_skip_ahead).
+struct FlatLookupAhead : FlatLookup {
+  static constexpr int kSkip = kSkipLong;
+  static constexpr bool kAhead = true;
 };
 
 // Result of one traceMap call in a dense world.
@@ -1303,6 +1311,163 @@ __device__ __forceinline__ int dense_skip_positive(float dx, float dy, float dz,
   return status;
 }
 
+// The two rules of an iteration for dense_skip_ahead: any direction
+// (SkipGeneral, dense_skip_empty's) and directions positive on every axis
+// (SkipPositive, dense_skip_positive's).
+struct SkipState {
+  float wx, wy, wz;
+  uint32_t c;
+};
+
+template <int K>
+struct SkipGeneral {
+  float Px, Py, Pz, Ax, Ay, Az, dx, dy, dz, ix, iy, iz;
+  uint32_t mx, my, mz, flip;
+  __amdgpu_buffer_rsrc_t bytes;
+  // The K steps from a: the state b after them; probe(i, address) for each.
+  template <class P>
+  __device__ __forceinline__ void run(const SkipState& a, SkipState& b, bool& tie,
+                                      P probe) const {
+    float wx = a.wx, wy = a.wy, wz = a.wz;
+    uint32_t c = a.c;
+    float mn = 1.0f;  // smallest crossing time of the steps from S_1 .. S_K-1
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      const float tm = dense_advance(Px, Py, Pz, Ax, Ay, Az, dx, dy, dz, ix, iy, iz, mx, my, mz,
+                                     wx, wy, wz, c);
+      if (i > 0) mn = fminf(mn, tm);
+      probe(i, c ^ flip);
+    }
+    tie = (mn <= 0.0f) | (fmaxf(fmaxf(wx, wy), wz) >= 8.0f);
+    b.wx = wx;
+    b.wy = wy;
+    b.wz = wz;
+    b.c = c;
+  }
+  // Whether the iteration from a to b ends the phase; any = its bytes or-ed.
+  __device__ __forceinline__ bool stops(const SkipState& a, const SkipState& b, bool tie,
+                                        uint32_t any) const {
+    if (tie) {  // the same steps again, with the corrected lookups
+      DenseCell n;
+      n.wx = a.wx;
+      n.wy = a.wy;
+      n.wz = a.wz;
+      n.c = a.c;
+      any = 0u;
+#pragma unroll 1
+      for (int i = 0; i < K; ++i) {
+        n = dense_step(Px, Py, Pz, Ax, Ay, Az, dx, dy, dz, ix, iy, iz, mx, my, mz, flip, n);
+        any |= (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(bytes, (int)n.a, 0, 0);
+      }
+    }
+    return dense_left_grid(a.c, b.c, mx, my, mz) | (any != 0u);
+  }
+};
+
+template <int K>
+struct SkipPositive {
+  float dx, dy, dz, ix, iy, iz;
+  uint32_t mx, my, mz;
+  __amdgpu_buffer_rsrc_t bytes;
+  template <class P>
+  __device__ __forceinline__ void run(const SkipState& a, SkipState& b, bool& tie,
+                                      P probe) const {
+    float wx = a.wx, wy = a.wy, wz = a.wz;
+    uint32_t c = a.c;
+    float med = 1.0f;  // smallest median crossing time of the iteration
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+      // the step from S_i (S_0 is the iteration's start, already probed)
+      const float tx = (8.0f - wx) * ix;
+      const float ty = (8.0f - wy) * iy;
+      const float tz = (8.0f - wz) * iz;
+      const float tm = fminf(fminf(tx, ty), tz);
+      const StepAxis ax = step_axis(ty, tz, tm);
+      const float nwx = wx + dx * tm;
+      const float nwy = wy + dy * tm;
+      const float nwz = wz + dz * tm;
+      wx = ax.yz ? nwx : 0.0f;
+      wy = ax.y ? 0.0f : nwy;
+      wz = ax.z ? 0.0f : nwz;
+      const uint32_t cn = morton_step(c, ax.z ? mz : (ax.y ? my : mx));
+      if (i > 0) {  // the lookup of S_i
+        probe(i - 1, tm <= 0.0f ? cn : c);
+        med = fminf(med, __builtin_amdgcn_fmed3f(tx, ty, tz));
+      }
+      c = cn;
+    }
+    uint32_t q = c;
+    if (fmaxf(fmaxf(wx, wy), wz) >= 8.0f) {  // the lookup of S_K
+      if (wx >= 8.0f) q = morton_inc_or_out(q, mx);
+      if (wy >= 8.0f) q = morton_inc_or_out(q, my);
+      if (wz >= 8.0f) q = morton_inc_or_out(q, mz);
+    }
+    probe(K - 1, q);
+    tie = med <= 0.0f;
+    b.wx = wx;
+    b.wy = wy;
+    b.wz = wz;
+    b.c = c;
+  }
+  __device__ __forceinline__ bool stops(const SkipState& a, const SkipState& b, bool tie,
+                                        uint32_t any) const {
+    return tie | dense_left_grid(a.c, b.c, mx, my, mz) | (any != 0u);
+  }
+};
+
+// The empty-space phase without the clearance map, an iteration ahead: the
+// steps of iteration i + 1 are taken while the bytes of iteration i are on
+// their way, and thrown away when those end the phase.  Same contract as
+// dense_skip_empty.  For launches whose waves are all resident at once
+// (launch_dense_select): they last as long as their longest wave, which runs
+// alone on its SIMD towards the end, and there the wait for an iteration's
+// bytes cost as much as its steps.  16 frames of 128x128 of a 256^3 height
+// field 1047 -> 851 us, of 512x512 with their backward 1257 -> 1162.  A full
+// chip loses what is thrown away: the same world at 1080p 44.2 -> 47.2 us, a
+// batch of 32 views 1060 -> 1140.
+template <int K, class It>
+__device__ __forceinline__ void dense_skip_ahead(const It& it, DenseCell& s, int& steps,
+                                                 int limit) {
+  int sb = steps;
+  if (sb + K >= limit) return;
+  SkipState x, y, z;
+  x.wx = s.wx;
+  x.wy = s.wy;
+  x.wz = s.wz;
+  x.c = s.c;
+  uint32_t p[K], v[K];
+  bool ty, tz;
+  it.run(x, y, ty, [&](int i, uint32_t a) {
+    v[i] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(it.bytes, (int)a, 0, 0);
+  });
+  for (;;) {
+    it.run(y, z, tz, [&](int i, uint32_t a) { p[i] = a; });
+    uint32_t any = 0u;
+#pragma unroll
+    for (int i = 0; i < K; ++i) any |= v[i];
+    // The next requests only after this iteration's bytes have arrived (the
+    // asm orders them): on every path to the loop's head just these K are in
+    // flight, into the registers the last K left, so nothing waits for them
+    // before the `or` above.
+#pragma unroll
+    for (int i = 0; i < K; ++i) asm volatile("" : "+v"(any), "+v"(p[i]));
+#pragma unroll
+    for (int i = 0; i < K; ++i)
+      v[i] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b8(it.bytes, (int)p[i], 0, 0);
+    if (it.stops(x, y, ty, any)) break;
+    x = y;
+    y = z;
+    ty = tz;
+    sb += K;
+    if (sb + K >= limit) break;
+  }
+  s.wx = x.wx;
+  s.wy = x.wy;
+  s.wz = x.wz;
+  s.c = x.c;
+  steps = sb;
+}
+
 // The flat lookup's traversal from r's block-level state: the empty-space
 // phase, then the exact loop to the ray's end.
 // kShadow: the ray starts next to a nonempty voxel.  kPositive: the caller
@@ -1364,6 +1529,9 @@ __device__ __forceinline__ void dense_run_prefetch(DenseRay& r, L& lk, const Den
       h.steps = min(steps0, max_steps);
       return;
     }
+  } else if constexpr (kPositive && L::kAhead) {
+    const SkipPositive<L::kSkip> it = {r.dx, r.dy, r.dz, r.ix, r.iy, r.iz, mx, my, mz, vox};
+    dense_skip_ahead<L::kSkip>(it, s0, steps0, limit);
   } else if constexpr (kPositive) {
     dense_skip_positive<L::kSkip, false>(r.dx, r.dy, r.dz, r.ix, r.iy, r.iz, mx, my, mz, s0,
                                          steps0, limit, vox, vox, false);
@@ -1374,9 +1542,15 @@ __device__ __forceinline__ void dense_run_prefetch(DenseRay& r, L& lk, const Den
       dense_skip_blind<L::kSkip>(r.Px, r.Py, r.Pz, r.Ax, r.Ay, r.Az, r.dx, r.dy, r.dz, r.ix,
                                  r.iy, r.iz, mx, my, mz, s0, steps0,
                                  min(r.blind, max_steps - 1));
-    dense_skip_empty<L::kSkip, false>(r.Px, r.Py, r.Pz, r.Ax, r.Ay, r.Az, r.dx, r.dy, r.dz, r.ix,
-                                      r.iy, r.iz, mx, my, mz, flip, s0, steps0, limit, vox, vox,
-                                      0u, false);
+    if constexpr (L::kAhead) {
+      const SkipGeneral<L::kSkip> it = {r.Px, r.Py, r.Pz, r.Ax, r.Ay, r.Az, r.dx, r.dy, r.dz,
+                                        r.ix, r.iy, r.iz, mx,   my,   mz,   flip, vox};
+      dense_skip_ahead<L::kSkip>(it, s0, steps0, limit);
+    } else {
+      dense_skip_empty<L::kSkip, false>(r.Px, r.Py, r.Pz, r.Ax, r.Ay, r.Az, r.dx, r.dy, r.dz, r.ix,
+                                        r.iy, r.iz, mx, my, mz, flip, s0, steps0, limit, vox, vox,
+                                        0u, false);
+    }
   }
   float fwx, fwy, fwz;
   uint32_t fc, fM, fa, fv;
