@@ -268,8 +268,7 @@ ShadeConsts shade_consts(const vt_render_params& p) {
   sc.illum_lit = unorm ? unorm8(0.3f) : 0.3f;
   sc.illum_occ = unorm ? unorm8(-0.3f) : -0.3f;
   const float li = len3(sc.illum[0], sc.illum[1], sc.illum[2]);
-  sky_dome(sc.sun_n, sc.illum[0] / li, sc.illum[1] / li, sc.illum[2] / li, sc.illum[1], sc.sky[0],
-           sc.sky[1], sc.sky[2]);
+  sc.sky = sky_base(sc.sun_n, sc.illum[0] / li, sc.illum[1] / li, sc.illum[2] / li, sc.illum[1]);
   sc.max_primary = p.max_steps_primary;
   sc.max_shadow = p.max_steps_shadow;
   sc.flags = p.flags;

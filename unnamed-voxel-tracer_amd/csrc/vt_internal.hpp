@@ -113,7 +113,7 @@ struct ShadeConsts {
   float sun_n[3], sun_len;     // sun / |sun| and |sun|
   float illum[3];              // illumination.xyz, through rgba8 if the G-buffer is
   float illum_lit, illum_occ;  // illumination.w
-  float sky[3];                // the sky's colour along illumination.xyz
+  SkyBase sky;                 // of the sky along illumination.xyz
   bool cull_entities;          // may_meet_entities holds for the sun
   int max_primary, max_shadow;
   uint32_t flags;

@@ -487,8 +487,10 @@ __device__ __forceinline__ void store_ref_composite(const ViewConsts& v, const S
                                                     bool hit) {
   float4 s;
   if (hit) {
-    s = make_float4(col.x + ill.w * sc.sky[0], col.y + ill.w * sc.sky[1],
-                    col.z + ill.w * sc.sky[2], col.w + ill.w * 1.0f);
+    float r, g, b;
+    sky_glow(sc.sky, r, g, b);
+    s = make_float4(col.x + ill.w * r, col.y + ill.w * g, col.z + ill.w * b,
+                    col.w + ill.w * 1.0f);
   } else {
     s = col;
   }

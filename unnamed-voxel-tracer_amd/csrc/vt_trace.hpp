@@ -45,10 +45,10 @@ __device__ __forceinline__ int f2i_sat(float x) {
 // size (divisible) and quotients in the normal range; 0 / x keeps its sign.
 // What a pixel costs besides its rays' steps came to 900 instructions of the
 // 2600-6600 a wave takes; with the shared quotients, the constants of a
-// launch's hits in ShadeConsts, may_meet_entities and sky_dome's products it
-// is a third of that (six views at 1080p 272 -> 248 us, a 333x187 frame with
-// its G-buffer 30.8 -> 21.6, the engine's 720p frame 134 -> 120, a batch of 64
-// views 2180 -> 1960).
+// launch's hits in ShadeConsts, may_meet_entities and sky_base it
+// is under half of that (six views at 1080p 272 -> 252 us, a 333x187 frame with
+// its G-buffer 30.8 -> 22.3, the engine's 720p frame 134 -> 122, a batch of 64
+// views 2180 -> 1970).
 __device__ __forceinline__ double recip64(float x) {
   const double d = (double)x, y = (double)__builtin_amdgcn_rcpf(x);
   const double e = fma(-d, y, 1.0);
@@ -254,24 +254,38 @@ __device__ __forceinline__ bool trace_entities(float ox, float oy, float oz, flo
   return id >= 0;  // the re-test on map.glsl:199-200 repeats a test that passed
 }
 
-// SkyDome2 (camera.glsl:11-19) along a ray whose normalised direction is rn,
-// sun_n the normalised sun.  The powers are products in binary64, rounded
-// once.
-__host__ __device__ inline void sky_dome(const float* sun_n, float rnx, float rny, float rnz,
-                                         float ry, float& r, float& g, float& b) {
+// SkyDome2 (camera.glsl:11-19) in two halves.  The clamped cosine between the
+// normalised sun and the normalised ray, and the colour before the sun's
+// glow, are the same for every hit of a launch, and made on the host (each
+// operation rounded as on the device); the powers are taken on the device,
+// whose pow the colour bytes have always been rounded from.
+struct SkyBase {
+  float sv;       // clamp(dot(sun, ray), 0, 1.2)
+  float r, g, b;  // colour without the glow
+};
+__host__ __device__ inline SkyBase sky_base(const float* sun_n, float rnx, float rny, float rnz,
+                                            float ry) {
+  SkyBase s;
   float dt = sun_n[0] * rnx;
   dt = dt + sun_n[1] * rny;
   dt = dt + sun_n[2] * rnz;
-  const float sv = fminf(fmaxf(dt, 0.0f), 1.2f);
-  const double s1 = (double)sv, s2 = s1 * s1, s4 = s2 * s2;
-  const float p8 = (float)(s4 * s4), p3 = (float)(s2 * s1);
-  float k = ry * 0.2f;
-  r = ((0.6f - k * 1.0f) + 0.075f);
-  g = ((0.71f - k * 0.5f) + 0.075f);
-  b = ((0.75f - k * 1.0f) + 0.075f);
-  r = r + (0.4f * 1.0f) * p8;
-  g = g + (0.4f * 0.6f) * p8;
-  b = b + (0.4f * 0.1f) * p8;
+  s.sv = fminf(fmaxf(dt, 0.0f), 1.2f);
+  const float k = ry * 0.2f;
+  s.r = ((0.6f - k * 1.0f) + 0.075f);
+  s.g = ((0.71f - k * 0.5f) + 0.075f);
+  s.b = ((0.75f - k * 1.0f) + 0.075f);
+  return s;
+}
+// pow(0, y) = 0 exactly: the sky away from the sun needs no powers.
+__device__ __forceinline__ void sky_glow(const SkyBase& s, float& r, float& g, float& b) {
+  float p8 = s.sv, p3 = s.sv;
+  if (s.sv != 0.0f) {
+    p8 = powf(s.sv, 8.0f);
+    p3 = powf(s.sv, 3.0f);
+  }
+  r = s.r + (0.4f * 1.0f) * p8;
+  g = s.g + (0.4f * 0.6f) * p8;
+  b = s.b + (0.4f * 0.1f) * p8;
   r = r + 0.2f * p3;
   g = g + 0.08f * p3;
   b = b + 0.04f * p3;
@@ -291,7 +305,7 @@ __device__ __forceinline__ void sky(const float* sun_n, float rx, float ry, floa
     ny = ry / lr;
     nz = rz / lr;
   }
-  sky_dome(sun_n, nx, ny, nz, ry, r, g, b);
+  sky_glow(sky_base(sun_n, nx, ny, nz, ry), r, g, b);
 }
 
 // ---------------------------------------------------------------------------
