@@ -56,6 +56,7 @@ void free_world(vt_world* w) {
   dev_free(w->pool);
   dev_free(w->atlas);
   dev_free(w->occ);
+  dev_free(w->masks);
   dev_free(w->brick_bits);
   dev_free(w->freemap);
   dev_free(w->clear);
@@ -150,6 +151,7 @@ BrickmapWorld brickmap_view(const vt_world* w) {
   b.atlas = w->atlas;
   b.dim = w->dim;
   b.occ = w->occ;
+  b.masks = w->masks;
   b.nvox = w->dim * w->dim * w->dim;
   uint32_t bits = 0;
   while ((1u << bits) < w->dim) bits++;
@@ -508,6 +510,7 @@ int vt_world_create_brickmap(vt_ctx* ctx, uint32_t dim, const uint32_t* chunks,
   if ((dim & (dim - 1)) == 0) {  // power-of-two map: occupancy bytes for the fast loop
     const size_t n = (size_t)dim * dim * dim;
     if ((st = dev_alloc(w, (void**)&w->occ, n, "block occupancy")) != VT_OK ||
+        (st = dev_alloc(w, (void**)&w->masks, vt::kAtlasMaskWords * 8, "model masks")) != VT_OK ||
         (st = dev_alloc(w, (void**)&w->brick_bits, (size_t)vt::brick_bit_words(dim) * 8,
                         "block brick bits")) != VT_OK ||
         (st = alloc_maps(w)) != VT_OK) {
@@ -516,6 +519,7 @@ int vt_world_create_brickmap(vt_ctx* ctx, uint32_t dim, const uint32_t* chunks,
     }
     e = vt::launch_build_occupancy(vt::brickmap_view(w), w->occ, w->brick_bits, w->clear_tmp,
                                    nullptr);
+    if (e == hipSuccess) e = vt::launch_atlas_masks(w->atlas, w->masks, nullptr);
     if (e == hipSuccess) e = vt::rebuild_maps(w, nullptr);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess) {

@@ -69,6 +69,7 @@ struct vt_world {
   size_t pool_capacity;  // words the device pool holds
   uint32_t* chunk_mirror;  // host copy of the chunk table (edit allocation)
   uint8_t* occ;            // block occupancy in Morton order (power-of-two dim)
+  uint64_t* masks;         // texel masks of the atlas's models (with occ)
   uint64_t* brick_bits;    // brickmap: bit per 4^3 brick of blocks, from occ
   // free-region map (dense worlds and power-of-two brickmap worlds)
   uint32_t* freemap;       // 8 octants x free_words_per_octant(dim) words, then a
@@ -187,6 +188,9 @@ hipError_t launch_render_brickmap(const BrickmapWorld& w, const ViewConsts& v,
 // bits of those layers' 4^3 bricks (bits of a partly covered word are set
 // only, never cleared: the other layers' bits must be right already).
 // sub (may be null): the clearance map's byte of each of those bricks.
+// The texel masks of all 32^3 models of an atlas (BrickmapWorld::masks).
+constexpr size_t kAtlasMaskWords = 32768u * 8u;
+hipError_t launch_atlas_masks(const uint32_t* atlas, uint64_t* masks, hipStream_t stream);
 hipError_t launch_build_occupancy(const BrickmapWorld& w, uint8_t* occ, uint64_t* brick_bits,
                                   uint8_t* sub, hipStream_t stream, uint32_t y_end = 0);
 // Grows a brickmap world's block pool to at least `blocks` blocks by

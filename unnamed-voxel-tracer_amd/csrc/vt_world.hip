@@ -667,6 +667,31 @@ bool use_clear_map(const vt_world* w, uint32_t flags) {
   return (flags & VT_FLAG_FREE_MAP_ON) || w->near_frac <= kClearNearShare;
 }
 
+// The texel masks of an atlas: a thread makes one word (layer z of a model)
+// from 64 texels, lanes along x, so that a wave reads whole rows of the atlas
+// (64 MiB once: 16 us).
+__global__ __launch_bounds__(256) void k_atlas_masks(const uint4* __restrict__ atlas,
+                                                     uint64_t* __restrict__ masks) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  const uint32_t mx = i & 31u, z = (i >> 5) & 7u, my = (i >> 8) & 31u, mz = i >> 13;
+  uint64_t m = 0u;
+#pragma unroll
+  for (uint32_t y = 0; y < 8u; ++y) {
+    const uint4* row = atlas + (((mz * 8u + z) * 256u + my * 8u + y) * 256u + mx * 8u) / 4u;
+    const uint4 a = row[0], b = row[1];
+    const uint32_t t[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (uint32_t x = 0; x < 8u; ++x) m |= (uint64_t)(t[x] != 0u) << (x + 8u * y);
+  }
+  masks[(mx + 32u * (my + 32u * mz)) * 8u + z] = m;
+}
+
+hipError_t launch_atlas_masks(const uint32_t* atlas, uint64_t* masks, hipStream_t stream) {
+  hipLaunchKernelGGL(k_atlas_masks, dim3((uint32_t)(kAtlasMaskWords / 256)), dim3(256), 0, stream,
+                     reinterpret_cast<const uint4*>(atlas), masks);
+  return hipGetLastError();
+}
+
 // One thread per 4^3 brick of the layers y < 4 ny: a brick lies in one chunk,
 // so one chunk-table read and 16 rows of 4 pool words make its 64 occupancy
 // bytes (Morton order).  A whole 512^3 map, mostly empty chunks: 384 us as
