@@ -390,8 +390,9 @@ __device__ __forceinline__ void flush_albedo(const ShadeConsts& sc, GradAcc& acc
 // block's waves in LDS, then one atomic per quantity and block.  Float
 // atomics on one address serialise in the memory system, so they are kept
 // to a few thousand per launch.  Every thread of the block must call this.
+template <uint32_t kWaves = 4u>
 __device__ __forceinline__ void flush_grad(const ShadeConsts& sc, const GradAcc& acc) {
-  __shared__ float part[4][4];  // [quantity][wave], 256-thread blocks
+  __shared__ float part[4][kWaves];  // [quantity][wave]
   const float v[4] = {wave_sum_f(acc.loss), wave_sum_f(acc.sx), wave_sum_f(acc.sy),
                       wave_sum_f(acc.sz)};
   const uint32_t wave = threadIdx.x >> 6;
@@ -402,7 +403,10 @@ __device__ __forceinline__ void flush_grad(const ShadeConsts& sc, const GradAcc&
   __syncthreads();
   if (threadIdx.x < 4u) {
     const uint32_t q = threadIdx.x;
-    const float t = (part[q][0] + part[q][1]) + (part[q][2] + part[q][3]);
+    float t = 0.0f;
+#pragma unroll
+    for (uint32_t k = 0; k < kWaves; k += 4u)
+      t += (part[q][k] + part[q][k + 1]) + (part[q][k + 2] + part[q][k + 3]);
     float* dst = q == 0u ? sc.loss : (sc.grad_sun ? sc.grad_sun + (q - 1u) : nullptr);
     if (dst) atomicAdd(dst, t);
   }
