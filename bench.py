@@ -64,9 +64,9 @@ def counted_stats(vt, torch, ctx, world, jobs, free):
     """Statistics summed over views, jobs = [(camera, W, H, params maker)]
     where params maker(flags) returns the view's params.  free=False:
     traceMap's steps (the statistics kernel variant); free=True: the steps
-    the free-region kernel executes (VT_FLAG_FREE_MAP_ON: a ray ends where
-    nothing is left to hit), the work the timed kernel does when it takes
-    the test."""
+    the clearance map's kernel executes (VT_FLAG_FREE_MAP_ON: a ray ends
+    where nothing is left to hit), the work the timed kernel does when it
+    reads the map."""
     stats = torch.zeros(8, dtype=torch.int64, device="cuda")
     for cam, W, H, mk in jobs:
         f = vt.Frame.alloc(W, H, shaded=False)
@@ -216,7 +216,7 @@ def bench_batched(args):
         },
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 5),
-                     # counters of the flat free-region batch kernel (the tuning picked here)
+                     # counters of the flat batch kernel with the clearance map (the tuning picked here)
                      "traffic": measured_traffic(bkey) if bkey else None,
                      "issue": measured_issue(bkey, ms) if bkey else None},
         "cpu_baseline": None,

@@ -9,7 +9,8 @@
 // chunks are allocated on first touch in edit order (pool block index =
 // allocation count, voxel.zig:47-56), and of several edits of one voxel the
 // last wins.  The host resolves that order (chunk allocation, last-writer
-// dedup) and the device applies the surviving writes in one scatter:
+// dedup) and the device applies the surviving writes in one kernel that reads
+// them from page-locked host memory:
 //   brickmap: pool words and new chunk-table entries; the pool grows by
 //             doubling like GpuBlockAllocator.alloc (gpu_block_allocator.zig:
 //             20-30), new blocks zero;
