@@ -221,16 +221,12 @@ hipError_t launch_build_l1b(const uint64_t* l0, uint64_t n0, const uint32_t* wor
 // reports whether it was and the free regions of each octant.
 uint32_t free_regions(uint32_t dim);
 uint32_t free_words_per_octant(uint32_t dim);
-hipError_t launch_build_freemap(const uint64_t* l1, uint32_t dim, uint32_t* fm,
-                                const uint32_t* changed, CtxReport* report, hipStream_t stream);
 // Clearance map (ClearMap in vt_trace.hpp): 2 x 8 octant planes of
 // clear_cells(dim) bytes, built from one byte per 4^3 brick (a bit per 2^3
 // sub-block) at the start of tmp, unless *changed (device, may be null) is 0;
 // reports the near cells.
 uint32_t clear_cells(uint32_t dim);
 size_t clear_tmp_bytes(uint32_t dim);
-hipError_t launch_build_clear(uint8_t* tmp, uint32_t dim, uint8_t* map, const uint32_t* changed,
-                              CtxReport* report, hipStream_t stream);
 // Whether launches with these flags use the clearance map: it is valid and
 // VT_FLAG_FREE_MAP_ON, or neither FREE_MAP flag and a world open enough for
 // it to pay.

@@ -948,7 +948,7 @@ enum SkipStatus : int {
   kSkipOpen = 3,     // the wave's rays stand clear of everything: clear_advance
 };
 
-// ---- ClearMap: the clearance map (built by launch_build_clear) ----
+// ---- ClearMap: the clearance map (built by k_maps_first, k_clear_planes and k_clear_cubes) ----
 // Cells of 8^3 blocks, R = dim / 8 per axis.  A cell is near when the cell
 // widened by 2 blocks a side holds a nonempty block.  For each direction
 // octant (bit k = travelling negatively on axis k) the byte of a cell is the

@@ -283,8 +283,10 @@ hipError_t launch_build_dense(const uint8_t* linear, uint32_t dim, uint8_t* vox,
 // each of the 8 direction octants o, free_o(r) = no region r' at or ahead of
 // r on every axis in o's travel direction (the forward orthant, r itself
 // included) holds a nonempty block.  Bit r (region Morton code) of octant
-// o's bitmap is free_o(r).  The traversal loops read it to end a ray that can
-// hit nothing more.
+// o's bitmap is free_o(r).  vt_free_map_used decides by its largest share.
+
+// Threads of a block of the maps' first launch.
+constexpr uint32_t kMapBlock = 1024;
 
 // One block per octant, the regions as bit rows along x in LDS (R = 1 << lg,
 // at most 64 rows of 64 bits a layer, 32 KiB).  A row's bit x becomes the OR
@@ -294,15 +296,22 @@ hipError_t launch_build_dense(const uint8_t* linear, uint32_t dim, uint8_t* vox,
 // has: 16 us at 512^3 (five kernels over byte planes: 36).  An edit rarely
 // empties or fills a whole region, so it passes `changed` (device word: a
 // region did) and the launch ends at once, in 3 us, when none did.
-__global__ __launch_bounds__(1024) void k_free_map(const uint64_t* __restrict__ l1, uint32_t lg,
-                                                   uint32_t words, uint32_t* __restrict__ fm,
-                                                   const uint32_t* __restrict__ changed,
-                                                   CtxReport* __restrict__ report) {
-  const bool run = !changed || *changed != 0u;
+struct FreeMapArgs {
+  const uint64_t* l1;
+  uint32_t lg, words;
+  uint32_t* fm;
+  const uint32_t* changed;
+  CtxReport* report;
+};
+__device__ __forceinline__ void free_map_block(const FreeMapArgs& a, uint64_t* row,
+                                               uint32_t& total) {
+  const uint64_t* __restrict__ l1 = a.l1;
+  const uint32_t lg = a.lg, words = a.words;
+  uint32_t* __restrict__ fm = a.fm;
+  CtxReport* __restrict__ report = a.report;
+  const bool run = !a.changed || *a.changed != 0u;
   if (blockIdx.x == 0u && threadIdx.x == 0u) report->free_built = run ? 1u : 0u;
   if (!run) return;  // the same for every thread
-  __shared__ uint64_t row[4096];
-  __shared__ uint32_t total;
   const uint32_t R = 1u << lg, rows = R << lg, n = rows << lg;
   const uint32_t o = blockIdx.x, t = threadIdx.x;
   if (t == 0u) total = 0u;
@@ -394,15 +403,6 @@ uint32_t free_words_per_octant(uint32_t dim) {
   return (R * R * R + 31u) / 32u;
 }
 
-hipError_t launch_build_freemap(const uint64_t* l1, uint32_t dim, uint32_t* fm,
-                                const uint32_t* changed, CtxReport* report, hipStream_t stream) {
-  uint32_t lg = 0;
-  while ((1u << lg) < free_regions(dim)) lg++;
-  hipLaunchKernelGGL(k_free_map, dim3(8), dim3(1024), 0, stream, l1, lg,
-                     free_words_per_octant(dim), fm, changed, report);
-  return hipGetLastError();
-}
-
 // ---- clearance map: how far a ray's line stays clear of everything ----
 // Cells of 8^3 blocks, R = dim / 8 per axis (a power of two, 4 .. 128).  A
 // cell is near when the cell widened by 2 blocks a side holds a nonempty
@@ -417,8 +417,9 @@ hipError_t launch_build_freemap(const uint64_t* l1, uint32_t dim, uint32_t* fm,
 // x the distance to the first near cell of the row, along y min over j of
 // max(j, that of the row j ahead), along z the same of those planes -- 2, 4
 // and 8 direction variants.  Bound by the search (at most the distance itself
-// per cell): four cells a thread, as 16-bit pairs.  512^3: 12 + 12 + 13 us
-// (one cell a thread: 32 + 21 + 57), 1024^3 about 8 times that.
+// per cell): four cells a thread, as 16-bit pairs.  512^3, with the rows
+// alone: 12 + 9 + 12 us (one cell a thread: 32 + 21 + 57), 1024^3 about 8
+// times that.
 
 // Whether the cell is near: its own word, and of each neighbour the
 // sub-blocks that face it.  Neighbours' codes by dilated increments; a
@@ -451,25 +452,35 @@ __device__ __forceinline__ bool cell_near(const uint64_t* __restrict__ words, ui
 }
 
 // Rows of cells along x, one thread per cell: the distance along +x (plane 0)
-// and -x (plane 1) to the first near cell of the row.  A block takes 256
+// and -x (plane 1) to the first near cell of the row.  A block takes kMapBlock
 // cells (whole rows), finds the rows' near cells by ballot and notes how many
 // it has.
-__global__ __launch_bounds__(256) void k_clear_rows(const uint64_t* __restrict__ words,
-                                                    uint32_t lg, uint8_t* __restrict__ rows,
-                                                    uint32_t* __restrict__ near_count,
-                                                    const uint32_t* __restrict__ changed) {
-  if (changed && *changed == 0u) return;  // the same for every thread
-  __shared__ uint64_t bits[4];
+struct ClearRowsArgs {
+  const uint64_t* words;
+  uint32_t lg;
+  uint8_t* rows;
+  uint32_t* near_count;
+  const uint32_t* changed;
+};
+__device__ __forceinline__ void clear_rows_block(const ClearRowsArgs& a, uint32_t block,
+                                                 uint64_t* bits) {
+  const uint64_t* __restrict__ words = a.words;
+  uint8_t* __restrict__ rows = a.rows;
+  const uint32_t lg = a.lg;
+  if (a.changed && *a.changed == 0u) return;  // the same for every thread
   const uint32_t R = 1u << lg, n = 1u << (3u * lg);
-  const uint32_t i = blockIdx.x * 256u + threadIdx.x, x = i & (R - 1u);
+  const uint32_t i = block * kMapBlock + threadIdx.x, x = i & (R - 1u);
   bool near = false;
   if (i < n) near = cell_near(words, R, x, (i >> lg) & (R - 1u), i >> (2u * lg));
   const uint64_t b = __ballot(near);
   if ((threadIdx.x & 63u) == 0u) bits[threadIdx.x >> 6] = b;
   __syncthreads();
-  if (threadIdx.x == 0u)
-    near_count[blockIdx.x] = (uint32_t)(__popcll(bits[0]) + __popcll(bits[1]) +
-                                        __popcll(bits[2]) + __popcll(bits[3]));
+  if (threadIdx.x == 0u) {
+    uint32_t count = 0u;
+#pragma unroll
+    for (uint32_t k = 0; k < kMapBlock / 64u; k++) count += (uint32_t)__popcll(bits[k]);
+    a.near_count[block] = count;
+  }
   if (i >= n) return;
   // the row's bits, as one or two words (R <= 64: part of the wave's)
   const uint32_t first = threadIdx.x - x, w0 = first >> 6, sh = first & 63u;
@@ -490,6 +501,21 @@ __global__ __launch_bounds__(256) void k_clear_rows(const uint64_t* __restrict__
     down = x - (63u - (uint32_t)__builtin_clzll(dn_lo));
   rows[i] = (uint8_t)up;
   rows[(size_t)n + i] = (uint8_t)down;
+}
+
+// The free-region map and the clearance map's first pass in one launch: they
+// read different words and neither waits for the other, and each was a
+// launch of 12-15 us with most of the chip idle (8 blocks; 262,144 threads of
+// one wave's latency).  The first 8 blocks take the octants' bitmaps, the
+// others the rows of cells.  A rebuild at 512^3 37 us instead of 48 (this
+// launch 17 of them; the octants' blocks, one CU each, bound it).
+__global__ __launch_bounds__(1024) void k_maps_first(FreeMapArgs fa, ClearRowsArgs ca) {
+  __shared__ uint64_t row[4096];
+  __shared__ uint32_t total;
+  if (blockIdx.x < 8u)
+    free_map_block(fa, row, total);
+  else
+    clear_rows_block(ca, blockIdx.x - 8u, row);
 }
 
 // Four bytes as two pairs of 16 bits, and back.
@@ -548,7 +574,8 @@ __global__ __launch_bounds__(256) void k_clear_planes(const uint8_t* __restrict_
     if (threadIdx.x == 0u) total = 0u;
     __syncthreads();
     uint32_t sum = 0;
-    for (uint32_t b = threadIdx.x; b < (n + 255u) / 256u; b += 256u) sum += near_count[b];
+    for (uint32_t b = threadIdx.x; b < (n + kMapBlock - 1u) / kMapBlock; b += 256u)
+      sum += near_count[b];
     if (sum) atomicAdd(&total, sum);
     __syncthreads();
     if (threadIdx.x == 0u) report->near_cells = total;
@@ -599,19 +626,31 @@ size_t clear_tmp_bytes(uint32_t dim) {
   return 14u * n + 4u * ((n + 255u) / 256u);
 }
 
-hipError_t launch_build_clear(uint8_t* tmp, uint32_t dim, uint8_t* map, const uint32_t* changed,
-                              CtxReport* report, hipStream_t stream) {
+// The rebuild of a world's maps; without a clearance map (map null) the
+// free-region map alone.  changed: two device words, whether a region and
+// whether a sub-block emptied or filled; null = rebuild both.
+static hipError_t launch_build_maps(const uint64_t* l1, uint32_t dim, uint32_t* fm, uint8_t* tmp,
+                                    uint8_t* map, const uint32_t* changed, CtxReport* report,
+                                    hipStream_t stream) {
+  FreeMapArgs fa = {l1, 0u, free_words_per_octant(dim), fm, changed, report};
+  while ((1u << fa.lg) < free_regions(dim)) fa.lg++;
+  if (!map) {
+    hipLaunchKernelGGL(k_maps_first, dim3(8), dim3(kMapBlock), 0, stream, fa, ClearRowsArgs{});
+    return hipGetLastError();
+  }
   const uint32_t n = clear_cells(dim);
   uint32_t lg = 0;
   while ((8u << lg) < dim) lg++;
   uint8_t *rows = tmp + 8u * (size_t)n, *planes = rows + 2u * (size_t)n;
   uint32_t* near_count = reinterpret_cast<uint32_t*>(planes + 4u * (size_t)n);
-  hipLaunchKernelGGL(k_clear_rows, dim3((n + 255u) / 256u), dim3(256), 0, stream,
-                     reinterpret_cast<const uint64_t*>(tmp), lg, rows, near_count, changed);
+  const uint32_t* moved = changed ? changed + 1 : nullptr;
+  const ClearRowsArgs ca = {reinterpret_cast<const uint64_t*>(tmp), lg, rows, near_count, moved};
+  hipLaunchKernelGGL(k_maps_first, dim3(8u + (n + kMapBlock - 1u) / kMapBlock), dim3(kMapBlock), 0,
+                     stream, fa, ca);
   hipLaunchKernelGGL(k_clear_planes, dim3((n + 255u) / 256u), dim3(256), 0, stream, rows, lg,
-                     planes, near_count, changed, report);
+                     planes, near_count, moved, report);
   hipLaunchKernelGGL(k_clear_cubes, dim3((2u * n + 255u) / 256u), dim3(256), 0, stream, planes,
-                     lg, map, changed);
+                     lg, map, moved);
   return hipGetLastError();
 }
 
@@ -624,14 +663,8 @@ hipError_t rebuild_maps(vt_world* w, hipStream_t stream, const uint32_t* changed
   if (!w->maps_valid) changed = nullptr;  // whatever the maps hold is not current
   w->maps_valid = false;
   if (!w->freemap) return hipSuccess;
-  CtxReport* report = w->ctx->report_dev();
-  if (w->clear) {
-    const hipError_t e = launch_build_clear(w->clear_tmp, w->dim, w->clear,
-                                            changed ? changed + 1 : nullptr, report, stream);
-    if (e != hipSuccess) return e;
-  }
-  return launch_build_freemap(w->kind == WorldKind::Dense ? w->l1 : w->brick_bits, w->dim,
-                              w->freemap, changed, report, stream);
+  return launch_build_maps(w->kind == WorldKind::Dense ? w->l1 : w->brick_bits, w->dim, w->freemap,
+                           w->clear_tmp, w->clear, changed, w->ctx->report_dev(), stream);
 }
 
 void finish_maps(vt_world* w) {
