@@ -946,6 +946,7 @@ enum SkipStatus : int {
   kSkipBlocked = 1,  // an iteration met a nonzero byte or left the grid
   kSkipFree = 2,     // nothing ahead of the ray on all three axes: a miss
   kSkipOpen = 3,     // the wave's rays stand clear of everything: clear_advance
+  kSkipPause = 4,    // most of the wave's rays wait for the others
 };
 
 // ---- ClearMap: the clearance map (built by k_maps_first, k_clear_planes and k_clear_cubes) ----
@@ -1157,7 +1158,9 @@ __device__ __forceinline__ void dense_skip_blind(float Px, float Py, float Pz, f
 // kSkipFree, the ray can hit nothing more; when the cells of all the wave's
 // rays in the loop have clear neighbours ahead (>= 2) they leave together
 // with kSkipOpen for clear_advance (one ray at a time would have the wave
-// alternate between the loops).  Returns kSkipBlocked when it stopped at an
+// alternate between the loops).  With kPause the last quarter of the `entered`
+// rays that began together leave with kSkipPause, to take the run up again
+// later.  Returns kSkipBlocked when it stopped at an
 // iteration that met a nonzero byte or left the grid, kSkipLimit at the
 // limit; either way `s` is a state the exact loop (or another call)
 // continues from.
@@ -1167,7 +1170,7 @@ __device__ __forceinline__ void dense_skip_blind(float Px, float Py, float Pz, f
 // taken again with it when a crossing time says that such a state was among
 // them (4% of the rays of a terrain frame meet one): 29 VALU + 8 SALU a step
 // against 39 + 19, and 25 + 3 with step_axis and morton_step.
-template <int K, bool kClear>
+template <int K, bool kClear, bool kPause = false>
 __device__ __forceinline__ int dense_skip_empty(float Px, float Py, float Pz, float Ax, float Ay,
                                                 float Az, float dx, float dy, float dz, float ix,
                                                 float iy, float iz, uint32_t mx, uint32_t my,
@@ -1175,7 +1178,7 @@ __device__ __forceinline__ int dense_skip_empty(float Px, float Py, float Pz, fl
                                                 int& steps, int limit,
                                                 __amdgpu_buffer_rsrc_t bytes,
                                                 __amdgpu_buffer_rsrc_t cm, uint32_t cofs,
-                                                bool usable) {
+                                                bool usable, int entered = 0) {
   float bx = s.wx, by = s.wy, bz = s.wz;
   uint32_t bc = s.c;
   int sb = steps;
@@ -1224,6 +1227,10 @@ __device__ __forceinline__ int dense_skip_empty(float Px, float Py, float Pz, fl
       status = kSkipOpen;
       break;
     }
+    if (kPause && 4 * __popcll(__ballot(true)) < entered) {
+      status = kSkipPause;
+      break;
+    }
   }
   s.wx = bx;
   s.wy = by;
@@ -1251,12 +1258,13 @@ __device__ __forceinline__ int dense_skip_empty(float Px, float Py, float Pz, fl
 // on lattice points, so this correction is frequent for them: as a branch it
 // ran in about half of the wave-steps.
 // The clearance map's part is dense_skip_empty's, on octant 0's plane.
-template <int K, bool kClear>
+template <int K, bool kClear, bool kPause = false>
 __device__ __forceinline__ int dense_skip_positive(float dx, float dy, float dz, float ix,
                                                    float iy, float iz, uint32_t mx, uint32_t my,
                                                    uint32_t mz, DenseCell& s, int& steps,
                                                    int limit, __amdgpu_buffer_rsrc_t bytes,
-                                                   __amdgpu_buffer_rsrc_t cm, bool usable) {
+                                                   __amdgpu_buffer_rsrc_t cm, bool usable,
+                                                   int entered = 0) {
   float bx = s.wx, by = s.wy, bz = s.wz;
   uint32_t bc = s.c;
   int sb = steps;
@@ -1314,6 +1322,10 @@ __device__ __forceinline__ int dense_skip_positive(float dx, float dy, float dz,
     sb += K;
     if (kClear && __ballot(!((m >= 2u) & usable)) == 0ull) {
       status = kSkipOpen;
+      break;
+    }
+    if (kPause && 4 * __popcll(__ballot(true)) < entered) {
+      status = kSkipPause;
       break;
     }
   }
@@ -1876,17 +1888,19 @@ __device__ bool trace_brickmap_fast(const BrickmapWorld& w, float ox, float oy, 
   const __amdgpu_buffer_rsrc_t cm = clear_rsrc(w.clear, w.clear_bytes);
   const bool usable = kClear && ordered && clear_usable(inv[0], inv[1], inv[2]);
   bool open = kClear && !kShadow;
+  bool paused = false;  // in the middle of an empty-space run
   for (;;) {
     // The literal loop (both levels) until the lane stands at an empty
     // block at the block level, hits, leaves the map or reaches the cap.
     // Lanes at an empty block wait here for the rest of the wave, so the
     // wave's empty-space runs below start together.
-    bool fast = false;
+    bool fast = paused;
+    paused = false;
     // The block of the last lookup, so that the lookup of a step inside it
     // makes no load.  Successive lookups are neighbours, so 11 bits an axis
     // tell their blocks apart.
     uint32_t key = 0xFFFFFFFFu, block = 0u;
-    for (;;) {
+    while (!fast) {
       if (step >= max_steps || g[0] >= B || g[1] >= B || g[2] >= B || g[0] < 0 || g[1] < 0 ||
           g[2] < 0)
         break;
@@ -1981,6 +1995,7 @@ __device__ bool trace_brickmap_fast(const BrickmapWorld& w, float ox, float oy, 
     int status;
     const uint32_t cofs =
         kPositive || !kClear ? 0u : clear_octant_offset(flip, mx, my, mz, w.clear_oct_bytes);
+    const int entered = __popcll(__ballot(true));
     for (;;) {
       if constexpr (kClear) {
         if (open & usable) {
@@ -1994,17 +2009,39 @@ __device__ bool trace_brickmap_fast(const BrickmapWorld& w, float ox, float oy, 
         }
       }
       if constexpr (kPositive)
-        status = dense_skip_positive<kSkip, kClear>(d[0], d[1], d[2], inv[0], inv[1], inv[2], mx,
-                                                    my, mz, s0, s0steps, limit, occ, cm, usable);
+        status = dense_skip_positive<kSkip, kClear, kClear>(d[0], d[1], d[2], inv[0], inv[1], inv[2], mx,
+                                                    my, mz, s0, s0steps, limit, occ, cm, usable,
+                                                    entered);
       else
-        status = dense_skip_empty<kSkip, kClear>(P3[0], P3[1], P3[2], A3[0], A3[1], A3[2], d[0],
+        status = dense_skip_empty<kSkip, kClear, kClear>(P3[0], P3[1], P3[2], A3[0], A3[1], A3[2], d[0],
                                                  d[1], d[2], inv[0], inv[1], inv[2], mx, my, mz,
                                                  flip, s0, s0steps, limit, occ, cm, cofs,
-                                                 usable);
+                                                 usable, entered);
       if (status != kSkipOpen) break;
       open = true;
     }
     open = false;  // the next run starts at a nonempty block
+    if (kClear && status == kSkipPause) {
+      // Three quarters of the rays that began this run wait for the rest, at
+      // blocks of their own: those go on first, and this ray takes its run up
+      // again with them, from the state it has reached.  Otherwise every run of
+      // a wave lasts as long as its longest ray's, and a wave whose rays meet
+      // model blocks at different depths pays the longest run once per block
+      // (half of the cycles of a frame's last waves).  Six views of the engine's
+      // map with long caps at 1600x900 203 -> 184 us, at 320x180 143 -> 135, an
+      // edit with its frame 312 -> 296, the engine's frame 104.5 -> 104.6; at half
+      // of the rays 175, 142, 290 and 107; at a sixth 194, 140, 300 and 105.
+      paused = true;
+      const uint32_t gc = s0.c ^ flip;
+      g[0] = (int)(compact1by2(gc) << 3);
+      g[1] = (int)(compact1by2(gc >> 1) << 3);
+      g[2] = (int)(compact1by2(gc >> 2) << 3);
+      wc[0] = s0.wx;
+      wc[1] = s0.wy;
+      wc[2] = s0.wz;
+      step = s0steps;
+      continue;
+    }
     if (kClear && status == kSkipFree) {
       step = s0steps;
       break;
