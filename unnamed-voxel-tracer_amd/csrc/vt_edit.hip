@@ -106,7 +106,7 @@ __global__ __launch_bounds__(256) void k_edit_dense(uint8_t* __restrict__ vox,
 }
 
 // The L0 words of the listed 4^3 bricks (one wave per word: ballot over its
-// 64 bytes) and their sub-block bits.
+// 64 bytes; no list: of the first n) and their sub-block bits.
 __global__ __launch_bounds__(256) void k_edit_l0(const uint8_t* __restrict__ vox,
                                                  uint64_t* __restrict__ l0,
                                                  const uint32_t* __restrict__ bricks, uint32_t n,
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(256) void k_edit_l0(const uint8_t* __restrict__ vox
                                                  uint32_t* __restrict__ changed) {
   const uint32_t wave = (blockIdx.x * 256u + threadIdx.x) >> 6, lane = threadIdx.x & 63u;
   if (wave >= n) return;  // whole waves leave together
-  const uint32_t b = bricks[wave];
+  const uint32_t b = bricks ? bricks[wave] : wave;
   const uint64_t m = __ballot(vox[(size_t)b * 64u + lane] != 0);
   if (lane == 0) {
     l0[b] = m;
@@ -122,16 +122,16 @@ __global__ __launch_bounds__(256) void k_edit_l0(const uint8_t* __restrict__ vox
   }
 }
 
-// The L1 words of the listed 16^3 regions, one wave per word: bit l =
-// (l0[region * 64 + l] != 0).  Sets changed[0] when a word stops or starts
-// being zero.
+// The L1 words of the listed 16^3 regions (no list: of the first n), one wave
+// per word: bit l = (l0[region * 64 + l] != 0).  Sets changed[0] when a word
+// stops or starts being zero.
 __global__ __launch_bounds__(256) void k_edit_l1(const uint64_t* __restrict__ l0,
                                                  uint64_t* __restrict__ l1,
                                                  const uint32_t* __restrict__ regions, uint32_t n,
                                                  uint32_t* __restrict__ changed) {
   const uint32_t wave = (blockIdx.x * 256u + threadIdx.x) >> 6, lane = threadIdx.x & 63u;
   if (wave >= n) return;  // whole waves leave together
-  const uint32_t r = regions[wave];
+  const uint32_t r = regions ? regions[wave] : wave;
   const uint64_t m = __ballot(l0[(size_t)r * 64u + lane] != 0ull);
   if (lane == 0) {
     if ((l1[r] == 0ull) != (m == 0ull)) changed[0] = 1u;
@@ -402,21 +402,28 @@ int set_brickmap(vt_world* w, const uint32_t* xyz, const uint32_t* values, uint3
   Lists lists(w->ctx, s);
   VT_HIP(lists.put(words));
   const uint32_t* d_chunks = lists.dev + 3 * (size_t)nw;
+  const bool current = vt::begin_occupancy_change(w);
   hipLaunchKernelGGL(vt::k_edit_brickmap, dim3(blocks_for(std::max(nw, nc), 256)), dim3(256), 0, s,
                      w->pool, w->occ, w->chunks, lists.dev, nw, nc, vt::maps_changed(w));
   hipError_t e = hipGetLastError();
   if (e == hipSuccess && w->occ) {
-    hipLaunchKernelGGL(vt::k_edit_bricks, dim3(blocks_for(nb, 4)), dim3(256), 0, s, w->occ,
-                       d_chunks + 2 * (size_t)nc, nb, (unsigned long long*)w->brick_bits,
-                       w->clear_tmp, vt::maps_changed(w));
-    e = hipGetLastError();
-    if (e == hipSuccess) e = vt::rebuild_maps(w, s, vt::maps_changed(w));
+    if (current) {
+      hipLaunchKernelGGL(vt::k_edit_bricks, dim3(blocks_for(nb, 4)), dim3(256), 0, s, w->occ,
+                         d_chunks + 2 * (size_t)nc, nb, (unsigned long long*)w->brick_bits,
+                         w->clear_tmp, vt::maps_changed(w));
+      e = hipGetLastError();
+    } else {  // an earlier change failed midway: everything from the pool
+      e = vt::launch_build_occupancy(vt::brickmap_view(w), w->occ, w->brick_bits, w->clear_tmp, s);
+    }
+    if (e == hipSuccess) e = vt::rebuild_maps(w, s, current ? vt::maps_changed(w) : nullptr);
   }
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) {
     // Undo what may have reached the device: new chunk entries back to 0
     // and the new blocks zero again (edits allocate zero blocks), so the
-    // device agrees with the unchanged host chunk table and pool count.
+    // device agrees with the unchanged host chunk table and pool count.  The
+    // occupancy bytes may stay set where the pool is zero again (a lookup
+    // then reads the empty block) until the next change makes them anew.
     if (nc)
       hipLaunchKernelGGL(vt::k_unset_chunks, dim3(blocks_for(nc, 256)), dim3(256), 0, s, w->chunks,
                          d_chunks, nc);
@@ -461,6 +468,7 @@ int set_dense(vt_world* w, const uint32_t* xyz, const uint32_t* values, uint32_t
     if (regions.empty() || regions.back() != b >> 6) regions.push_back(b >> 6);
     if (regions8.empty() || regions8.back() != b >> 9) regions8.push_back(b >> 9);
   }
+  const uint64_t nwords = (uint64_t)w->dim * w->dim * w->dim / 64u;
   const uint32_t nw = (uint32_t)(words.size() / 2u), nb = (uint32_t)bricks.size(),
                  nr = (uint32_t)regions.size(), nr8 = (uint32_t)regions8.size();
   words.insert(words.end(), bricks.begin(), bricks.end());
@@ -469,18 +477,28 @@ int set_dense(vt_world* w, const uint32_t* xyz, const uint32_t* values, uint32_t
   Lists lists(w->ctx, s);
   VT_HIP(lists.put(words));
   const uint32_t* d_bricks = lists.dev + 2 * (size_t)nw;
+  const bool current = vt::begin_occupancy_change(w);
   hipLaunchKernelGGL(vt::k_edit_dense, dim3(blocks_for(nw, 256)), dim3(256), 0, s, w->vox,
                      lists.dev, nw, vt::maps_changed(w));
-  hipLaunchKernelGGL(vt::k_edit_l0, dim3(blocks_for(nb, 4)), dim3(256), 0, s, w->vox, w->l0,
-                     d_bricks, nb, w->clear_tmp, vt::maps_changed(w));
-  hipLaunchKernelGGL(vt::k_edit_l1, dim3(blocks_for(nr, 4)), dim3(256), 0, s, w->l0, w->l1,
-                     d_bricks + nb, nr, vt::maps_changed(w));
-  VT_HIP(hipGetLastError());
-  VT_HIP(vt::launch_build_l1b(w->l0, (uint64_t)w->dim * w->dim * w->dim / 64u,
-                              d_bricks + nb + nr, nr8, w->l1b, s));
-  VT_HIP(vt::rebuild_maps(w, s, vt::maps_changed(w)));
+  if (current) {
+    hipLaunchKernelGGL(vt::k_edit_l0, dim3(blocks_for(nb, 4)), dim3(256), 0, s, w->vox, w->l0,
+                       d_bricks, nb, w->clear_tmp, vt::maps_changed(w));
+    hipLaunchKernelGGL(vt::k_edit_l1, dim3(blocks_for(nr, 4)), dim3(256), 0, s, w->l0, w->l1,
+                       d_bricks + nb, nr, vt::maps_changed(w));
+    VT_HIP(hipGetLastError());
+    VT_HIP(vt::launch_build_l1b(w->l0, nwords, d_bricks + nb + nr, nr8, w->l1b, s));
+  } else {  // an earlier change failed midway: every level from the voxels
+    const uint32_t n0 = (uint32_t)nwords, n1 = (uint32_t)(nwords / 64u);
+    hipLaunchKernelGGL(vt::k_edit_l0, dim3(blocks_for(n0, 4)), dim3(256), 0, s, w->vox, w->l0,
+                       nullptr, n0, w->clear_tmp, vt::maps_changed(w));
+    hipLaunchKernelGGL(vt::k_edit_l1, dim3(blocks_for(n1, 4)), dim3(256), 0, s, w->l0, w->l1,
+                       nullptr, n1, vt::maps_changed(w));
+    VT_HIP(hipGetLastError());
+    VT_HIP(vt::launch_build_l1b(w->l0, nwords, nullptr, (uint32_t)vt::l1b_words(w->dim), w->l1b,
+                                s));
+  }
+  VT_HIP(vt::rebuild_maps(w, s, current ? vt::maps_changed(w) : nullptr));
   if (w->prefix) {  // keep the compact index current
-    const uint64_t nwords = (uint64_t)w->dim * w->dim * w->dim / 64u;
     const uint64_t ntiles = (nwords + 1023) / 1024;
     uint32_t* scratch = nullptr;
     VT_HIP(hipMalloc((void**)&scratch, (ntiles + 1) * 4));

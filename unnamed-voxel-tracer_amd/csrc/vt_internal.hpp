@@ -237,11 +237,21 @@ bool use_clear_map(const vt_world* w, uint32_t flags);
 // (they then count the steps executed); on the reference layout occupancy
 // bytes and no statistics.
 bool render_clear_map(const vt_world* w, const vt_render_params& p, const vt_frame& f);
+// To be called before the first kernel that changes a world's voxels is
+// enqueued: from here until finish_maps the maps and the occupancy levels may
+// differ from the voxels, and the renderers read neither map.  False: they
+// did already (an earlier change failed midway), so the levels have to be
+// made from all voxels and the maps rebuilt whatever this change does.
+inline bool begin_occupancy_change(vt_world* w) {
+  const bool current = w->maps_valid || !w->freemap;
+  w->maps_valid = false;
+  return current;
+}
 // Rebuilds a world's free-region and clearance maps from its current
 // occupancy (L1 words or brick bits, and the sub-block bits); no-op without
 // them.  `changed`: the two words of maps_changed (null: rebuild always).
-// Clears maps_valid: the caller calls finish_maps once the stream has
-// synchronised without error, and until then the renderers read neither.
+// Leaves maps_valid false: the caller calls finish_maps once the stream has
+// synchronised without error.
 hipError_t rebuild_maps(vt_world* w, hipStream_t stream, const uint32_t* changed = nullptr);
 // The words edits set: [0] a 16^3 region emptied or filled, [1] a 2^3
 // sub-block did.

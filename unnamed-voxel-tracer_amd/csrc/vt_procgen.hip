@@ -377,6 +377,7 @@ int vt_world_procgen(vt_ctx* ctx, vt_world* world, float offset_x, float offset_
   vt::TreeVoxel* d_tv = (vt::TreeVoxel*)(d_cols + 2 * ncol);
   // From here on the device map changes; the host chunk table and pool count
   // follow only once all of it succeeded.
+  const bool current = vt::begin_occupancy_change(world);
   hipError_t e = hipMemcpyAsync(world->chunks, walk.mirror.data(), nchunks * 4,
                                 hipMemcpyHostToDevice, s);
   if (e == hipSuccess)
@@ -395,9 +396,11 @@ int vt_world_procgen(vt_ctx* ctx, vt_world* world, float offset_x, float offset_
     e = hipGetLastError();
   }
   // the empty map's occupancy bytes were zero; only the written layers change
+  // (all of them where an earlier change that failed may have left some set)
   if (e == hipSuccess && world->occ)
     e = vt::launch_build_occupancy(vt::brickmap_view(world), world->occ, world->brick_bits,
-                                   world->clear_tmp, s, std::min(dim, (walk.y_end + 7u) & ~7u));
+                                   world->clear_tmp, s,
+                                   current ? std::min(dim, (walk.y_end + 7u) & ~7u) : dim);
   if (e == hipSuccess) e = vt::rebuild_maps(world, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) {

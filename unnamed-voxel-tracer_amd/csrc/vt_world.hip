@@ -660,7 +660,6 @@ uint32_t brick_bit_words(uint32_t dim) {
 }
 
 hipError_t rebuild_maps(vt_world* w, hipStream_t stream, const uint32_t* changed) {
-  if (!w->maps_valid) changed = nullptr;  // whatever the maps hold is not current
   w->maps_valid = false;
   if (!w->freemap) return hipSuccess;
   return launch_build_maps(w->kind == WorldKind::Dense ? w->l1 : w->brick_bits, w->dim, w->freemap,
