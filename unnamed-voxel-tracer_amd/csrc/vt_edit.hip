@@ -30,8 +30,9 @@
 
 namespace vt {
 
-// The edits of a brickmap world.  data: n records (pool word, value, block's
-// Morton code), then m records (chunk, its new entry).
+// The edits of a brickmap world.  data: n records (pool block, value, voxel's
+// Morton code), then m records (chunk, its new entry).  The code's low 9 bits
+// place the voxel in its pool block; a pool can hold more than 2^32 words.
 __global__ __launch_bounds__(256) void k_edit_brickmap(uint32_t* __restrict__ pool,
                                                        uint8_t* __restrict__ occ,
                                                        uint32_t* __restrict__ chunks,
@@ -42,7 +43,8 @@ __global__ __launch_bounds__(256) void k_edit_brickmap(uint32_t* __restrict__ po
   if (i < 2u && changed) changed[i] = 0u;  // for the kernels that follow
   if (i < n) {
     const uint3 r = reinterpret_cast<const uint3*>(data)[i];
-    pool[r.x] = r.y;
+    pool[(size_t)r.x * 512u + (compact1by2(r.z) & 7u) + 8u * (compact1by2(r.z >> 1) & 7u) +
+         64u * (compact1by2(r.z >> 2) & 7u)] = r.y;
     if (occ) occ[r.z] = r.y != 0u ? 1 : 0;
   }
   if (i < m) {
@@ -361,7 +363,7 @@ int set_brickmap(vt_world* w, const uint32_t* xyz, const uint32_t* values, uint3
   // table only once the device holds them, so a failed call leaves the
   // world as it was
   std::unordered_map<uint64_t, uint32_t> fresh;
-  std::vector<uint32_t> words;  // records (pool word, value, Morton code), see k_edit_brickmap
+  std::vector<uint32_t> words;  // records (pool block, value, Morton code), see k_edit_brickmap
   std::vector<uint32_t> chunks, bricks;
   uint64_t used = w->pool_words / 512u;
   last.reserve(n);
@@ -375,7 +377,9 @@ int set_brickmap(vt_world* w, const uint32_t* xyz, const uint32_t* values, uint3
       if (f != fresh.end()) {
         entry = f->second;
       } else {  // get_block_for_chunk: allocate on first touch
-        entry = (uint32_t)(++used);  // at most one block per chunk: (dim / 8)^3
+        // (after the blocks of the pool the world was made with, however many)
+        if (used >= 0xFFFFFFFEull) return fail(VT_ERR_OUT_OF_MEMORY, "vt_world_set_voxels: pool");
+        entry = (uint32_t)(++used);
         fresh.emplace(ci, entry);
         chunks.push_back((uint32_t)ci);
         chunks.push_back(entry);
@@ -386,7 +390,7 @@ int set_brickmap(vt_world* w, const uint32_t* xyz, const uint32_t* values, uint3
     auto it = last.find(a);
     if (it == last.end()) {
       last.emplace(a, (uint32_t)(words.size() / 3u));
-      words.insert(words.end(), {(uint32_t)a, values[i], code});
+      words.insert(words.end(), {entry - 1u, values[i], code});
       bricks.push_back(code >> 6);
     } else {
       words[3 * (size_t)it->second + 1] = values[i];
