@@ -59,8 +59,7 @@ void free_world(vt_world* w) {
   dev_free(w->masks);
   dev_free(w->brick_bits);
   dev_free(w->freemap);
-  dev_free(w->clear);
-  dev_free(w->clear_tmp);
+  dev_free(w->clear);  // (and its scratch)
   delete[] w->chunk_mirror;
   delete w;
 }
@@ -91,10 +90,14 @@ int dev_alloc(vt_world* w, void** p, size_t bytes, const char* what) {
 int alloc_maps(vt_world* w) {
   int st = dev_alloc(w, (void**)&w->freemap, (8u * vt::free_words_per_octant(w->dim) + 2u) * 4u,
                      "free-region map");
-  if (st != VT_OK || w->dim < 32u) return st;  // (a 16^3 map has 2 cells a side)
-  st = dev_alloc(w, (void**)&w->clear, 16u * (size_t)vt::clear_cells(w->dim), "clearance map");
-  if (st != VT_OK) return st;
-  return dev_alloc(w, (void**)&w->clear_tmp, vt::clear_tmp_bytes(w->dim), "clearance scratch");
+  if (st != VT_OK || w->dim < 16u) return st;
+  // the clearance map and, behind it, its scratch (k_clear_16 needs none)
+  const size_t map = 16u * (size_t)vt::clear_cells(w->dim);
+  const bool tmp = w->dim >= 32u;
+  st = dev_alloc(w, (void**)&w->clear, map + (tmp ? vt::clear_tmp_bytes(w->dim) : 0u),
+                 "clearance map");
+  if (st == VT_OK && tmp) w->clear_tmp = w->clear + map;
+  return st;
 }
 
 }  // namespace

@@ -75,10 +75,11 @@ struct vt_world {
   uint32_t* freemap;       // 8 octants x free_words_per_octant(dim) words, then a
                            // two words edits set: when a region empties or
                            // fills, when a 2^3 sub-block does
-  // clearance map (the same worlds, dim >= 32)
+  // clearance map (the same worlds, dim >= 16)
   uint8_t* clear;          // 2 orders x 8 octants x clear_cells(dim) bytes
   uint8_t* clear_tmp;      // clear_tmp_bytes(dim): the sub-block bits of every
-                           // 4^3 brick (kept current), then build scratch
+                           // 4^3 brick (kept current), then build scratch;
+                           // dim >= 32
   bool maps_valid;         // both maps match the occupancy (finish_maps)
   float near_frac;         // share of near cells in the clearance map
   float free_frac;         // largest share of free regions over the 8 octants

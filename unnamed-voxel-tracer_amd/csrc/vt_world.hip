@@ -404,7 +404,8 @@ uint32_t free_words_per_octant(uint32_t dim) {
 }
 
 // ---- clearance map: how far a ray's line stays clear of everything ----
-// Cells of 8^3 blocks, R = dim / 8 per axis (a power of two, 4 .. 128).  A
+// Cells of 8^3 blocks, R = dim / 8 per axis (a power of two, 4 .. 128; 2:
+// k_clear_16).  A
 // cell is near when the cell widened by 2 blocks a side holds a nonempty
 // block.  For each of the 8 direction octants, the byte of a cell is the
 // Chebyshev distance in cells to the first near cell of its forward orthant:
@@ -616,6 +617,17 @@ __global__ __launch_bounds__(256) void k_clear_cubes(const uint8_t* __restrict__
       m;
 }
 
+// A 16^3 map has 2 cells a side and is one region: clear all round (255) when
+// it holds nothing, else all of it near, so that no ray is asked to walk 2
+// cells.
+__global__ __launch_bounds__(128) void k_clear_16(const uint64_t* __restrict__ l1,
+                                                  uint8_t* __restrict__ map,
+                                                  CtxReport* __restrict__ report) {
+  const bool empty = l1[0] == 0ull;
+  map[threadIdx.x] = empty ? 255 : 0;
+  if (threadIdx.x == 0u) report->near_cells = empty ? 0u : 8u;
+}
+
 uint32_t clear_cells(uint32_t dim) {
   const uint32_t R = dim / 8u;
   return R * R * R;
@@ -626,16 +638,17 @@ size_t clear_tmp_bytes(uint32_t dim) {
   return 14u * n + 4u * ((n + 255u) / 256u);
 }
 
-// The rebuild of a world's maps; without a clearance map (map null) the
-// free-region map alone.  changed: two device words, whether a region and
+// The rebuild of a world's maps; without a clearance map (map null, dim < 16)
+// the free-region map alone.  changed: two device words, whether a region and
 // whether a sub-block emptied or filled; null = rebuild both.
 static hipError_t launch_build_maps(const uint64_t* l1, uint32_t dim, uint32_t* fm, uint8_t* tmp,
                                     uint8_t* map, const uint32_t* changed, CtxReport* report,
                                     hipStream_t stream) {
   FreeMapArgs fa = {l1, 0u, free_words_per_octant(dim), fm, changed, report};
   while ((1u << fa.lg) < free_regions(dim)) fa.lg++;
-  if (!map) {
+  if (dim < 32u) {
     hipLaunchKernelGGL(k_maps_first, dim3(8), dim3(kMapBlock), 0, stream, fa, ClearRowsArgs{});
+    if (map) hipLaunchKernelGGL(k_clear_16, dim3(1), dim3(128), 0, stream, l1, map, report);
     return hipGetLastError();
   }
   const uint32_t n = clear_cells(dim);
