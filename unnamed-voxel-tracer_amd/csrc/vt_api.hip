@@ -303,7 +303,7 @@ bool render_clear_map(const vt_world* w, const vt_render_params& p, const vt_fra
   if (w->kind == WorldKind::Dense ? p.traversal != VT_TRAVERSAL_FLAT : !w->occ) return false;
   // statistics count traceMap's steps exactly when vt_free_map_used says so
   if (f.stats && !render_free_map(w, p, f)) return false;
-  return use_clear_map(w, p.flags);
+  return use_clear_map(w, p.flags, p.max_steps_primary, p.max_steps_shadow);
 }
 
 FrameOut frame_out(const vt_frame* frame) {

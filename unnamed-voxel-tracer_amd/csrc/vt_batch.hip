@@ -173,7 +173,9 @@ hipError_t launch_batch(const vt_world* world, const vt::ShadeConsts& sc_in,
                         uint32_t* d_queues, const vt_tuning& tuning, uint32_t nblocks,
                         unsigned long long* stats, bool steps_out, hipStream_t s) {
   vt::DenseWorld w = vt::dense_view(world);
-  if (steps_out || stats || !vt::use_clear_map(world, sc_in.flags)) w.clear_bytes = 0;
+  if (steps_out || stats ||
+      !vt::use_clear_map(world, sc_in.flags, sc_in.max_primary, sc_in.max_shadow))
+    w.clear_bytes = 0;
   // rays end early at the reach box unless their step counts are observed
   if (steps_out || stats) vt::reach_everywhere(w.reach_lo, w.reach_hi);
   vt::ShadeConsts sc = sc_in;

@@ -28,7 +28,8 @@ constexpr size_t kCtxReportBytes = 256;  // after the staging: CtxReport
 struct CtxReport {
   uint32_t free_built;       // 0: no region had changed, the map was left as it is
   uint32_t free_regions[8];  // else: free regions of each octant
-  uint32_t near_cells;       // near cells of the clearance map
+  uint32_t near_cells;       // near cells of the clearance map that are not filled
+  uint32_t filled_cells;     // cells of it with something in every 2^3 sub-block
   int32_t box_lo[3], box_hi[3];  // box of the nonempty voxels; lo > hi: none
 };
 static_assert(sizeof(CtxReport) <= kCtxReportBytes, "CtxReport");
@@ -81,7 +82,8 @@ struct vt_world {
                            // 4^3 brick (kept current), then build scratch;
                            // dim >= 32
   bool maps_valid;         // both maps match the occupancy (finish_maps)
-  float near_frac;         // share of near cells in the clearance map
+  float near_frac;         // share of near cells among the clearance map's cells
+                           // that are not filled: of the space rays cross
   float free_frac;         // largest share of free regions over the 8 octants
   // the box of a dense world's nonempty voxels, inclusive; grown by edits,
   // never shrunk; box_any = false while the world has none
@@ -228,10 +230,10 @@ uint32_t free_words_per_octant(uint32_t dim);
 // reports the near cells.
 uint32_t clear_cells(uint32_t dim);
 size_t clear_tmp_bytes(uint32_t dim);
-// Whether launches with these flags use the clearance map: it is valid and
-// VT_FLAG_FREE_MAP_ON, or neither FREE_MAP flag and a world open enough for
-// it to pay.
-bool use_clear_map(const vt_world* w, uint32_t flags);
+// Whether launches with these flags and step caps use the clearance map: it is
+// valid and VT_FLAG_FREE_MAP_ON, or neither FREE_MAP flag and a world open
+// enough for it to pay.
+bool use_clear_map(const vt_world* w, uint32_t flags, int max_primary, int max_shadow);
 // Whether vt_render uses it for this world, parameters and frame: no stored
 // step counts (they would lack the steps of rays that end early); on dense
 // worlds the flat traversal, and statistics only with VT_FLAG_FREE_MAP_ON

@@ -424,9 +424,10 @@ uint32_t free_words_per_octant(uint32_t dim) {
 
 // Whether the cell is near: its own word, and of each neighbour the
 // sub-blocks that face it.  Neighbours' codes by dilated increments; a
-// neighbour outside the grid repeats the cell itself.
+// neighbour outside the grid repeats the cell itself.  filled: every sub-block
+// of the cell holds something.
 __device__ __forceinline__ bool cell_near(const uint64_t* __restrict__ words, uint32_t R,
-                                          uint32_t x, uint32_t y, uint32_t z) {
+                                          uint32_t x, uint32_t y, uint32_t z, bool& filled) {
   // sub-blocks of a word with x coordinate 0 / 3 (bits 0 and 3 of the code)
   constexpr uint64_t X0 = 0x0055005500550055ull, X3 = X0 << 9;
   constexpr uint64_t Y0 = 0x0000333300003333ull, Y3 = Y0 << 18;
@@ -449,13 +450,14 @@ __device__ __forceinline__ bool cell_near(const uint64_t* __restrict__ words, ui
         if (k != 1) mask &= k == 0 ? Z3 : Z0;
         any |= words[cx[i] | cy[j] | cz[k]] & mask;
       }
+  filled = words[cx[1] | cy[1] | cz[1]] == ~0ull;
   return any != 0ull;
 }
 
 // Rows of cells along x, one thread per cell: the distance along +x (plane 0)
 // and -x (plane 1) to the first near cell of the row.  A block takes kMapBlock
 // cells (whole rows), finds the rows' near cells by ballot and notes how many
-// it has.
+// of them are not filled (low half of its count) and how many are (high half).
 struct ClearRowsArgs {
   const uint64_t* words;
   uint32_t lg;
@@ -471,15 +473,21 @@ __device__ __forceinline__ void clear_rows_block(const ClearRowsArgs& a, uint32_
   if (a.changed && *a.changed == 0u) return;  // the same for every thread
   const uint32_t R = 1u << lg, n = 1u << (3u * lg);
   const uint32_t i = block * kMapBlock + threadIdx.x, x = i & (R - 1u);
-  bool near = false;
-  if (i < n) near = cell_near(words, R, x, (i >> lg) & (R - 1u), i >> (2u * lg));
-  const uint64_t b = __ballot(near);
-  if ((threadIdx.x & 63u) == 0u) bits[threadIdx.x >> 6] = b;
+  bool near = false, filled = false;
+  if (i < n) near = cell_near(words, R, x, (i >> lg) & (R - 1u), i >> (2u * lg), filled);
+  const uint64_t b = __ballot(near), f = __ballot(filled);
+  if ((threadIdx.x & 63u) == 0u) {
+    bits[threadIdx.x >> 6] = b;
+    bits[kMapBlock / 64u + (threadIdx.x >> 6)] = f;
+  }
   __syncthreads();
   if (threadIdx.x == 0u) {
-    uint32_t count = 0u;
+    uint32_t count = 0u;  // (a filled cell is near)
 #pragma unroll
-    for (uint32_t k = 0; k < kMapBlock / 64u; k++) count += (uint32_t)__popcll(bits[k]);
+    for (uint32_t k = 0; k < kMapBlock / 64u; k++) {
+      const uint32_t full = (uint32_t)__popcll(bits[kMapBlock / 64u + k]);
+      count += (uint32_t)__popcll(bits[k]) - full + (full << 16);
+    }
     a.near_count[block] = count;
   }
   if (i >= n) return;
@@ -571,15 +579,21 @@ __global__ __launch_bounds__(256) void k_clear_planes(const uint8_t* __restrict_
   const bool run = !changed || *changed != 0u;  // the same for every thread
   const uint32_t R = 1u << lg, n = 1u << (3u * lg);
   if (blockIdx.x == 0u) {
-    __shared__ uint32_t total;
-    if (threadIdx.x == 0u) total = 0u;
+    __shared__ uint32_t total[2];
+    if (threadIdx.x < 2u) total[threadIdx.x] = 0u;
     __syncthreads();
-    uint32_t sum = 0;
-    for (uint32_t b = threadIdx.x; b < (n + kMapBlock - 1u) / kMapBlock; b += 256u)
-      sum += near_count[b];
-    if (sum) atomicAdd(&total, sum);
+    uint32_t open = 0, full = 0;
+    for (uint32_t b = threadIdx.x; b < (n + kMapBlock - 1u) / kMapBlock; b += 256u) {
+      open += near_count[b] & 0xFFFFu;
+      full += near_count[b] >> 16;
+    }
+    if (open) atomicAdd(&total[0], open);
+    if (full) atomicAdd(&total[1], full);
     __syncthreads();
-    if (threadIdx.x == 0u) report->near_cells = total;
+    if (threadIdx.x == 0u) {
+      report->near_cells = total[0];
+      report->filled_cells = total[1];
+    }
   }
   const uint32_t t = 4u * (blockIdx.x * 256u + threadIdx.x);
   if (!run || t >= 4u * n) return;
@@ -625,7 +639,10 @@ __global__ __launch_bounds__(128) void k_clear_16(const uint64_t* __restrict__ l
                                                   CtxReport* __restrict__ report) {
   const bool empty = l1[0] == 0ull;
   map[threadIdx.x] = empty ? 255 : 0;
-  if (threadIdx.x == 0u) report->near_cells = empty ? 0u : 8u;
+  if (threadIdx.x == 0u) {
+    report->near_cells = empty ? 0u : 8u;
+    report->filled_cells = 0u;
+  }
 }
 
 uint32_t clear_cells(uint32_t dim) {
@@ -689,7 +706,10 @@ void finish_maps(vt_world* w) {
     for (uint32_t o = 0; o < 8; o++)
       w->free_frac = std::max(w->free_frac, (float)((double)r->free_regions[o] / (R * R * R)));
   }
-  if (w->clear) w->near_frac = (float)((double)r->near_cells / (double)clear_cells(w->dim));
+  if (w->clear) {
+    const uint32_t open = clear_cells(w->dim) - r->filled_cells;
+    w->near_frac = open ? (float)((double)r->near_cells / (double)open) : 1.0f;
+  }
   w->maps_valid = true;
 }
 
@@ -701,15 +721,33 @@ bool use_free_map(const vt_world* w, const ShadeConsts& sc) {
          w->free_frac * VT_FREE_MIN_SHARE >= 1.0f;
 }
 
-// The map pays where rays cross clear space.  Terrain worlds with open sky
-// have 15% of their cells near; where a block floats in nearly every cell (71%
-// near) the clear stretches are too short: 16 Lambert views of that 256^3
-// world take 1740 us with the map and 1420 without.
-constexpr float kClearNearShare = 0.5f;
+// The map pays where rays cross clear space, so the rule counts the cells they
+// can cross: a filled cell (solid ground) says nothing.  Microseconds with the
+// map and without, 256^3 at 1280x720 with caps of 2048 (of 192 / 48), by the
+// near share of what is not filled:
+//   scattered blocks, no sky    0.12 126, 177 (75, 95)    0.27 163, 168 (109, 107)
+//                               0.40 175, 165 (116, 106)  0.59 195, 175 (118, 106)
+//   terrain, blocks up to the top (0.50) 124, 120 (84, 78)
+//   ground with open sky        0.08 58, 96 (44, 49)      0.18 76, 131 (65, 87)
+// and worlds of 512^3 with open ground to 55% of their height 73, 165, in the
+// reference layout 81, 262.  Above the line the space between things is too
+// small to cross, but a ray that leaves it for the sky still ends at once with
+// the map and otherwise takes every step to the edge of the grid.  By the
+// largest share of free regions, blocks below an empty sky, caps of 2048:
+//   near 0.44, free 0.3: 162, 183     near 0.62, free 0.38: 81, 115
+//   near 0.71, free 0.25: 74, 84      near 0.80, free 0.19: 74, 74
+//   near 0.56, free 0.06: 213, 198
+// Caps of 192 / 48 end most such rays themselves, and it takes a sky of half
+// the world: near 0.49, free 0.5: 61, 79 at 512^3 and 44, 94 in the reference
+// layout; free 0.38: 65, 72, and at 256x256 32, 27; free 0.3: 105, 98.
+constexpr float kClearNearShare = 1.0f / 3.0f;
+constexpr float kClearFreeShare = 0.25f, kClearFreeShareShort = 0.45f;
 
-bool use_clear_map(const vt_world* w, uint32_t flags) {
+bool use_clear_map(const vt_world* w, uint32_t flags, int max_primary, int max_shadow) {
   if (!w->clear || !w->maps_valid || (flags & VT_FLAG_FREE_MAP_OFF)) return false;
-  return (flags & VT_FLAG_FREE_MAP_ON) || w->near_frac <= kClearNearShare;
+  if ((flags & VT_FLAG_FREE_MAP_ON) || w->near_frac <= kClearNearShare) return true;
+  const bool long_caps = max_primary >= VT_FREE_MIN_CAP || max_shadow >= VT_FREE_MIN_CAP;
+  return w->free_frac >= (long_caps ? kClearFreeShare : kClearFreeShareShort);
 }
 
 // The texel masks of an atlas: a thread makes one word (layer z of a model)
