@@ -72,3 +72,30 @@ def test_lists_in_any_order(ctx, layout):
         apply(w, grid, xyz.astype(np.uint32), val.astype(np.uint32))
         equals_fresh_world(ctx, layout, w, grid, f"{count} edits")
     w.close()
+
+
+@pytest.mark.parametrize("n", [32, 128])
+@pytest.mark.parametrize("layout", ["dense", "reference"])
+def test_cleared_and_refilled(ctx, layout, n):
+    """2^3 sub-blocks filled, cleared in part, cleared whole and filled again,
+    alone in clear space, next to other things, in the corners of the grid and
+    of the map's 8^3 cells, one by one and many at a time."""
+    rng = np.random.default_rng([n, 5])
+    grid = np.zeros((n, n, n), np.uint8)
+    grid[:, :2] = 3
+    grid[n // 2, :n // 3, n // 2] = 4
+    w = fresh(ctx, layout, grid)
+    sub = np.stack([v.ravel() for v in np.mgrid[0:2, 0:2, 0:2]], 1)
+    lows = np.vstack([[0, n - 2, 0], [n - 2, n - 2, n - 2], [6, 14, 6], [8, 16, 8],
+                      [n // 2, n // 3, n // 2], 2 * rng.integers(1, n // 2, (6, 3))])
+    all_of = (lows[:, None] + sub[None]).reshape(-1, 3).astype(np.uint32)
+    steps = [("filled", all_of, 5), ("thinned", all_of[::2], 0), ("cleared", all_of, 0)]
+    for k, low in enumerate(lows[:5]):
+        one = (low + sub).astype(np.uint32)
+        steps += [(f"one voxel of {k}", one[3:4], 6), (f"the rest of {k}", one, 6),
+                  (f"all but one of {k}", one[1:], 0), (f"none of {k}", one, 0)]
+    steps += [("filled again", all_of, 7), ("cleared again", all_of, 0)]
+    for label, xyz, v in steps:
+        apply(w, grid, xyz, np.full(len(xyz), v, np.uint32))
+        equals_fresh_world(ctx, layout, w, grid, f"{n}^3 {label}")
+    w.close()
