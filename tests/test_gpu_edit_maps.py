@@ -99,3 +99,29 @@ def test_cleared_and_refilled(ctx, layout, n):
         apply(w, grid, xyz, np.full(len(xyz), v, np.uint32))
         equals_fresh_world(ctx, layout, w, grid, f"{n}^3 {label}")
     w.close()
+
+
+@pytest.mark.parametrize("layout,n", [("reference", 64), ("reference", 256), ("dense", 256),
+                                      ("dense", 512), ("dense", 1024)])
+def test_layer_by_layer(ctx, layout, n):
+    """Edits that change a few of the map's layers along z (8 voxels each, 128
+    of them at 1024^3): at both ends, on either side of the 64th, at a layer's
+    faces, where a voxel is near cells of two; one layer and several at once;
+    placed and taken away in another order."""
+    rng = np.random.default_rng([n, 8])
+    grid = np.zeros((n, n, n), np.uint8)
+    grid[n // 4:n // 4 + 9, n // 3:n // 3 + 5, n // 2:n // 2 + 30] = 4
+    w = fresh(ctx, layout, grid)
+    at = sorted({0, 5, 7, 8, 10, n // 2 - 2, n // 2 - 1, n // 2, n // 2 + 4, n - 9, n - 8, n - 1})
+    put = []
+    for k, z in enumerate(at):
+        xyz = np.stack([rng.integers(0, n, 3), rng.integers(0, n, 3), np.full(3, z)], 1)
+        put.append(xyz.astype(np.uint32))
+        if k % 3 == 2 or k == len(at) - 1:  # the last few in one call
+            apply(w, grid, np.vstack(put[k - k % 3:]), np.full(3 * (k % 3 + 1), 5, np.uint32))
+            equals_fresh_world(ctx, layout, w, grid, f"{n}^3 up to layer {z // 8}")
+    for k in rng.permutation(len(at)):
+        apply(w, grid, put[k], np.zeros(3, np.uint32))
+        if k % 3 == 0:
+            equals_fresh_world(ctx, layout, w, grid, f"{n}^3 without {at[k]}")
+    w.close()

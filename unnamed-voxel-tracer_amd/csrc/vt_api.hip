@@ -88,7 +88,8 @@ int dev_alloc(vt_world* w, void** p, size_t bytes, const char* what) {
 
 // The free-region and clearance maps (built by vt::rebuild_maps).
 int alloc_maps(vt_world* w) {
-  int st = dev_alloc(w, (void**)&w->freemap, (8u * vt::free_words_per_octant(w->dim) + 2u) * 4u,
+  int st = dev_alloc(w, (void**)&w->freemap,
+                     (8u * vt::free_words_per_octant(w->dim) + vt::kChangedWords) * 4u,
                      "free-region map");
   if (st != VT_OK || w->dim < 16u) return st;
   // the clearance map and, behind it, its scratch (k_clear_16 needs none)

@@ -40,7 +40,7 @@ __global__ __launch_bounds__(256) void k_edit_brickmap(uint32_t* __restrict__ po
                                                        uint32_t n, uint32_t m,
                                                        uint32_t* __restrict__ changed) {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-  if (i < 2u && changed) changed[i] = 0u;  // for the kernels that follow
+  if (i < kChangedWords && changed) changed[i] = 0u;  // for the kernels that follow
   if (i < n) {
     const uint3 r = reinterpret_cast<const uint3*>(data)[i];
     pool[(size_t)r.x * 512u + (compact1by2(r.z) & 7u) + 8u * (compact1by2(r.z >> 1) & 7u) +
@@ -54,14 +54,17 @@ __global__ __launch_bounds__(256) void k_edit_brickmap(uint32_t* __restrict__ po
 }
 
 // The clearance map's byte of brick b (null: a world without the map), from
-// its occupancy word; sets changed[1] when it is another one.
+// its occupancy word; when it is another one, marks the brick's layer of cells
+// and the one it faces (of two bricks a cell has along z).
 __device__ __forceinline__ void put_sub(uint8_t* sub, uint32_t b, uint64_t word,
                                         uint32_t* changed) {
   if (!sub) return;
   const uint8_t v = (uint8_t)nonzero_bytes(word);
   if (sub[b] != v) {
     sub[b] = v;
-    changed[1] = 1u;
+    const uint32_t bz = compact1by2(b >> 2), z = bz >> 1, to = (bz & 1u) ? z + 1u : z - 1u;
+    atomicOr(&changed[1u + (z >> 5)], 1u << (z & 31u));
+    if (to < 128u) atomicOr(&changed[1u + (to >> 5)], 1u << (to & 31u));
   }
 }
 
@@ -104,7 +107,7 @@ __global__ __launch_bounds__(256) void k_edit_dense(uint8_t* __restrict__ vox,
                                                     const uint32_t* __restrict__ data,
                                                     uint32_t n, uint32_t* __restrict__ changed) {
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-  if (i < 2u) changed[i] = 0u;  // for the kernels that follow
+  if (i < kChangedWords) changed[i] = 0u;  // for the kernels that follow
   if (i < n) vox[data[2u * (size_t)i]] = (uint8_t)data[2u * (size_t)i + 1u];
 }
 

@@ -73,9 +73,8 @@ struct vt_world {
   uint64_t* masks;         // texel masks of the atlas's models (with occ)
   uint64_t* brick_bits;    // brickmap: bit per 4^3 brick of blocks, from occ
   // free-region map (dense worlds and power-of-two brickmap worlds)
-  uint32_t* freemap;       // 8 octants x free_words_per_octant(dim) words, then a
-                           // two words edits set: when a region empties or
-                           // fills, when a 2^3 sub-block does
+  uint32_t* freemap;       // 8 octants x free_words_per_octant(dim) words, then
+                           // the words edits set (maps_changed)
   // clearance map (the same worlds, dim >= 16)
   uint8_t* clear;          // 2 orders x 8 octants x clear_cells(dim) bytes
   uint8_t* clear_tmp;      // clear_tmp_bytes(dim): the sub-block bits of every
@@ -219,8 +218,8 @@ hipError_t launch_build_l1b(const uint64_t* l0, uint64_t n0, const uint32_t* wor
 // Free-region map: regions of 16^3 blocks, R = free_regions(dim) per axis;
 // bit r of octant o's bitmap (free_words_per_octant(dim) words) is set when
 // no region at or ahead of r on every axis in o's travel direction holds a
-// nonempty block.  Built from the brick bits (a dense world's L1 words, a
-// brickmap world's brick_bits), unless *changed (device, may be null) is 0;
+// nonempty block.  Built from a dense world's L1b words or a brickmap world's
+// brick_bits, unless *changed (device, may be null) is 0;
 // reports whether it was and the free regions of each octant.
 uint32_t free_regions(uint32_t dim);
 uint32_t free_words_per_octant(uint32_t dim);
@@ -251,13 +250,15 @@ inline bool begin_occupancy_change(vt_world* w) {
   return current;
 }
 // Rebuilds a world's free-region and clearance maps from its current
-// occupancy (L1 words or brick bits, and the sub-block bits); no-op without
-// them.  `changed`: the two words of maps_changed (null: rebuild always).
+// occupancy (L1b words or brick bits, and the sub-block bits); no-op without
+// them.  `changed`: the words of maps_changed (null: rebuild everything).
 // Leaves maps_valid false: the caller calls finish_maps once the stream has
 // synchronised without error.
 hipError_t rebuild_maps(vt_world* w, hipStream_t stream, const uint32_t* changed = nullptr);
-// The words edits set: [0] a 16^3 region emptied or filled, [1] a 2^3
-// sub-block did.
+// The words edits set: [0] a 16^3 region emptied or filled; [1 ..] bit z: a
+// 2^3 sub-block did from which the near cells of layer z follow (cells of the
+// clearance map, at most 128 layers).
+constexpr uint32_t kChangedWords = 5;
 inline uint32_t* maps_changed(const vt_world* w) {
   return w->freemap ? w->freemap + 8u * free_words_per_octant(w->dim) : nullptr;
 }

@@ -293,20 +293,21 @@ constexpr uint32_t kMapBlock = 1024;
 // of the regions at or ahead of x by shifts; along y and z the rows take the
 // OR of rows 1, 2, 4, ... ahead.  Then bit j of word w of the octant's bitmap
 // = the region with Morton code 32 w + j is free.  Bound by the one CU a block
-// has: 16 us at 512^3 (five kernels over byte planes: 36).  An edit rarely
+// has: 14 us at 512^3 (five kernels over byte planes: 36), 49 at 1024^3 (59
+// with a word of 8 bytes a region instead of a byte).  An edit rarely
 // empties or fills a whole region, so it passes `changed` (device word: a
 // region did) and the launch ends at once, in 3 us, when none did.
 struct FreeMapArgs {
-  const uint64_t* l1;
-  uint32_t lg, words;
+  const uint64_t* l1b;    // a dense world's 8^3-brick level
+  const uint64_t* words;  // else: a word per region
+  uint32_t lg, nwords;
   uint32_t* fm;
   const uint32_t* changed;
   CtxReport* report;
 };
 __device__ __forceinline__ void free_map_block(const FreeMapArgs& a, uint64_t* row,
                                                uint32_t& total) {
-  const uint64_t* __restrict__ l1 = a.l1;
-  const uint32_t lg = a.lg, words = a.words;
+  const uint32_t lg = a.lg, words = a.nwords;
   uint32_t* __restrict__ fm = a.fm;
   CtxReport* __restrict__ report = a.report;
   const bool run = !a.changed || *a.changed != 0u;
@@ -318,20 +319,25 @@ __device__ __forceinline__ void free_map_block(const FreeMapArgs& a, uint64_t* r
   const uint64_t full = R == 64u ? ~0ull : (1ull << R) - 1ull;
   for (uint32_t r = t; r < rows; r += 1024u) row[r] = 0ull;
   __syncthreads();
-  // eight consecutive codes (2^3 regions) a thread: two bits of four rows
+  // eight consecutive codes (2^3 regions) a thread: two bits of four rows.  A
+  // region is a byte of the 8^3-brick level's words (dense worlds) or a word of
+  // the brick bits.
   uint32_t* half = reinterpret_cast<uint32_t*>(row);
   for (uint32_t g = t; g < (n >= 8u ? n / 8u : 1u); g += 1024u) {
     uint32_t any = 0u;
-    if (n >= 8u) {
-      const uint4* p = reinterpret_cast<const uint4*>(l1 + 8u * (size_t)g);
+    if (a.l1b) {
+      any = nonzero_bytes(a.l1b[g]);
+    } else if (n >= 8u) {
+      const uint4* p = reinterpret_cast<const uint4*>(a.words + 8u * (size_t)g);
 #pragma unroll
       for (uint32_t k = 0; k < 4u; k++) {
         const uint4 q = p[k];
         any |= ((q.x | q.y) ? 1u : 0u) << (2u * k) | ((q.z | q.w) ? 2u : 0u) << (2u * k);
       }
     } else {
-      any = l1[0] != 0ull ? 1u : 0u;  // R = 1
+      any = a.words[0] != 0ull ? 1u : 0u;  // R = 1
     }
+    if (any == 0u) continue;
     const uint32_t x = 2u * compact1by2(g), y = 2u * compact1by2(g >> 1),
                    z = 2u * compact1by2(g >> 2);
 #pragma unroll
@@ -454,6 +460,42 @@ __device__ __forceinline__ bool cell_near(const uint64_t* __restrict__ words, ui
   return any != 0ull;
 }
 
+// The layers of cells whose near cells an edit may have changed, bit z of 128
+// (maps_changed).  A rebuild after an edit makes the rows and planes of these
+// alone: the scratch holds the others'.  1024^3, a brush of 4^3 blocks: the
+// rebuild's launches 49 + 9 + 58 us where all layers take 83 + 26 + 82, the
+// edit 147 us against 223; 64 blocks anywhere (most layers) 176 against 220.
+struct Layers {
+  uint64_t lo, hi;
+};
+__device__ __forceinline__ Layers changed_layers(const uint32_t* __restrict__ changed) {
+  return {changed[0] | (uint64_t)changed[1] << 32, changed[2] | (uint64_t)changed[3] << 32};
+}
+// Whether one of layers z0 .. z1 is among them.
+__device__ __forceinline__ bool some_layer(const Layers& l, uint32_t z0, uint32_t z1) {
+  for (uint32_t z = z0; z <= z1; z++)
+    if ((z < 64u ? l.lo >> z : l.hi >> (z - 64u)) & 1u) return true;
+  return false;
+}
+// Layers from z on (z itself: 0) to the first of them upwards or downwards;
+// 255: none.
+__device__ __forceinline__ uint32_t next_layer(const Layers& l, uint32_t z, bool down) {
+  uint64_t near, far;  // `near` the half that z lies in, from z on
+  uint32_t to_far;
+  if (down) {
+    near = z < 64u ? l.lo << (63u - z) : l.hi << (127u - z);
+    far = z < 64u ? 0ull : l.lo;
+    to_far = z - 63u;
+    if (near) return (uint32_t)__builtin_clzll(near);
+    return far ? to_far + (uint32_t)__builtin_clzll(far) : 255u;
+  }
+  near = z < 64u ? l.lo >> z : l.hi >> (z - 64u);
+  far = z < 64u ? l.hi : 0ull;
+  to_far = 64u - z;
+  if (near) return (uint32_t)__builtin_ctzll(near);
+  return far ? to_far + (uint32_t)__builtin_ctzll(far) : 255u;
+}
+
 // Rows of cells along x, one thread per cell: the distance along +x (plane 0)
 // and -x (plane 1) to the first near cell of the row.  A block takes kMapBlock
 // cells (whole rows), finds the rows' near cells by ballot and notes how many
@@ -470,9 +512,12 @@ __device__ __forceinline__ void clear_rows_block(const ClearRowsArgs& a, uint32_
   const uint64_t* __restrict__ words = a.words;
   uint8_t* __restrict__ rows = a.rows;
   const uint32_t lg = a.lg;
-  if (a.changed && *a.changed == 0u) return;  // the same for every thread
-  const uint32_t R = 1u << lg, n = 1u << (3u * lg);
-  const uint32_t i = block * kMapBlock + threadIdx.x, x = i & (R - 1u);
+  const uint32_t R = 1u << lg, n = 1u << (3u * lg), i0 = block * kMapBlock;
+  if (a.changed &&  // the same for every thread
+      !some_layer(changed_layers(a.changed), i0 >> (2u * lg),
+                  min(i0 + kMapBlock - 1u, n - 1u) >> (2u * lg)))
+    return;
+  const uint32_t i = i0 + threadIdx.x, x = i & (R - 1u);
   bool near = false, filled = false;
   if (i < n) near = cell_near(words, R, x, (i >> lg) & (R - 1u), i >> (2u * lg), filled);
   const uint64_t b = __ballot(near), f = __ballot(filled);
@@ -516,8 +561,9 @@ __device__ __forceinline__ void clear_rows_block(const ClearRowsArgs& a, uint32_
 // read different words and neither waits for the other, and each was a
 // launch of 12-15 us with most of the chip idle (8 blocks; 262,144 threads of
 // one wave's latency).  The first 8 blocks take the octants' bitmaps, the
-// others the rows of cells.  A rebuild at 512^3 37 us instead of 48 (this
-// launch 17 of them; the octants' blocks, one CU each, bound it).
+// others the rows of cells.  A rebuild at 512^3 37 us instead of 48, after an
+// edit of a few layers 28 (this launch 14 of them; the octants' blocks, one CU
+// each, bound it).
 __global__ __launch_bounds__(1024) void k_maps_first(FreeMapArgs fa, ClearRowsArgs ca) {
   __shared__ uint64_t row[4096];
   __shared__ uint32_t total;
@@ -576,7 +622,6 @@ __global__ __launch_bounds__(256) void k_clear_planes(const uint8_t* __restrict_
                                                       const uint32_t* __restrict__ near_count,
                                                       const uint32_t* __restrict__ changed,
                                                       CtxReport* __restrict__ report) {
-  const bool run = !changed || *changed != 0u;  // the same for every thread
   const uint32_t R = 1u << lg, n = 1u << (3u * lg);
   if (blockIdx.x == 0u) {
     __shared__ uint32_t total[2];
@@ -596,8 +641,10 @@ __global__ __launch_bounds__(256) void k_clear_planes(const uint8_t* __restrict_
     }
   }
   const uint32_t t = 4u * (blockIdx.x * 256u + threadIdx.x);
-  if (!run || t >= 4u * n) return;
+  if (t >= 4u * n) return;
   const uint32_t v = t >> (3u * lg), i = t & (n - 1u), y = (i >> lg) & (R - 1u);
+  const uint32_t layer = i >> (2u * lg);
+  if (changed && !some_layer(changed_layers(changed), layer, layer)) return;
   const bool neg = (v & 2u) != 0u;
   *reinterpret_cast<uint32_t*>(planes + t) =
       ahead(rows + (size_t)(v & 1u) * n + i, neg ? -(ptrdiff_t)R : (ptrdiff_t)R,
@@ -605,11 +652,12 @@ __global__ __launch_bounds__(256) void k_clear_planes(const uint8_t* __restrict_
 }
 
 // The map: octant plane o with its negative axes complemented, in Morton
-// order and (8 planes on) in linear order.
+// order and (8 planes on) in linear order.  A byte m follows from the layers
+// up to m ahead (a near cell further on is further off), so after an edit it
+// stays what it is when none of those changed.
 __global__ __launch_bounds__(256) void k_clear_cubes(const uint8_t* __restrict__ planes,
                                                      uint32_t lg, uint8_t* __restrict__ map,
                                                      const uint32_t* __restrict__ changed) {
-  if (changed && *changed == 0u) return;
   const uint32_t R = 1u << lg, n = 1u << (3u * lg);
   const uint32_t t = 4u * (blockIdx.x * 256u + threadIdx.x);
   if (t >= 8u * n) return;
@@ -617,27 +665,35 @@ __global__ __launch_bounds__(256) void k_clear_cubes(const uint8_t* __restrict__
   const uint32_t x = i & (R - 1u), y = (i >> lg) & (R - 1u), z = i >> (2u * lg);
   const ptrdiff_t layer = (ptrdiff_t)R * R;
   const bool neg = (o & 4u) != 0u;
-  uint32_t m = ahead(planes + (size_t)(o & 3u) * n + i, neg ? -layer : layer,
-                     neg ? z + 1u : R - z);
-  if (o & 1u) m = __builtin_bswap32(m);
   const uint32_t fx = (o & 1u) ? R - 4u - x : x, fy = (o & 2u) ? R - 1u - y : y,
                  fz = (o & 4u) ? R - 1u - z : z;
   uint8_t* plane = map + (size_t)o * n;
+  uint32_t* linear =
+      reinterpret_cast<uint32_t*>(plane + 8u * (size_t)n + fx + (size_t)R * (fy + (size_t)R * fz));
+  if (changed) {
+    const uint32_t next = next_layer(changed_layers(changed), z, neg);
+    if (next == 255u) return;  // nothing ahead
+    const uint32_t old = *linear;
+    const uint32_t most = max(max(old & 255u, (old >> 8) & 255u), max((old >> 16) & 255u, old >> 24));
+    if (next > most) return;
+  }
+  uint32_t m = ahead(planes + (size_t)(o & 3u) * n + i, neg ? -layer : layer,
+                     neg ? z + 1u : R - z);
+  if (o & 1u) m = __builtin_bswap32(m);
   // cells fx .. fx + 3 have Morton codes c, c + 1, c + 8, c + 9
   uint16_t* mor = reinterpret_cast<uint16_t*>(plane + morton3(fx, fy, fz));
   mor[0] = (uint16_t)m;
   mor[4] = (uint16_t)(m >> 16);
-  *reinterpret_cast<uint32_t*>(plane + 8u * (size_t)n + fx + (size_t)R * (fy + (size_t)R * fz)) =
-      m;
+  *linear = m;
 }
 
 // A 16^3 map has 2 cells a side and is one region: clear all round (255) when
 // it holds nothing, else all of it near, so that no ray is asked to walk 2
 // cells.
-__global__ __launch_bounds__(128) void k_clear_16(const uint64_t* __restrict__ l1,
+__global__ __launch_bounds__(128) void k_clear_16(const uint64_t* __restrict__ word,
                                                   uint8_t* __restrict__ map,
                                                   CtxReport* __restrict__ report) {
-  const bool empty = l1[0] == 0ull;
+  const bool empty = word[0] == 0ull;
   map[threadIdx.x] = empty ? 255 : 0;
   if (threadIdx.x == 0u) {
     report->near_cells = empty ? 0u : 8u;
@@ -656,16 +712,18 @@ size_t clear_tmp_bytes(uint32_t dim) {
 }
 
 // The rebuild of a world's maps; without a clearance map (map null, dim < 16)
-// the free-region map alone.  changed: two device words, whether a region and
-// whether a sub-block emptied or filled; null = rebuild both.
-static hipError_t launch_build_maps(const uint64_t* l1, uint32_t dim, uint32_t* fm, uint8_t* tmp,
-                                    uint8_t* map, const uint32_t* changed, CtxReport* report,
+// the free-region map alone.  changed: the words of maps_changed; null =
+// rebuild both.
+static hipError_t launch_build_maps(const uint64_t* l1b, const uint64_t* words, uint32_t dim,
+                                    uint32_t* fm, uint8_t* tmp, uint8_t* map,
+                                    const uint32_t* changed, CtxReport* report,
                                     hipStream_t stream) {
-  FreeMapArgs fa = {l1, 0u, free_words_per_octant(dim), fm, changed, report};
+  FreeMapArgs fa = {l1b, words, 0u, free_words_per_octant(dim), fm, changed, report};
   while ((1u << fa.lg) < free_regions(dim)) fa.lg++;
   if (dim < 32u) {
     hipLaunchKernelGGL(k_maps_first, dim3(8), dim3(kMapBlock), 0, stream, fa, ClearRowsArgs{});
-    if (map) hipLaunchKernelGGL(k_clear_16, dim3(1), dim3(128), 0, stream, l1, map, report);
+    if (map) hipLaunchKernelGGL(k_clear_16, dim3(1), dim3(128), 0, stream, l1b ? l1b : words, map,
+                                report);
     return hipGetLastError();
   }
   const uint32_t n = clear_cells(dim);
@@ -692,8 +750,8 @@ uint32_t brick_bit_words(uint32_t dim) {
 hipError_t rebuild_maps(vt_world* w, hipStream_t stream, const uint32_t* changed) {
   w->maps_valid = false;
   if (!w->freemap) return hipSuccess;
-  return launch_build_maps(w->kind == WorldKind::Dense ? w->l1 : w->brick_bits, w->dim, w->freemap,
-                           w->clear_tmp, w->clear, changed, w->ctx->report_dev(), stream);
+  return launch_build_maps(w->l1b, w->brick_bits, w->dim, w->freemap, w->clear_tmp, w->clear,
+                           changed, w->ctx->report_dev(), stream);
 }
 
 void finish_maps(vt_world* w) {
