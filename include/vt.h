@@ -90,8 +90,9 @@ typedef struct vt_camera {
  * lookups and ends as a miss when its line meets nothing more (before its
  * step cap).  Every output is unchanged except the step counts, so it is
  * never done for a frame that stores them (frame.steps).  Default: done in
- * worlds open enough for it to pay; these flags force it either way (not
- * both).
+ * worlds open enough for it to pay, by the share of the space rays cross that
+ * lies near something, the sky above it and the caps; these flags force it
+ * either way (not both).
  * The library also keeps the free-region map, a bitmap of the 16^3 regions
  * from which no ray of a given direction octant can meet a nonempty block
  * (every region ahead of it on all three axes is empty: traceMap's blocks
@@ -341,11 +342,13 @@ int vt_world_info(const vt_world* world, uint32_t* dim, size_t* device_bytes);
 int vt_render(vt_ctx* ctx, const vt_world* world, const vt_camera* camera,
               const vt_render_params* params, const vt_frame* frame, void* stream);
 
-/* The free-region rule above for vt_render with these arguments: *used = 1
- * when the caps, the world's free regions and the flags let rays end early
- * in free regions, and a frame's statistics then count the steps executed;
- * 0 when its statistics are traceMap's step counts.  No counterpart in the
- * reference, whose traceMap runs every ray to its end.                     */
+/* The free-region rule above for vt_render with these arguments, a rule on
+ * the caps, the world's free regions and the flags: with statistics *used = 1
+ * when they count the steps executed, 0 when they are traceMap's step counts.
+ * For a frame without statistics 1 says that the world and the caps leave
+ * rays something to end early in; whether the launch reads the clearance map
+ * is its own rule (above), and the outputs are the same either way.  No
+ * counterpart in the reference, whose traceMap runs every ray to its end.   */
 int vt_free_map_used(const vt_world* world, const vt_render_params* params,
                      const vt_frame* frame, int* used);
 

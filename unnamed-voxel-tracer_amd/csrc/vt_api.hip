@@ -592,8 +592,7 @@ int vt_render(vt_ctx* ctx, const vt_world* world, const vt_camera* camera,
   } else {
     vt::BrickmapWorld bw = vt::brickmap_view(world);
     if (!clear) bw.clear_bytes = 0;
-    e = vt::launch_render_brickmap(bw, v, sc, o, frame->schedule, tile,
-                                   (uint32_t)ctx->compute_units, (hipStream_t)stream);
+    e = vt::launch_render_brickmap(bw, v, sc, o, frame->schedule, tile, (hipStream_t)stream);
   }
   if (e != hipSuccess) return hip_fail(e, "vt_render: launch");
   return VT_OK;

@@ -255,8 +255,7 @@ static void launch_brickmap(bool sched, const BrickmapWorld& w, const ViewConsts
 
 hipError_t launch_render_brickmap(const BrickmapWorld& w_in, const ViewConsts& v,
                                   const ShadeConsts& sc, const FrameOut& out, uint32_t* schedule,
-                                  TileShape tile, uint32_t compute_units, hipStream_t stream) {
-  (void)compute_units;
+                                  TileShape tile, hipStream_t stream) {
   BrickmapWorld w = w_in;
   // a map of fewer blocks a side than two empty-space iterations take steps
   // (8^3: one chunk) stays on the literal loop (dense_left_grid)
